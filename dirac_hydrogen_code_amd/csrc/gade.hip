@@ -10,6 +10,7 @@
 #include <chrono>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "gade_internal.h"
@@ -161,6 +162,13 @@ __device__ __forceinline__ int xcd_order(int b, int G) {
     return j * q + min(j, r) + k;
 }
 
+// element e of a base that is uniform over the wave: a scalar base and a 32-bit offset, so the address costs no
+// vector arithmetic
+template <class T>
+__device__ __forceinline__ T ld_off(const T *base, unsigned e) {
+    return *(const T *)((const char *)base + (unsigned)(e * sizeof(T)));
+}
+
 constexpr int kAngThreads = 256;
 constexpr int kAngLB = 2;  // default multipoles per block
 
@@ -207,18 +215,18 @@ __global__ __launch_bounds__(kAngThreads) void k_angular(const T *__restrict__ x
         for (int u = 0; u < U; u++) {
             const int p = p0 + u;
             if (p >= len) break;
-            const T kx = cscale(xv[u], (Rt)shk[p].y);
+            const Rt kc = (Rt)shk[p].y;
             const T *cp = shc + (size_t)p * LB * 2;
 #pragma unroll
             for (int l = 0; l < LB; l++) {
                 const T h0 = cp[2 * l], h1 = cp[2 * l + 1];
                 if (cnz(h0)) {
                     z0[l] = cfma(h0, xv[u], z0[l]);
-                    z2[l] = cfma(h0, kx, z2[l]);
+                    z2[l] = cfma(cscale(h0, kc), xv[u], z2[l]);
                 }
                 if (cnz(h1)) {
                     w0[l] = cfma(h1, xv[u], w0[l]);
-                    w1[l] = cfma(h1, kx, w1[l]);
+                    w1[l] = cfma(cscale(h1, kc), xv[u], w1[l]);
                 }
             }
         }
@@ -246,22 +254,35 @@ __global__ __launch_bounds__(kAngThreads) void k_angular(const T *__restrict__ x
 // contiguous stream; the next group's x loads are issued before the current group is summed.  Lists are per
 // instance-local row; x is offset to the instance.
 constexpr int kAngListU = 4;
-template <class T>
-__device__ __forceinline__ void ang_list_group(const T (&xv)[kAngListU], const int2 *__restrict__ ck,
-                                               const T *__restrict__ cf, T &z0, T &z2, T &w0, T &w1) {
+
+// One list entry's terms of the four sums: h0 x, (h0 k) x, h1 x, (h1 k) x.  RC (all couplings real up to one common
+// factor 1 or i): the entry is the real pairs (h0, h1) and (h0 k, h1 k) and the sums leave the factor out; half the
+// products of the complex form (cf: h0, then h1).
+template <bool RC, class T>
+__device__ __forceinline__ void ang_terms(const T xv, const int kc, const T *__restrict__ cf, T &z0, T &z2, T &w0,
+                                          T &w1) {
     using Rt = typename cx<T>::R;
-#pragma unroll
-    for (int u = 0; u < kAngListU; u++) {
-        const T h0 = cf[2 * u], h1 = cf[2 * u + 1];
-        const T kx = cscale(xv[u], (Rt)ck[u].y);
-        z0 = cfma(h0, xv[u], z0);
-        z2 = cfma(h0, kx, z2);
-        w0 = cfma(h1, xv[u], w0);
-        w1 = cfma(h1, kx, w1);
+    if constexpr (RC) {
+        const T h = cf[0], hk = cf[1];
+        z0 = rfma(h.x, xv, z0);
+        z2 = rfma(hk.x, xv, z2);
+        w0 = rfma(h.y, xv, w0);
+        w1 = rfma(hk.y, xv, w1);
+    } else {
+        z0 = cfma(cf[0], xv, z0);
+        z2 = cfma(cscale(cf[0], (Rt)kc), xv, z2);
+        w0 = cfma(cf[1], xv, w0);
+        w1 = cfma(cscale(cf[1], (Rt)kc), xv, w1);
     }
 }
+template <bool RC, class T>
+__device__ __forceinline__ void ang_list_group(const T (&xv)[kAngListU], const int2 *__restrict__ ck,
+                                               const T *__restrict__ cf, T &z0, T &z2, T &w0, T &w1) {
+#pragma unroll
+    for (int u = 0; u < kAngListU; u++) ang_terms<RC>(xv[u], ck[u].y, cf + 2 * u, z0, z2, w0, w1);
+}
 
-template <int LB, class T = double2>
+template <int LB, class T = double2, bool RC = false>
 __global__ __launch_bounds__(kAngThreads) void k_angular_list(const T *__restrict__ x, const int *__restrict__ aoff,
                                                               const int2 *__restrict__ ack,
                                                               const T *__restrict__ acf, int n, int lmax,
@@ -298,7 +319,7 @@ __global__ __launch_bounds__(kAngThreads) void k_angular_list(const T *__restric
 #pragma unroll
                 for (int u = 0; u < kAngListU; u++)
                     nxt[u] = xi[(size_t)ack[min(g + kAngListU + u, E1 - 1)].x * n + ac];
-                ang_list_group(cur, ack + g, acf + 2 * g, z0[li], z2[li], w0[li], w1[li]);
+                ang_list_group<RC>(cur, ack + g, acf + 2 * g, z0[li], z2[li], w0[li], w1[li]);
                 if (g + kAngListU >= e) {  // odd number of groups: the loaded group opens the next list
 #pragma unroll
                     for (int u = 0; u < kAngListU; u++) cur[u] = nxt[u];
@@ -308,8 +329,8 @@ __global__ __launch_bounds__(kAngThreads) void k_angular_list(const T *__restric
 #pragma unroll
                 for (int u = 0; u < kAngListU; u++)
                     cur[u] = xi[(size_t)ack[min(g + 2 * kAngListU + u, E1 - 1)].x * n + ac];
-                ang_list_group(nxt, ack + g + kAngListU, acf + 2 * (g + kAngListU), z0[li], z2[li], w0[li],
-                               w1[li]);
+                ang_list_group<RC>(nxt, ack + g + kAngListU, acf + 2 * (g + kAngListU), z0[li], z2[li],
+                                   w0[li], w1[li]);
             }
         }
     }
@@ -323,6 +344,16 @@ __global__ __launch_bounds__(kAngThreads) void k_angular_list(const T *__restric
         V[base + plane] = z2[l];
         V[base + 2 * plane] = w0[l];
         V[base + 3 * plane] = w1[l];
+    }
+}
+
+// FP32 copy of the real lists: the products with kappa from the rounded couplings, as the complex form takes them
+__global__ __launch_bounds__(256) void k_acr32(int ne, const double2 *__restrict__ acr, const int2 *__restrict__ ack,
+                                               float2 *__restrict__ out) {
+    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += gridDim.x * blockDim.x) {
+        const float2 h = to_f32(acr[2 * (size_t)e]);
+        out[2 * (size_t)e] = h;
+        out[2 * (size_t)e + 1] = cscale(h, (float)ack[e].y);
     }
 }
 
@@ -512,27 +543,25 @@ __global__ __launch_bounds__(256) void k_radial_sum(const T *__restrict__ ypart,
 // radial product is a sum over d of coefficient[d][i] * window[i+d]: no column
 // indices, and the window of a wave is one contiguous run staged in LDS.
 //
-// One wave owns R row blocks of one kappa (kDiaR by default), one output half h,
+// One wave takes the rows of a tile (R row blocks of one kappa),
 // 64*P consecutive outputs (P per lane, so each staged window value is read
 // once per lane and reused across the diagonals) and one multipole l; the grid
 // is ordered so that each XCD works through a few (segment, multipole) slices
 // at a time.  The per-multipole results go to ypart and are summed in a fixed
 // order.
 // ---------------------------------------------------------------------------
-constexpr int kDiaR = 8;        // default rows per tile
 constexpr int kDiaSegMax = 256; // longest output run of a wave (64 lanes x 4 outputs); nhp is a multiple of it
 constexpr int kDiaBW = 7;
 
-// LDS slot of window position p: swaps neighbours on alternate 8-slot rows so
-// that lanes reading positions 2*lane+t hit distinct banks
-// (P = 2); for P = 4 (lanes reading positions 4*lane+t) the low two bits are XORed instead.  Both are
-// conflict-free for the sliding reads and for the stride-1 staging writes (64 banks, 16 lanes per pass).
-// With one output per lane (P = 1) the lanes read consecutive positions: no swizzle.
+// LDS slot of window position p of a run of 64*P outputs: position p at [p % P][p / P], so the lanes' positions
+// P*lane + t (t fixed) are consecutive slots: conflict-free reads whose addresses differ by constants only.
 template <int P>
-__device__ __forceinline__ int dia_swz(int p) {
-    if constexpr (P == 1) return p;
-    if constexpr (P == 4) return p ^ (((p >> 2) ^ (p >> 4)) & 3);
-    return p ^ (((p >> 3) ^ (p >> 4)) & 1);
+constexpr int dia_wp() {  // slots per residue
+    return (64 * P + 2 * kDiaBW + P - 1) / P;
+}
+template <int P>
+__device__ __forceinline__ int dia_slot(int p) {
+    return (p % P) * dia_wp<P>() + p / P;
 }
 
 // GD[l][v][qd][d][ip] = (G_m1, G_m2) of the kappa-folded pair of v, from the
@@ -541,7 +570,10 @@ __device__ __forceinline__ int dia_swz(int p) {
 // component v (six loads each).
 // Coefficients: by value (cg, instances b0 + blockIdx.y), or from the device window table
 // cf_dev[slot][B] at slot gctl[GC_WSLOT] (the form a replayed step graph uses).
-__global__ __launch_bounds__(256) void k_gsums_dia(const double2 *__restrict__ gs, const double2 *__restrict__ gts,
+// RC: real couplings (E = double) and real f(t), so that every sum is i times a real one: the pair is stored as one
+// complex word (G, G') without the i, half the bytes read and written (the same sums: the other half is zero).
+template <bool RC, class E>
+__global__ __launch_bounds__(256) void k_gsums_dia(const E *__restrict__ gs, const E *__restrict__ gts,
                                                    CoefGroup cg, int b0, size_t gd_stride, int lmax, int nd, int nhp,
                                                    double2 *__restrict__ GD0, const int *gate, int gstride,
                                                    const Coef6 *__restrict__ cf_dev, const int *__restrict__ gctl,
@@ -565,19 +597,28 @@ __global__ __launch_bounds__(256) void k_gsums_dia(const double2 *__restrict__ g
         const int e = (int)(idx - (long long)lv * S);  // (qd, d, ip)
         const int l = lv >> 2, v = lv & 3;
         // (Gs0,Gs1) (Gs2,Gs3) (Gts0,Gts2) (Gts1,Gts3) pair with Z0, Z2, W0, W1
-        const double2 *src = v < 2 ? gs : gts;
+        const E *src = v < 2 ? gs : gts;
         const int n1 = v == 0 ? 0 : v == 1 ? 2 : v == 2 ? 0 : 1, n2 = v == 0 ? 1 : v == 1 ? 3 : v == 2 ? 2 : 3;
         double2 G1 = make_double2(0, 0), G2 = make_double2(0, 0);
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             const double2 c = (l % 2 == 0) ? c_even[j] : c_odd[j];
             const size_t o = (size_t)(l * 3 + j) * 4 * S + e;
-            G1 = cfma(c, src[o + (size_t)n1 * S], G1);
-            G2 = cfma(c, src[o + (size_t)n2 * S], G2);
+            if constexpr (RC) {
+                G1.y = fma(c.y, src[o + (size_t)n1 * S], G1.y);
+                G2.y = fma(c.y, src[o + (size_t)n2 * S], G2.y);
+            } else {
+                G1 = cfma(c, src[o + (size_t)n1 * S], G1);
+                G2 = cfma(c, src[o + (size_t)n2 * S], G2);
+            }
         }
-        const size_t o = ((size_t)lv * S + e) * 2;
-        GD[o] = G1;
-        GD[o + 1] = G2;
+        if constexpr (RC) {
+            GD[(size_t)lv * S + e] = make_double2(G1.y, G2.y);
+        } else {
+            const size_t o = ((size_t)lv * S + e) * 2;
+            GD[o] = G1;
+            GD[o + 1] = G2;
+        }
     }
 }
 
@@ -585,7 +626,8 @@ __global__ __launch_bounds__(256) void k_gsums_dia(const double2 *__restrict__ g
 // the radial CSR index of that entry or -1.
 __global__ void k_build_gdia(const double2 *__restrict__ g, const int *__restrict__ dia_src,
                              const int *__restrict__ tmap, int lmax, int nd, int nhp, int nnzb,
-                             double2 *__restrict__ gs, double2 *__restrict__ gts) {
+                             double2 *__restrict__ gs, double2 *__restrict__ gts, double *__restrict__ gsr,
+                             double *__restrict__ gtsr) {
     const int S = 4 * nd * nhp;
     const long long total = (long long)lmax * 12 * S;
     for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
@@ -604,6 +646,10 @@ __global__ void k_build_gdia(const double2 *__restrict__ g, const int *__restric
         }
         gs[idx] = a;
         gts[idx] = b;
+        if (gsr) {
+            gsr[idx] = a.x;
+            gtsr[idx] = b.x;
+        }
     }
 }
 
@@ -624,35 +670,57 @@ __global__ void k_build_DD(const double2 *__restrict__ D, const int *__restrict_
 
 // DUAL: a second output y2/ypart2 = (D_sel2 + G-part) x from the same G sweeps (beta must be 0); with
 // cH = -1, sel = 1, sel2 = 0 this is the CN pair (S - H) x, (S + H) x, each bit-identical to its own launch.
-// HW = 2: one workgroup of two waves serves both output halves h of a tile (wave h), staging each window once
-// for both; HW = 1: one wave per (tile, h).
-// The G-part sums the source halves hp and parts v (Z0, Z2, W0, W1) in the order (hp, v).
+//
+// A workgroup of four waves owns R row blocks of one kappa, 64*P consecutive outputs of HV output halves h (2: both,
+// 1: one) and one multipole.  Wave v takes part v of V (Z0, Z2, W0, W1): it stages its own windows (no workgroup
+// barrier) and sweeps each for the HV halves, so with HV = 2 a window value read from LDS serves two products.  The
+// four waves' sums meet in LDS, G = ((g0 + g1) + g2) + g3, each wave finishing R/4 rows.  The l = 0 workgroups then
+// form the stationary products, one source half per wave (with HV = 2 also one output half, or for DUAL one of the
+// two operators), D = d(hp=0) + d(hp=1), and y = D + cH G.  Every (R, P, HV) runs these sums in the same order.
+// One wave per half running all four parts in turn (the form before) was a chain of ten staged windows: 31 us at 40
+// blocks of 110 functions, where nothing else fills the chip, and 72 us at 400 blocks of 510 after 42 us of angular
+// kernel.  This form (4 rows, both halves, FUSED, RC) takes 11 and 70 us with no angular kernel before it.  At 400 x
+// 510 it is bound by vector issue (2.0e7 wave instructions, about half the time) and by its loads' way through L1 (the
+// coefficients, then the gathered x): with neither loads nor LDS reads the same instructions take 52 us.
 // FUSED: no V input.  The windows of V_{l,v} (all four parts of a half hp) are formed from x by the coupling
 // lists of phase A (aoff, ack, acf: the lists of k_angular_list), with the same terms in the same order as
 // k_angular_list forms V, so the results are bit-identical to the two-kernel form and V never goes to HBM.
-template <int BW, bool DUAL, class T, int R, int P, int HW = 1, bool FUSED = false>
-__global__ __launch_bounds__(64 * HW) void k_radial_dia(
+// RC: real G-sums and couplings (k_gsums_dia<true>, k_angular_list<..., true>): V holds the angular sums without the
+// couplings' common factor and GD one word (G, G') per entry without its i, so a G product takes two FMAs instead of
+// four and half the coefficient bytes; the factor i (rot 2) or i*i (rot 1) is applied to the finished sum G.  The
+// terms left out are products with zero, so the results equal the complex form's bit for bit.  At 400 x 510 and 4 rows
+// the complex form takes 93 us where the real one takes 58 (both without FUSED), 16 and 11 us at 40 x 110.
+template <int BW, bool DUAL, class T, int R, int P, int HV, bool FUSED, bool RC>
+__global__ __launch_bounds__(256) void k_radial_dia(
     const T *__restrict__ x, const T *__restrict__ V, const T *__restrict__ GD, const T *__restrict__ DD,
     const int *__restrict__ tiles, const int *__restrict__ tile_q, const double *__restrict__ tile_k, int nblk, int n,
     int nh, int nhp, int nseg, int lgrid, int nq, int sel, double cH, double beta, T *__restrict__ y,
     T *__restrict__ ypart, const int *gate, int gstride, const int *__restrict__ tile_b, size_t gd_stride,
     T *__restrict__ y2, T *__restrict__ ypart2, int sel2, const int *__restrict__ aoff = nullptr,
-    const int2 *__restrict__ ack = nullptr, const T *__restrict__ acf = nullptr, int lmax = 0, int nblk1 = 0) {
-    constexpr int SEG = 64 * P, ND = 2 * BW + 1, W = SEG + 2 * BW;
-    constexpr int NT = 64 * HW;  // threads of the workgroup
+    const int2 *__restrict__ ack = nullptr, const T *__restrict__ acf = nullptr, int lmax = 0, int nblk1 = 0, int rot = 0) {
+    constexpr int SEG = 64 * P, ND = 2 * BW + 1, W = SEG + 2 * BW, RW = R / 4;
+    constexpr int WS = P * dia_wp<P>();  // LDS slots of a window
+    static_assert(R % 4 == 0, "each of the four waves finishes R/4 rows");
     using Rt = typename cx<T>::R;
-    __shared__ T sm[(FUSED ? 4 : 1) * R * W];  // FUSED: the windows of the four parts
+    __shared__ T sm[4 * 2 * R * WS];  // a window set per wave; reused for the sums over the waves
     const int lane = threadIdx.x & 63;
-    // (segment, multipole, tile [, half]) with tiles fastest, in XCD order: an XCD works through a few
-    // (segment, multipole) slices at a time, whose G-sums and x windows stay in its L2
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // (segment, tile range, multipole, tile [, half]) with tiles fastest, in XCD order: an XCD works through the
+    // multipoles of about one tile range one after the other, with the G-sums of one or two (segment, multipole)
+    // slices in its L2 at a time, and every XCD has its share of the l = 0 workgroups (which also have the
+    // stationary products)
     const int nt2 = (int)gridDim.x / (nseg * lgrid);
     int rest = xcd_order((int)blockIdx.x, (int)gridDim.x);
-    const int t2 = rest % nt2;
-    rest /= nt2;
-    const int l = rest % lgrid;
-    const int seg = rest / lgrid;
-    const int h = HW == 2 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (t2 & 1);
-    const int tile = HW == 2 ? t2 : t2 >> 1;
+    const int seg = rest / (lgrid * nt2);
+    rest -= seg * lgrid * nt2;
+    const int tc = max(1, nt2 / max(1, 8 / nseg));  // tiles of a range
+    const int rng = min(rest / (lgrid * tc), (nt2 - 1) / tc);
+    rest -= rng * lgrid * tc;
+    const int tn = min(tc, nt2 - rng * tc);
+    const int l = rest / tn;
+    const int t2 = rng * tc + rest % tn;
+    const int h0 = HV == 2 ? 0 : (t2 & 1);
+    const int tile = HV == 2 ? t2 : t2 >> 1;
     const int inst = tile_b[tile];
     GADE_GATED_B(gate, gstride, inst);
     GD += (size_t)inst * gd_stride;  // this instance's G-sums
@@ -664,221 +732,274 @@ __global__ __launch_bounds__(64 * HW) void k_radial_dia(
     for (int i = 0; i < R; i++) rows[i] = tiles[tile * R + i];
     const size_t plane = (size_t)nblk * n;
     const int S = 4 * ND * nhp;
+    T *const win = sm + wave * 2 * R * WS;
 
-    T acc[R][P];
+    T acc[HV][R][P];
+    auto clear = [&]() {
 #pragma unroll
-    for (int i = 0; i < R; i++)
+        for (int hh = 0; hh < HV; hh++)
 #pragma unroll
-        for (int j = 0; j < P; j++) acc[i][j] = czero<T>();
-
-    // window of half hp of 'src' for every row of the tile: position p <-> half index i0 - BW + p.
-    // All loads of the window are issued before the first LDS write.
-    auto stage = [&](const T *src, int hp) {
-        constexpr int NC = (W + NT - 1) / NT;
-        T t[R][NC];
+            for (int i = 0; i < R; i++)
 #pragma unroll
-        for (int i = 0; i < R; i++) {
-            const T *rp = src + (size_t)(rows[i] >= 0 ? rows[i] : 0) * n + hp * nh;
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                const int p = c * NT + (int)threadIdx.x;
-                const int b = i0 - BW + p;
-                t[i][c] = czero<T>();
-                if (rows[i] >= 0 && p < W && b >= 0 && b < nh) t[i][c] = rp[b];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < R; i++)
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                const int p = c * NT + (int)threadIdx.x;
-                if (p < W) sm[i * W + dia_swz<P>(p)] = t[i][c];
-            }
-        __syncthreads();
+                for (int j = 0; j < P; j++) acc[hh][i][j] = czero<T>();
     };
-    // FUSED: the windows of V_{l,v} (v = 0..3) for half hp of every row into sm[v][i][p], each entry the sums
-    // Z0 = sum_e h0_e x_{c_e}, Z2 = sum_e h0_e (k_{c_e} x_{c_e}), W0, W1 likewise with h1, over the row's list
-    // (l) in list order from +0, as k_angular_list forms them (positions outside the half are 0).  Wave h of a
-    // two-wave workgroup takes rows h, h + 2, ...; each lane positions lane + 64c.  The list entries are
-    // wave-uniform (scalar loads); each x value is loaded once for the four sums.
-    auto gather = [&](int hp) {
-        constexpr int NCG = (W + 63) / 64;
+
+    // This wave's windows of half hs of 'src' for every row of the tile into window set ws: position p <-> half index
+    // i0 - BW + p, clamped into the half (the coefficients are zero where a position lies outside it); padding rows
+    // read row 0 of the vector and are never stored.  The loads of RB rows are in flight together.
+    constexpr int NC = (W + 63) / 64;
+    unsigned bc[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c++) bc[c] = min(max(i0 - BW + c * 64 + lane, 0), nh - 1);
+    auto stage = [&](const T *src, int hs, int ws) {
+        constexpr int RB = R < 8 ? R : (P == 1 ? 8 : 4);
+        wave_lds_sync();
+#pragma unroll
+        for (int i1 = 0; i1 < R; i1 += RB) {
+            Rt tr[RB][NC], ti[RB][NC];
+#pragma unroll
+            for (int i = 0; i < RB; i++) {
+                const T *rp = src + (size_t)max(rows[i1 + i], 0) * n + hs * nh;
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    const T v = ld_off(rp, bc[c]);
+                    tr[i][c] = v.x;
+                    ti[i][c] = v.y;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RB; i++)
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    const int p = c * 64 + lane;
+                    if (p < W) win[(ws * R + i1 + i) * WS + dia_slot<P>(p)] = cx<T>::mk(tr[i][c], ti[i][c]);
+                }
+        }
+        wave_lds_sync();
+    };
+    // FUSED: the windows of V_{l,v} (v = 0..3) for both halves of every row into the waves' window sets, each entry the
+    // sums Z0 = sum_e h0_e x_{c_e}, Z2 = sum_e h0_e k_{c_e} x_{c_e}, W0, W1 likewise with h1, over the row's list (l) in
+    // list order from +0, as k_angular_list forms them.  Wave w takes rows w, w + 4, ...; the two halves' windows are
+    // one run of 2 W positions over the lanes.  The list entries are wave-uniform (scalar loads); each x value is
+    // loaded once for the four sums.
+    auto gather = [&]() {
+        constexpr int NCG = (2 * W + 63) / 64;
         constexpr int U = kAngListU;
-        const int w0 = HW == 2 ? h : 0;
-        const T *xh = x + (size_t)inst * nblk1 * n + hp * nh;
-        int bc[NCG];
+        const T *xh = x + (size_t)inst * nblk1 * n;
+        unsigned gc[NCG];
 #pragma unroll
-        for (int c = 0; c < NCG; c++) bc[c] = min(max(i0 - BW + c * 64 + lane, 0), nh - 1);
+        for (int c = 0; c < NCG; c++) {
+            const int p = c * 64 + lane, hs = p >= W;
+            gc[c] = (hs ? nh : 0) + min(max(i0 - BW + p - (hs ? W : 0), 0), nh - 1);
+        }
 #pragma unroll
-        for (int k = 0; k < R / HW; k++) {
-            const int i = w0 + HW * k;
+        for (int k = 0; k < RW; k++) {
+            const int i = wave + 4 * k;
+            const int row = tiles[tile * R + i];
             T z[4][NCG];
 #pragma unroll
             for (int v = 0; v < 4; v++)
 #pragma unroll
                 for (int c = 0; c < NCG; c++) z[v][c] = czero<T>();
-            if (rows[i] >= 0) {
-                const int *off = aoff + (size_t)(rows[i] - inst * nblk1) * lmax + l;
+            if (row >= 0) {
+                const int *off = aoff + (size_t)(row - inst * nblk1) * lmax + l;
                 const int e1 = off[1];
-#pragma unroll 2
+#pragma unroll 1
                 for (int e = off[0]; e < e1; e += U) {
                     T xv[U][NCG];
 #pragma unroll
                     for (int u = 0; u < U; u++) {
                         const T *xc = xh + (size_t)ack[e + u].x * n;
 #pragma unroll
-                        for (int c = 0; c < NCG; c++) xv[u][c] = xc[bc[c]];
+                        for (int c = 0; c < NCG; c++) xv[u][c] = ld_off(xc, gc[c]);
                     }
 #pragma unroll
                     for (int u = 0; u < U; u++) {
-                        const T h0 = acf[2 * (e + u)], h1 = acf[2 * (e + u) + 1];
-                        const Rt kc = (Rt)ack[e + u].y;
 #pragma unroll
-                        for (int c = 0; c < NCG; c++) {
-                            const T kx = cscale(xv[u][c], kc);
-                            z[0][c] = cfma(h0, xv[u][c], z[0][c]);
-                            z[1][c] = cfma(h0, kx, z[1][c]);
-                            z[2][c] = cfma(h1, xv[u][c], z[2][c]);
-                            z[3][c] = cfma(h1, kx, z[3][c]);
-                        }
+                        for (int c = 0; c < NCG; c++)
+                            ang_terms<RC>(xv[u][c], ack[e + u].y, acf + 2 * (e + u), z[0][c], z[1][c], z[2][c],
+                                          z[3][c]);
                     }
                 }
             }
-            if (k == 0) __syncthreads();  // the previous sweeps' reads of sm are done
 #pragma unroll
             for (int c = 0; c < NCG; c++) {
-                const int p = c * 64 + lane;
-                const int b = i0 - BW + p;
-                const bool ok = rows[i] >= 0 && b >= 0 && b < nh;
-                if (p < W) {
+                const int p = c * 64 + lane, hs = p >= W;
+                if (p < 2 * W) {
 #pragma unroll
-                    for (int v = 0; v < 4; v++) sm[(v * R + i) * W + dia_swz<P>(p)] = ok ? z[v][c] : czero<T>();
+                    for (int v = 0; v < 4; v++)
+                        sm[((v * 2 + hs) * R + i) * WS + dia_slot<P>(p - (hs ? W : 0))] = z[v][c];
                 }
             }
         }
         __syncthreads();
     };
-    // acc[i][j] += sum_d M_d[i0 + P*lane + j] * win[i][P*lane + j + d] (win: R windows of W); with two
-    // coefficient streams M = C1 + kap*C2 (pairs), else M = C1.  Coefficients are fetched PF diagonals ahead.
-    auto sweep = [&](const T *win, const T *C, bool pair) {
-        constexpr int PF = P >= 4 ? 2 : P == 2 ? 3 : (R <= 8 ? 8 : 4);  // coefficient diagonals in flight
-        const int stride = pair ? 2 : 1;
-        const T *cp = C + (size_t)(i0 + P * lane) * stride;
+    // acc[hh][i][j] += sum_d M^{hh}_d[i0 + P*lane + j] * win[i][P*lane + j + d] for NH output halves whose
+    // coefficients start hstep apart; with pairs M = C1 + kap*C2, else M = C1.  Coefficients are fetched PF - 1
+    // diagonals ahead.
+    auto sweep = [&](auto nh_tag, int ws, const T *C, size_t hstep, auto pair_tag) {
+        const T *const wn = win + ws * R * WS;
+        constexpr int NH = decltype(nh_tag)::value;
+        constexpr bool PAIR = decltype(pair_tag)::value;
+        constexpr int PF = P >= 4 ? 2 : P == 2 ? 3 : (NH * R <= 16 ? 4 : 3);
+        constexpr int stride = PAIR && !RC ? 2 : 1;
+        const unsigned lo = P * lane * stride;  // this lane's coefficients, from a base common to the wave
         T w[R][P];
 #pragma unroll
         for (int i = 0; i < R; i++)
 #pragma unroll
-            for (int j = 0; j < P; j++) w[i][j] = win[i * W + dia_swz<P>(P * lane + j)];
-        T c1[PF][P], c2[PF][P];
+            for (int j = 0; j < P; j++) w[i][j] = wn[i * WS + (j % P) * dia_wp<P>() + j / P + lane];
+        T c1[PF][NH][P], c2[PF][NH][P];
+        auto fetch = [&](int d) {
 #pragma unroll
-        for (int d = 0; d < PF - 1; d++)
-#pragma unroll
-            for (int j = 0; j < P; j++) {
-                const T *np = cp + (size_t)d * nhp * stride;
-                c1[d][j] = np[j * stride];
-                c2[d][j] = pair ? np[j * stride + 1] : czero<T>();
-            }
-#pragma unroll
-        for (int d = 0; d < ND; d++) {
-            if (d + PF - 1 < ND) {
-                const T *np = cp + (size_t)(d + PF - 1) * nhp * stride;
+            for (int hh = 0; hh < NH; hh++) {
+                const T *np = C + hh * hstep + ((size_t)d * nhp + i0) * stride;
 #pragma unroll
                 for (int j = 0; j < P; j++) {
-                    c1[(d + PF - 1) % PF][j] = np[j * stride];
-                    c2[(d + PF - 1) % PF][j] = pair ? np[j * stride + 1] : czero<T>();
+                    c1[d % PF][hh][j] = ld_off(np, lo + j * stride);
+                    if constexpr (stride == 2) c2[d % PF][hh][j] = ld_off(np, lo + j * stride + 1);
                 }
             }
-            T M[P];
+        };
 #pragma unroll
-            for (int j = 0; j < P; j++) {
-                const T a = c1[d % PF][j], g = c2[d % PF][j];
-                M[j] = pair ? cx<T>::mk(fma(kap, g.x, a.x), fma(kap, g.y, a.y)) : a;
-            }
+        for (int d = 0; d < PF - 1; d++) fetch(d);
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            if (d + PF - 1 < ND) fetch(d + PF - 1);
+            T M[NH][P];
+#pragma unroll
+            for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+                for (int j = 0; j < P; j++) {
+                    const T a = c1[d % PF][hh][j];
+                    if constexpr (PAIR && RC) {
+                        M[hh][j].x = fma(kap, a.y, a.x);
+                    } else if constexpr (PAIR) {
+                        const T b = c2[d % PF][hh][j];
+                        M[hh][j] = cx<T>::mk(fma(kap, b.x, a.x), fma(kap, b.y, a.y));
+                    } else {
+                        M[hh][j] = a;
+                    }
+                }
 #pragma unroll
             for (int i = 0; i < R; i++) {
 #pragma unroll
-                for (int j = 0; j < P; j++) acc[i][j] = cfma(M[j], w[i][j], acc[i][j]);
+                for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+                    for (int j = 0; j < P; j++) acc[hh][i][j] = PAIR && RC ? rfma(M[hh][j].x, w[i][j], acc[hh][i][j])
+                                                   : cfma(M[hh][j], w[i][j], acc[hh][i][j]);
                 if (d + 1 < ND) {
 #pragma unroll
                     for (int j = 0; j + 1 < P; j++) w[i][j] = w[i][j + 1];
-                    w[i][P - 1] = win[i * W + dia_swz<P>(P * lane + P + d)];
+                    w[i][P - 1] = wn[i * WS + ((P + d) % P) * dia_wp<P>() + (P + d) / P + lane];
                 }
             }
         }
     };
-
-    // acc -> output (per-multipole partial, or y itself when there is a single multipole grid)
-#define DIA_EMIT(YO, YPO)                                                     \
-    _Pragma("unroll") for (int i = 0; i < R; i++) {                           \
-        if (rows[i] < 0) continue;                                            \
-        _Pragma("unroll") for (int j = 0; j < P; j++) {                       \
-            const int ip = i0 + P * lane + j;                                 \
-            if (ip >= nh) continue;                                           \
-            const size_t o = (size_t)rows[i] * n + h * nh + ip;               \
-            if (YPO) {                                                        \
-                (YPO)[(size_t)l * plane + o] = acc[i][j];                     \
-            } else {                                                          \
-                T r_ = acc[i][j];                                             \
-                if (beta != 0.0) r_ = cadd(r_, cscale((YO)[o], (Rt)beta));    \
-                (YO)[o] = r_;                                                 \
-            }                                                                 \
-        }                                                                     \
-    }
-
-    if (cH != 0.0) {
-        // k = (hp, v): one copy of the sweep in the code (its own loops are unrolled)
-#pragma unroll 1
-        for (int k = 0; k < 8; k++) {
-            const int hp = k >> 2, v = k & 3;
-            if constexpr (FUSED) {
-                if (v == 0) gather(hp);
-            } else {
-                stage(V + (size_t)(l * 4 + v) * plane, hp);
-            }
-            sweep(FUSED ? sm + v * R * W : sm, GD + ((size_t)(l * 4 + v) * S + (size_t)(2 * h + hp) * ND * nhp) * 2,
-                  true);
-        }
-    }
-    // the second output's unscaled G-part: final for l > 0, parked in its own output slot for l = 0
-    if constexpr (DUAL) {
-        DIA_EMIT(y2, ypart2)
-    }
-    if (cH != 0.0 && cH != 1.0) {
+    // the waves' sums of NH halves side by side in LDS (each in its own window sets)
+    auto share = [&](auto nh_tag) {
+        __syncthreads();
 #pragma unroll
-        for (int i = 0; i < R; i++)
-#pragma unroll
-            for (int j = 0; j < P; j++) acc[i][j] = cscale(acc[i][j], (Rt)cH);
-    }
-    if (l == 0) {
-        for (int hp = 0; hp < 2; hp++) {
-            stage(x, hp);
-            sweep(sm, DD + ((size_t)(sel * nq + q) * S + (size_t)(2 * h + hp) * ND * nhp), false);
-        }
-    }
-    DIA_EMIT(y, ypart)
-    if constexpr (DUAL) {
-        if (l == 0) {
-            // reload this lane's parked values (written by this thread above), then add D_sel2 x
+        for (int hh = 0; hh < decltype(nh_tag)::value; hh++)
 #pragma unroll
             for (int i = 0; i < R; i++)
 #pragma unroll
-                for (int j = 0; j < P; j++) {
-                    const int ip = i0 + P * lane + j;
-                    acc[i][j] = czero<T>();
-                    if (rows[i] >= 0 && ip < nh) {
-                        const size_t o = (size_t)rows[i] * n + h * nh + ip;
-                        acc[i][j] = ypart2 ? ypart2[o] : y2[o];
-                    }
-                }
-            for (int hp = 0; hp < 2; hp++) {
-                stage(x, hp);
-                sweep(sm, DD + ((size_t)(sel2 * nq + q) * S + (size_t)(2 * h + hp) * ND * nhp), false);
-            }
-            DIA_EMIT(y2, ypart2)
+                for (int j = 0; j < P; j++) win[((hh * R + i) * P + j) * 64 + lane] = acc[hh][i][j];
+        __syncthreads();
+    };
+    auto shared_of = [&](int w, int hh, int i, int j) {
+        return sm[w * 2 * R * WS + ((hh * R + i) * P + j) * 64 + lane];
+    };
+    // output (or multipole partial) of this wave's row k, output j, half hh
+    auto emit = [&](T *YO, T *YPO, int k, int j, int hh, T r) {
+        const int row = tiles[tile * R + wave * RW + k];
+        const int ip = i0 + P * lane + j;
+        if (row < 0 || ip >= nh) return;
+        const size_t o = (size_t)row * n + (h0 + hh) * nh + ip;
+        if (YPO) {
+            YPO[(size_t)l * plane + o] = r;
+        } else {
+            if (beta != 0.0) r = cadd(r, cscale(YO[o], (Rt)beta));
+            YO[o] = r;
         }
+    };
+
+    T g[HV][RW][P];  // this wave's rows of the G-part
+#pragma unroll
+    for (int hh = 0; hh < HV; hh++)
+#pragma unroll
+        for (int k = 0; k < RW; k++)
+#pragma unroll
+            for (int j = 0; j < P; j++) g[hh][k][j] = czero<T>();
+    if (cH != 0.0) {
+        clear();
+        if constexpr (FUSED) {
+            gather();
+        } else {
+            stage(V + (size_t)(l * 4 + wave) * plane, 0, 0);
+            stage(V + (size_t)(l * 4 + wave) * plane, 1, 1);
+        }
+#pragma unroll 1
+        for (int hp = 0; hp < 2; hp++)
+            sweep(std::integral_constant<int, HV>{}, hp,
+                  GD + ((size_t)(l * 4 + wave) * S + (size_t)(2 * h0 + hp) * ND * nhp) * (RC ? 1 : 2),
+                  (size_t)2 * ND * nhp * (RC ? 1 : 2), std::true_type{});
+        share(std::integral_constant<int, HV>{});
+#pragma unroll
+        for (int hh = 0; hh < HV; hh++)
+#pragma unroll
+            for (int k = 0; k < RW; k++)
+#pragma unroll
+                for (int j = 0; j < P; j++) {
+                    T s = shared_of(0, hh, wave * RW + k, j);
+#pragma unroll
+                    for (int w = 1; w < 4; w++) s = cadd(s, shared_of(w, hh, wave * RW + k, j));
+                    if constexpr (RC) s = rot == 1 ? cx<T>::mk(-s.x, -s.y) : cx<T>::mk(-s.y, s.x);
+                    g[hh][k][j] = s;
+                }
     }
-#undef DIA_EMIT
+    if (l != 0) {
+#pragma unroll
+        for (int hh = 0; hh < HV; hh++)
+#pragma unroll
+            for (int k = 0; k < RW; k++)
+#pragma unroll
+                for (int j = 0; j < P; j++) {
+                    emit(y, ypart, k, j, hh, cscale(g[hh][k][j], (Rt)cH));
+                    if constexpr (DUAL) emit(y2, ypart2, k, j, hh, g[hh][k][j]);
+                }
+        return;
+    }
+    // stationary products of this wave: source half wave & 1 and, by wave >> 1, the operator (DUAL) or the output
+    // half (HV = 2); with one operator and one half two waves have none
+    const int hpD = wave & 1, part = wave >> 1;
+    constexpr int NHD = DUAL ? HV : 1;
+    __syncthreads();  // the reads of the shared sums are done
+    clear();
+    if (DUAL || HV == 2 || part == 0) {
+        stage(x, hpD, 0);
+        const int hD = DUAL || HV == 1 ? h0 : part;
+        const int sD = DUAL && part == 1 ? sel2 : sel;
+        sweep(std::integral_constant<int, NHD>{}, 0,
+              DD + ((size_t)(sD * nq + q) * S + (size_t)(2 * hD + hpD) * ND * nhp), (size_t)2 * ND * nhp,
+              std::false_type{});
+    }
+    share(std::integral_constant<int, NHD>{});
+#pragma unroll
+    for (int hh = 0; hh < HV; hh++) {
+        const int w0 = DUAL ? 0 : 2 * hh, hs = DUAL ? hh : 0;  // waves (two source halves) and set that hold D
+#pragma unroll
+        for (int k = 0; k < RW; k++)
+#pragma unroll
+            for (int j = 0; j < P; j++) {
+                const int i = wave * RW + k;
+                const T gr = g[hh][k][j];
+                emit(y, ypart, k, j, hh,
+                     cadd(cadd(shared_of(w0, hs, i, j), shared_of(w0 + 1, hs, i, j)), cscale(gr, (Rt)cH)));
+                if constexpr (DUAL)
+                    emit(y2, ypart2, k, j, hh, cadd(cadd(shared_of(2, hs, i, j), shared_of(3, hs, i, j)), gr));
+            }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1250,6 +1371,7 @@ int gade::hip_alloc(void **p, size_t bytes) {
 }
 
 namespace {
+using gade::drop_step_graph;
 using gade::hip_alloc;
 
 template <typename T>
@@ -1305,7 +1427,7 @@ void free_all(gade_model *m) {
                     (void *)m->lu32[2], (void *)m->lu32[3], (void *)m->tw32, (void *)m->mp_r, (void *)m->mp_r0, (void *)m->mp_p,
                     (void *)m->mp_v, (void *)m->mp_y, (void *)m->mp_z, (void *)m->mp_s, (void *)m->mp_t,
                     (void *)m->mp_d, (void *)m->d_mp_ax, (void *)m->d_sc32, (void *)m->d_aoff, (void *)m->d_ack,
-                    (void *)m->d_acf, (void *)m->d_acf32, (void *)m->d_GF, (void *)m->d_DF, (void *)m->d_mg_rows,
+                    (void *)m->d_acf, (void *)m->d_acf32, (void *)m->d_acr, (void *)m->d_acr32, (void *)m->d_gsr, (void *)m->d_gtsr, (void *)m->d_GF, (void *)m->d_DF, (void *)m->d_mg_rows,
                     (void *)m->d_mg_q, (void *)m->d_mg_b, (void *)m->d_mg_k})
         if (p) hipFree(p);
     resolve_pending(m);
@@ -1321,13 +1443,18 @@ bool ang_lds_ok(const gade_model *m, int lb) {
 // the angular kernel with the model's multipole group size (2, 4 or 8 multipoles per block; each V entry is
 // summed over the row's couplings in the same order for every group size)
 template <class T>
-int launch_angular_t(gade_model *m, const T *x, const T *coef, const T *acf, T *V) {
+int launch_angular_t(gade_model *m, const T *x, const T *coef, const T *acf, const T *acr, T *V) {
     const int LB = m->ang_lb;
     dim3 grid(m->nblk, (m->n + kAngThreads - 1) / kAngThreads, (m->lmax + LB - 1) / LB);
     if (m->ang_list) {
-#define GADE_ANGL(LB_)                                                                                        \
-    hipLaunchKernelGGL((k_angular_list<LB_, T>), grid, dim3(kAngThreads), 0, m->stream, x, m->d_aoff, m->d_ack, \
-                       acf, m->n, m->lmax, m->nblk, V, m->gate, m->gstride, m->nblk1)
+#define GADE_ANGL1(LB_, RC_, CF_)                                                                             \
+    hipLaunchKernelGGL((k_angular_list<LB_, T, RC_>), grid, dim3(kAngThreads), 0, m->stream, x, m->d_aoff,     \
+                       m->d_ack, CF_, m->n, m->lmax, m->nblk, V, m->gate, m->gstride, m->nblk1)
+#define GADE_ANGL(LB_)                     \
+    if (m->gd_real && m->radial_kind == 2) \
+        GADE_ANGL1(LB_, true, acr);        \
+    else                                   \
+        GADE_ANGL1(LB_, false, acf)
         switch (LB) {
             case 2: GADE_ANGL(2); break;
             case 4: GADE_ANGL(4); break;
@@ -1337,6 +1464,7 @@ int launch_angular_t(gade_model *m, const T *x, const T *coef, const T *acf, T *
                 return GADE_EINVAL;
         }
 #undef GADE_ANGL
+#undef GADE_ANGL1
         GADE_HIP(hipGetLastError());
         return GADE_OK;
     }
@@ -1358,7 +1486,7 @@ int launch_angular_t(gade_model *m, const T *x, const T *coef, const T *acf, T *
 }
 
 int launch_angular(gade_model *m, const double2 *x) {
-    return launch_angular_t<double2>(m, x, m->d_coef, m->d_acf, m->d_V);
+    return launch_angular_t<double2>(m, x, m->d_coef, m->d_acf, m->d_acr, m->d_V);
 }
 
 template <class T>
@@ -1377,11 +1505,11 @@ bool dia_shape_ok(int r, int p) {
     return (r == 4 && (p == 1 || p == 2 || p == 4)) || (r == 8 && (p == 1 || p == 2)) || (r == 16 && p == 1);
 }
 
-// phase A inside the banded radial kernel (its windows formed from x and the coupling lists, no V): the
-// FP64 form when the MFMA kernel is off, the FP32 form of the mixed solve always (it has no MFMA kernel)
+// phase A inside the banded radial kernel (its windows formed from x and the coupling lists, no V): built for the
+// real form of the couplings; otherwise the two kernels run, with the same results
 template <class T>
 bool ang_in_radial(const gade_model *m) {
-    return m->ang_fused && m->radial_kind == 2 && (sizeof(T) == sizeof(float2) || !m->radial_mfma);
+    return m->ang_fused && m->radial_kind == 2 && m->gd_real;
 }
 
 // tile shapes with a fused form: one row's window sums per lane fit the registers for up to 2 outputs per lane
@@ -1395,46 +1523,44 @@ int launch_dia(gade_model *m, int lgrid, const T *x, const T *V, const T *GD, co
     const int P = m->dia_p;
     const int nseg = (m->nh + 64 * P - 1) / (64 * P);
     const bool fused = ang_in_radial<T>(m);
-    // the paired (DUAL) two-kernel form runs one wave per output half whatever the model's choice: with both
-    // halves in one workgroup it measured 30-40 % slower at every shape (its two accumulator sets per wave)
-    const int hw = DUAL && !fused ? 1 : m->dia_hw;
-    const dim3 grid((unsigned)m->ndtiles * (2 / hw) * nseg * lgrid);
-    const T *acf = sizeof(T) == sizeof(float2) ? (const T *)m->d_acf32 : (const T *)m->d_acf;
+    const int hv = m->gd_real ? m->dia_hw : 2;  // the complex form is built for both halves per workgroup
+    const dim3 grid((unsigned)m->ndtiles * (2 / hv) * nseg * lgrid);
+    const T *acr = sizeof(T) == sizeof(float2) ? (const T *)m->d_acr32 : (const T *)m->d_acr;
     if (fused && !fused_shape_ok(m->dia_r, P)) {
         gade::set_error("the fused angular + radial form needs at most 2 outputs per lane");
         return GADE_EINVAL;
     }
-#define GADE_DIA1(R_, P_, HW_, F_)                                                                               \
-    hipLaunchKernelGGL((k_radial_dia<kDiaBW, DUAL, T, R_, P_, HW_, F_>), grid, dim3(64 * HW_), 0, m->stream, x, V, \
+#define GADE_DIA1(R_, P_, HV_, F_, RC_, CF_)                                                                     \
+    hipLaunchKernelGGL((k_radial_dia<kDiaBW, DUAL, T, R_, P_, HV_, F_, RC_>), grid, dim3(256), 0, m->stream, x, V, \
                        GD, DD, m->d_dtiles, m->d_dtile_q, m->d_dtile_k, m->nblk, m->n, m->nh, m->nhp, nseg, lgrid, \
                        m->nq, sel, cH, beta, y, yp, m->gate, m->gstride, m->d_dtile_b, m->gd_stride, y2, yp2, sel2, \
-                       m->d_aoff, (const int2 *)m->d_ack, acf, m->lmax, m->nblk1)
-#define GADE_DIA(R_, P_)                 \
-    if (hw == 2 && fused) {              \
-        GADE_DIA1(R_, P_, 2, true);      \
-    } else if (fused) {                  \
-        GADE_DIA1(R_, P_, 1, true);      \
-    } else if (hw == 2) {                \
-        GADE_DIA1(R_, P_, 2, false);     \
-    } else {                             \
-        GADE_DIA1(R_, P_, 1, false);     \
+                       m->d_aoff, (const int2 *)m->d_ack, CF_, m->lmax, m->nblk1, m->h_rot)
+#define GADE_DIA(R_, P_, F_)                         \
+    if (!m->gd_real) {                               \
+        GADE_DIA1(R_, P_, 2, false, false, nullptr); \
+    } else if (hv == 2) {                            \
+        GADE_DIA1(R_, P_, 2, F_, true, acr);         \
+    } else {                                         \
+        GADE_DIA1(R_, P_, 1, F_, true, acr);         \
+    }
+#define GADE_DIAF(R_, P_)           \
+    if (fused) {                    \
+        GADE_DIA(R_, P_, true);     \
+    } else {                        \
+        GADE_DIA(R_, P_, false);    \
     }
     switch (m->dia_r * 10 + P) {
-        case 82: GADE_DIA(8, 2); break;
-        case 42: GADE_DIA(4, 2); break;
-        case 44:
-            if (hw == 2)
-                GADE_DIA1(4, 4, 2, false);
-            else
-                GADE_DIA1(4, 4, 1, false);
-            break;
-        case 81: GADE_DIA(8, 1); break;
-        case 41: GADE_DIA(4, 1); break;
-        case 161: GADE_DIA(16, 1); break;
+        case 82: GADE_DIAF(8, 2); break;
+        case 42: GADE_DIAF(4, 2); break;
+        case 44: GADE_DIA(4, 4, false); break;
+        case 81: GADE_DIAF(8, 1); break;
+        case 41: GADE_DIAF(4, 1); break;
+        case 161: GADE_DIAF(16, 1); break;
         default:
             gade::set_error("unsupported banded tile shape (rows, outputs per lane)");
             return GADE_EINVAL;
     }
+#undef GADE_DIAF
 #undef GADE_DIA
 #undef GADE_DIA1
     GADE_HIP(hipGetLastError());
@@ -1575,19 +1701,46 @@ int setup_dia(gade_model *m) {
     GADE_TRY(upload(&m->d_dia_src, dia_src.data(), dia_src.size()));
     GADE_TRY(hip_alloc((void **)&m->d_gs, sizeof(double2) * (size_t)lmax * 12 * S));
     GADE_TRY(hip_alloc((void **)&m->d_gts, sizeof(double2) * (size_t)lmax * 12 * S));
+    if (m->g_real) {
+        GADE_TRY(hip_alloc((void **)&m->d_gsr, sizeof(double) * (size_t)lmax * 12 * S));
+        GADE_TRY(hip_alloc((void **)&m->d_gtsr, sizeof(double) * (size_t)lmax * 12 * S));
+    }
     m->gd_stride = (size_t)lmax * 4 * S * 2;
     GADE_TRY(hip_alloc((void **)&m->d_GD, sizeof(double2) * m->gd_stride * m->B));
     GADE_HIP(hipMemset(m->d_GD, 0, sizeof(double2) * m->gd_stride * m->B));  // f = 0 until the first set_time
     GADE_TRY(hip_alloc((void **)&m->d_DD, sizeof(double2) * (size_t)3 * m->nq * S));
     const long long tg = (long long)lmax * 12 * S, td = (long long)3 * m->nq * S;
     hipLaunchKernelGGL(k_build_gdia, dim3(grid_for(tg, 256)), dim3(256), 0, m->stream, m->d_g, m->d_dia_src, m->d_tmap,
-                       lmax, m->nd, m->nhp, m->nnzb, m->d_gs, m->d_gts);
+                       lmax, m->nd, m->nhp, m->nnzb, m->d_gs, m->d_gts, m->d_gsr, m->d_gtsr);
     hipLaunchKernelGGL(k_build_DD, dim3(grid_for(td, 256)), dim3(256), 0, m->stream, m->d_D, m->d_dia_src,
                        m->d_ell_pos, m->nq, m->ellw, n, m->nd, m->nhp, m->d_DD);
     GADE_HIP(hipGetLastError());
     GADE_HIP(hipStreamSynchronize(m->stream));
-    GADE_TRY(kappa_tiles(m, kDiaR, &m->d_dtiles, &m->d_dtile_q, &m->d_dtile_k, &m->ndtiles, &m->d_dtile_b));
+    GADE_TRY(kappa_tiles(m, m->dia_r, &m->d_dtiles, &m->d_dtile_q, &m->d_dtile_k, &m->ndtiles, &m->d_dtile_b));
     m->dia_ok = true;
+    return GADE_OK;
+}
+
+// the banded tile shape (rows per tile, outputs per lane, halves per workgroup) and the fused form in use
+int set_shape(gade_model *m, int r, int p, int hw, int fused) {
+    if (r == m->dia_r && p == m->dia_p && hw == m->dia_hw && fused == m->ang_fused) return GADE_OK;
+    drop_step_graph(m);
+    if (m->dia_ok && r != m->dia_r)
+        GADE_TRY(kappa_tiles(m, r, &m->d_dtiles, &m->d_dtile_q, &m->d_dtile_k, &m->ndtiles, &m->d_dtile_b));
+    m->dia_r = r;
+    m->dia_p = p;
+    m->dia_hw = hw;
+    m->ang_fused = fused;
+    return GADE_OK;
+}
+
+// the same as a caller's choice
+int use_shape(gade_model *m, int r, int p, int hw, int fused) {
+    GADE_TRY(set_shape(m, r, p, hw, fused));
+    m->par_r = r;
+    m->par_p = p;
+    m->par_hw = hw;
+    m->par_fused = fused;
     return GADE_OK;
 }
 
@@ -1651,6 +1804,34 @@ Coef6 coef_of(const gade_model *m, int b) {
 // mixed-precision form
 bool dia_gsums_needed(const gade_model *m) { return !m->radial_mfma || m->precision == 1; }
 
+// The banded kernels' real form serves when every radial coupling is real, the angular ones are real up to one common
+// factor 1 or i, and f(t) is real (every coupling file and every pulse of the physics; gade_set_time takes complex
+// f(t)).  It holds half the coefficient bytes and half the products of the complex form, which runs otherwise; the
+// results are the same.  The Hall-row angular kernel and the matrix-core kernel have the complex form only.
+// ft: [..][12] pulse coefficients of every instance (and step) concerned
+bool real_form(const gade_model *m, const std::vector<double> &ft) {
+    if (!m->g_real || !m->h_rot || !m->ang_list || m->radial_mfma) return false;
+    for (size_t i = 1; i < ft.size(); i += 2)
+        if (ft[i] != 0.0) return false;
+    return true;
+}
+
+// the banded G-sums that follow are written, and every product until the next ones runs, in this form
+void set_form(gade_model *m, bool real) {
+    if (m->gd_real == real) return;
+    drop_step_graph(m);  // its launches are of the other form
+    m->gd_real = real;
+}
+
+void run_gsums_dia(gade_model *m, dim3 grid, const CoefGroup &cg, int b0, const Coef6 *table, const int *gctl) {
+    if (m->gd_real)
+        hipLaunchKernelGGL((k_gsums_dia<true, double>), grid, dim3(256), 0, m->stream, m->d_gsr, m->d_gtsr, cg, b0,
+                           m->gd_stride, m->lmax, m->nd, m->nhp, m->d_GD, m->gate, m->gstride, table, gctl, m->B);
+    else
+        hipLaunchKernelGGL((k_gsums_dia<false, double2>), grid, dim3(256), 0, m->stream, m->d_gs, m->d_gts, cg, b0,
+                           m->gd_stride, m->lmax, m->nd, m->nhp, m->d_GD, m->gate, m->gstride, table, gctl, m->B);
+}
+
 // G-sums of the current f(t) of every instance in the layout of the active radial kernel
 int launch_gsums(gade_model *m, bool ell) {
     Prof pr(m, "gsums", GADE_PROF_GSUMS);
@@ -1661,14 +1842,13 @@ int launch_gsums(gade_model *m, bool ell) {
     } else {
         long long total = (long long)m->lmax * 16 * m->nd * m->nhp;  // (l, v, qd, d, ip)
         const long long totf = (long long)m->lmax * 16 * m->nmi * 5 * kMfmaFrag;
+        set_form(m, real_form(m, m->ft));
         for (int b0 = 0; b0 < m->B; b0 += kCoefGroup) {
             const int nb = std::min(kCoefGroup, m->B - b0);
             CoefGroup cg{};
             for (int k = 0; k < nb; k++) cg.c[k] = coef_of(m, b0 + k);
             if (dia_gsums_needed(m))
-                hipLaunchKernelGGL(k_gsums_dia, dim3(grid_for(total, 256, 4096), nb), dim3(256), 0, m->stream,
-                                   m->d_gs, m->d_gts, cg, b0, m->gd_stride, m->lmax, m->nd, m->nhp, m->d_GD, m->gate,
-                                   m->gstride, (const Coef6 *)nullptr, (const int *)nullptr, m->B);
+                run_gsums_dia(m, dim3(grid_for(total, 256, 4096), nb), cg, b0, nullptr, nullptr);
             if (m->radial_mfma)
                 hipLaunchKernelGGL(k_gsums_frag, dim3(grid_for(totf, 256, 4096), nb), dim3(256), 0, m->stream,
                                    m->d_gs, m->d_gts, cg, b0, m->gf_stride, m->lmax, m->nd, m->nhp, m->nmi, m->d_GF,
@@ -1883,6 +2063,17 @@ int gade_model_create_batch(const gade_inputs_t *in, int B, double h, double dt,
             }
         }
     m->h_aoff.back() = (int)ack.size();
+    // the couplings' real form (real_form): lists without their common factor 1 or i, and whether the radial ones
+    // are real
+    bool h_re = true, h_im = true;
+    for (size_t i = 0; i < acf.size(); i += 2) {
+        h_re = h_re && acf[i + 1] == 0.0;
+        h_im = h_im && acf[i] == 0.0;
+    }
+    m->h_rot = h_im ? 1 : h_re ? 2 : 0;
+    m->g_real = true;
+    for (int i = 0; i < 24 * lmax && m->g_real; i++)
+        for (int k = 0; k < m->nnzb && m->g_real; k++) m->g_real = in->g[i][2 * k + 1] == 0.0;
     if (ack.empty()) {  // no coupling: one unread entry keeps the uploads non-empty
         ack.push_back(make_int2(0, 0));
         acf.assign(4, 0.0);
@@ -1944,6 +2135,16 @@ int gade_model_create_batch(const gade_inputs_t *in, int B, double h, double dt,
         (rc = upload(&m->d_acf, (const double2 *)acf.data(), acf.size() / 2)) ||
         (rc = upload(&m->d_diag, diag.data(), diag.size())))
         return fail(rc);
+    if (m->h_rot) {
+        std::vector<double> acr(acf.size());  // (h0, h1, h0 k, h1 k) per entry
+        for (size_t e = 0; e < ack.size(); e++)
+            for (int j = 0; j < 2; j++) {
+                const double hv = acf[4 * e + 2 * j + (m->h_rot == 1 ? 1 : 0)];
+                acr[4 * e + j] = hv;
+                acr[4 * e + 2 + j] = hv * ack[e].y;
+            }
+        if ((rc = upload(&m->d_acr, (const double2 *)acr.data(), acr.size() / 2))) return fail(rc);
+    }
     if ((rc = hip_alloc((void **)&m->d_GE, sizeof(double2) * (size_t)lmax * 8 * ellw * n)) ||
         (rc = hip_alloc((void **)&m->d_D, sizeof(double2) * (size_t)3 * m->nq * ellw * n)) ||
         (rc = hip_alloc((void **)&m->d_V, sizeof(double2) * (size_t)lmax * 4 * m->N)) ||
@@ -2307,7 +2508,6 @@ void drop_step_graph(gade_model *m) {
     memset(m->graph_key, 0, sizeof(m->graph_key));
 }
 }  // namespace gade
-using gade::drop_step_graph;
 namespace {
 
 int ensure_step_buffers(gade_model *m, int nsteps) {
@@ -2393,6 +2593,7 @@ int mp_setup(gade_model *m) {
     GADE_TRY(hip_alloc((void **)&m->d_coef32, sizeof(float2) * nco));
     const size_t nacf = 2 * (size_t)m->h_aoff.back();  // (h0, h1) per list entry
     GADE_TRY(hip_alloc((void **)&m->d_acf32, sizeof(float2) * std::max<size_t>(nacf, 1)));
+    if (m->d_acr) GADE_TRY(hip_alloc((void **)&m->d_acr32, sizeof(float2) * std::max<size_t>(nacf, 1)));
     for (auto &f : m->lu32) GADE_TRY(hip_alloc((void **)&f, sizeof(float2) * nlu));
     for (float2 **v : {&m->mp_r, &m->mp_r0, &m->mp_p, &m->mp_v, &m->mp_y, &m->mp_z, &m->mp_s, &m->mp_t, &m->mp_d})
         GADE_TRY(hip_alloc((void **)v, sizeof(float2) * N));
@@ -2401,6 +2602,9 @@ int mp_setup(gade_model *m) {
     conv(m->d_DD, m->d_DD32, nDD);
     conv(m->d_coef, m->d_coef32, nco);
     if (nacf) conv(m->d_acf, m->d_acf32, nacf);
+    if (nacf && m->d_acr)
+        hipLaunchKernelGGL(k_acr32, dim3(grid_for((long long)nacf / 2, 256, 8192)), dim3(256), 0, m->stream,
+                           (int)(nacf / 2), (const double2 *)m->d_acr, (const int2 *)m->d_ack, m->d_acr32);
     conv(m->pre->d_Linv, m->lu32[0], nlu);
     conv(m->pre->d_Uinv, m->lu32[1], nlu);
     conv(m->pre->d_Loff, m->lu32[2], nlu);
@@ -2419,7 +2623,8 @@ int mp_setup(gade_model *m) {
 int apply32_async(gade_model *m, const float2 *x, float2 *y) {
     if (!ang_in_radial<float2>(m)) {
         Prof pr(m, "angular_f32", GADE_PROF_ANGULAR);
-        GADE_TRY(launch_angular_t<float2>(m, x, (const float2 *)m->d_coef32, (const float2 *)m->d_acf32, m->d_V32));
+        GADE_TRY(launch_angular_t<float2>(m, x, (const float2 *)m->d_coef32, (const float2 *)m->d_acf32,
+                                          (const float2 *)m->d_acr32, m->d_V32));
     }
     const int lgrid = m->lmax;
     float2 *yp = lgrid > 1 ? m->d_ypart32 : nullptr;
@@ -2507,9 +2712,9 @@ int enqueue_sweeps(gade_model *m, double2 *psi, int J) {
 
 // the FP32 G-sums of the step (after the FP64 ones), per instance under the step-prologue gate
 int mp_convert_gsums(gade_model *m) {
-    hipLaunchKernelGGL(k_to_f32, dim3(grid_for((long long)m->gd_stride, 256, 4096), m->B), dim3(256), 0, m->stream,
-                       (long long)m->gd_stride, m->gd_stride, (const double2 *)m->d_GD, m->d_GD32, m->gate,
-                       m->gstride);
+    const long long n = (long long)m->gd_stride / (m->gd_real ? 2 : 1);  // words of an instance in use
+    hipLaunchKernelGGL(k_to_f32, dim3(grid_for(n, 256, 4096), m->B), dim3(256), 0, m->stream, n, m->gd_stride,
+                       (const double2 *)m->d_GD, m->d_GD32, m->gate, m->gstride);
     GADE_HIP(hipGetLastError());
     return GADE_OK;
 }
@@ -2580,9 +2785,7 @@ int launch_gsums_window(gade_model *m) {
     long long total = (long long)m->lmax * 16 * m->nd * m->nhp;  // (l, v, qd, d, ip)
     CoefGroup cg{};
     if (dia_gsums_needed(m))
-        hipLaunchKernelGGL(k_gsums_dia, dim3(grid_for(total, 256, 4096), m->B), dim3(256), 0, m->stream, m->d_gs,
-                           m->d_gts, cg, 0, m->gd_stride, m->lmax, m->nd, m->nhp, m->d_GD, m->gate, m->gstride,
-                           (const Coef6 *)m->d_cfwin, m->d_gctl, m->B);
+        run_gsums_dia(m, dim3(grid_for(total, 256, 4096), m->B), cg, 0, (const Coef6 *)m->d_cfwin, m->d_gctl);
     if (m->radial_mfma) {
         const long long totf = (long long)m->lmax * 16 * m->nmi * 5 * kMfmaFrag;
         hipLaunchKernelGGL(k_gsums_frag, dim3(grid_for(totf, 256, 4096), m->B), dim3(256), 0, m->stream, m->d_gs,
@@ -2785,6 +2988,7 @@ int cn_run_device(gade_model *m, double2 *psi, const double *times, int nsteps, 
         const bool table = m->radial_kind == 2;
         if (table) {
             GADE_TRY(ensure_cfwin(m, W));
+            set_form(m, real_form(m, ft));
             Coef6 *tab = (Coef6 *)m->h_cfwin;
             for (int w = 0; w < W; w++) {
                 std::copy(ft.data() + (size_t)12 * B * w, ft.data() + (size_t)12 * B * (w + 1), m->ft.begin());
@@ -3155,20 +3359,12 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
     const int sv_window = m->window, sv_batch = m->iter_batch, sv_profile = m->profile, sv_k = m->last_k;
     const int sv_r = m->dia_r, sv_p = m->dia_p, sv_lb = m->ang_lb, sv_hw = m->dia_hw, sv_fused = m->ang_fused;
     const bool sv_graph = m->use_graph;
-    auto set_shape = [&](int r, int pp, int lb, int hw, int fused) -> int {
-        if (lb != m->ang_lb || hw != m->dia_hw || fused != m->ang_fused) {
+    auto shape = [&](int r, int pp, int lb, int hw, int fused) -> int {
+        if (lb != m->ang_lb) {
             drop_step_graph(m);
             m->ang_lb = lb;
-            m->dia_hw = hw;
-            m->ang_fused = fused;
         }
-        if (!m->dia_ok || (r == m->dia_r && pp == m->dia_p)) return GADE_OK;
-        drop_step_graph(m);
-        if (r != m->dia_r)
-            GADE_TRY(kappa_tiles(m, r, &m->d_dtiles, &m->d_dtile_q, &m->d_dtile_k, &m->ndtiles, &m->d_dtile_b));
-        m->dia_r = r;
-        m->dia_p = pp;
-        return GADE_OK;
+        return set_shape(m, r, pp, hw, fused);
     };
     auto restore = [&]() {
         m->window = sv_window;
@@ -3176,7 +3372,7 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
         m->use_graph = sv_graph;
         m->profile = sv_profile;
         m->last_k = sv_k;
-        (void)set_shape(sv_r, sv_p, sv_lb, sv_hw, sv_fused);
+        (void)shape(sv_r, sv_p, sv_lb, sv_hw, sv_fused);
         const int rc = copy_state(false);
         (void)hipStreamSynchronize(m->stream);
         (void)hipFree(work);
@@ -3197,8 +3393,8 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
         if (c == nshape && nshape > 0) {
             for (size_t k = 1; k < nshape; k++)
                 if (cands[k].ms < cands[best_shape].ms) best_shape = k;
-            if (int rc = set_shape(cands[best_shape].dia_r, cands[best_shape].dia_p, cands[best_shape].ang_lb,
-                                   cands[best_shape].dia_hw, cands[best_shape].fused)) {
+            if (int rc = shape(cands[best_shape].dia_r, cands[best_shape].dia_p, cands[best_shape].ang_lb,
+                               cands[best_shape].dia_hw, cands[best_shape].fused)) {
                 restore();
                 return rc;
             }
@@ -3209,8 +3405,7 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
             cands[c].ang_lb = m->ang_lb;
             cands[c].dia_hw = m->dia_hw;
             cands[c].fused = m->ang_fused;
-        } else if (int rc = set_shape(cands[c].dia_r, cands[c].dia_p, cands[c].ang_lb, cands[c].dia_hw,
-                                      cands[c].fused)) {
+        } else if (int rc = shape(cands[c].dia_r, cands[c].dia_p, cands[c].ang_lb, cands[c].dia_hw, cands[c].fused)) {
             restore();
             return rc;
         }
@@ -3265,8 +3460,9 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
     m->window = cands[pick].window;
     m->iter_batch = cands[pick].iter_batch;
     m->use_graph = cands[pick].graph != 0;
-    GADE_TRY(set_shape(cands[pick].dia_r, cands[pick].dia_p, cands[pick].ang_lb, cands[pick].dia_hw,
-                       cands[pick].fused));
+    GADE_TRY(shape(cands[pick].dia_r, cands[pick].dia_p, cands[pick].ang_lb, cands[pick].dia_hw, cands[pick].fused));
+    if (m->radial_kind == 2)
+        GADE_TRY(use_shape(m, cands[pick].dia_r, cands[pick].dia_p, cands[pick].dia_hw, cands[pick].fused));
     if (report)
         for (size_t c = 0; c < cands.size() && c < GADE_TUNE_MAX; c++) {
             double *r = report + (size_t)GADE_TUNE_COLS * c;
@@ -3492,8 +3688,11 @@ int gade_set_param(gade_model_t *m, const char *name, int value) {
             gade::set_error("ang_list must be 0 (Hall rows) or 1 (coupling lists)");
             return GADE_EINVAL;
         }
-        if (m->ang_list != value) drop_step_graph(m);
-        m->ang_list = value;
+        if (m->ang_list != value) {
+            drop_step_graph(m);
+            m->ang_list = value;
+            if (m->radial_kind == 2) GADE_TRY(launch_gsums(m, false));  // the current f(t) in that form's layout
+        }
         return GADE_OK;
     }
     if (!strcmp(name, "ang_lb")) {
@@ -3508,13 +3707,11 @@ int gade_set_param(gade_model_t *m, const char *name, int value) {
     if (!strcmp(name, "ang_fused")) {
         // 1: the banded radial kernel forms each V window from x and the coupling lists (no angular kernel, no
         // V in HBM; bit-identical results), 0: the angular kernel writes V and the radial kernel reads it
-        if ((value != 0 && value != 1) || (value == 1 && !fused_shape_ok(m->dia_r, m->dia_p))) {
+        if ((value != 0 && value != 1) || (value == 1 && !fused_shape_ok(m->par_r, m->par_p))) {
             gade::set_error("ang_fused must be 0 or 1 (1 needs a tile shape with at most 2 outputs per lane)");
             return GADE_EINVAL;
         }
-        if (value != m->ang_fused) drop_step_graph(m);
-        m->ang_fused = value;
-        return GADE_OK;
+        return use_shape(m, m->par_r, m->par_p, m->par_hw, value);
     }
     if (!strcmp(name, "dia_halves")) {
         // output halves per banded workgroup: 1 (one wave per half) or 2 (two waves share each window)
@@ -3522,19 +3719,17 @@ int gade_set_param(gade_model_t *m, const char *name, int value) {
             gade::set_error("dia_halves must be 1 or 2");
             return GADE_EINVAL;
         }
-        if (value != m->dia_hw) drop_step_graph(m);
-        m->dia_hw = value;
-        return GADE_OK;
+        return use_shape(m, m->par_r, m->par_p, value, m->par_fused);
     }
     if (!strcmp(name, "dia_rows") || !strcmp(name, "dia_outputs")) {
         const bool rows = name[4] == 'r';
-        const int r = rows ? value : m->dia_r, pp = rows ? m->dia_p : value;
+        const int r = rows ? value : m->par_r, pp = rows ? m->par_p : value;
         if (!dia_shape_ok(r, pp)) {
             gade::set_error("banded tile shape (dia_rows, dia_outputs) must be (4,1), (4,2), (4,4), (8,1), (8,2) "
                             "or (16,1)");
             return GADE_EINVAL;
         }
-        if (m->ang_fused && !fused_shape_ok(r, pp)) {
+        if (m->par_fused && !fused_shape_ok(r, pp)) {
             gade::set_error("the fused angular + radial form (ang_fused 1) has no (4,4) tile shape");
             return GADE_EINVAL;
         }
@@ -3542,12 +3737,7 @@ int gade_set_param(gade_model_t *m, const char *name, int value) {
             gade::set_error("the radial pattern is not banded");
             return GADE_EINVAL;
         }
-        drop_step_graph(m);
-        if (rows && r != m->dia_r)
-            GADE_TRY(kappa_tiles(m, r, &m->d_dtiles, &m->d_dtile_q, &m->d_dtile_k, &m->ndtiles, &m->d_dtile_b));
-        m->dia_r = r;
-        m->dia_p = pp;
-        return GADE_OK;
+        return use_shape(m, r, pp, m->par_hw, m->par_fused);
     }
     if (!strcmp(name, "precision")) {
         if (value != 0 && value != 1) {
@@ -3683,7 +3873,7 @@ int gade_get_param(const gade_model_t *m, const char *name, int *value) {
         return GADE_OK;
     }
     if (!strcmp(name, "dia_rows")) {
-        *value = m->dia_r;
+        *value = m->par_r;
         return GADE_OK;
     }
     if (!strcmp(name, "ang_list")) {
@@ -3699,15 +3889,15 @@ int gade_get_param(const gade_model_t *m, const char *name, int *value) {
         return GADE_OK;
     }
     if (!strcmp(name, "dia_halves")) {
-        *value = m->dia_hw;
+        *value = m->par_hw;
         return GADE_OK;
     }
     if (!strcmp(name, "ang_fused")) {
-        *value = m->ang_fused;
+        *value = m->par_fused;
         return GADE_OK;
     }
     if (!strcmp(name, "dia_outputs")) {
-        *value = m->dia_p;
+        *value = m->par_p;
         return GADE_OK;
     }
     if (!strcmp(name, "lg_features")) {

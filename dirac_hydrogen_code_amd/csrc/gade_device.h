@@ -21,6 +21,13 @@ __device__ __forceinline__ double2 cfma(double2 a, double2 b, double2 acc) {
     acc.y = fma(a.y, b.x, acc.y);
     return acc;
 }
+// acc + a*b, a real
+__device__ __forceinline__ double2 rfma(double a, double2 b, double2 acc) {
+    return make_double2(fma(a, b.x, acc.x), fma(a, b.y, acc.y));
+}
+__device__ __forceinline__ float2 rfma(float a, float2 b, float2 acc) {
+    return make_float2(fmaf(a, b.x, acc.x), fmaf(a, b.y, acc.y));
+}
 // acc + conj(a)*b
 __device__ __forceinline__ double2 cfmaconj(double2 a, double2 b, double2 acc) {
     acc.x = fma(a.x, b.x, acc.x);

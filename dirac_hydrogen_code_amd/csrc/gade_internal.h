@@ -112,6 +112,14 @@ struct gade_model {
     int2 *d_ack = nullptr;
     double2 *d_acf = nullptr;
     float2 *d_acf32 = nullptr;     // FP32 copy (mixed precision)
+    // real form of the couplings (banded kernels): h_rot 1 when every angular coupling is imaginary, 2 when every one
+    // is real, 0 otherwise; the lists without that factor, (h0, h1), (h0 k, h1 k) per entry; g_real: every radial coupling is real
+    int h_rot = 0;
+    bool g_real = false;
+    double2 *d_acr = nullptr;
+    float2 *d_acr32 = nullptr;
+    bool gd_real = false;          // form of the current G-sums d_GD, and so of the banded products
+    double *d_gsr = nullptr, *d_gtsr = nullptr;  // real parts of d_gs, d_gts
     int ang_list = 1;              // phase A from the coupling lists (1) or from the Hall rows (0)
     int *d_diag = nullptr;         // [hnnz] 1 when orig_row == orig_col
     // kappa-grouped row tiles for the radial phase
@@ -125,13 +133,18 @@ struct gade_model {
     int nh = 0, nhp = 0, nd = 0, ndtiles = 0;
     int *d_dia_src = nullptr;      // [4][nd][nhp] radial CSR index or -1
     double2 *d_gs = nullptr, *d_gts = nullptr;  // [lmax][3][4][4][nd][nhp] DIA-ordered couplings
-    double2 *d_GD = nullptr;       // [B][lmax][4][4][nd][nhp][2] kappa-folded G-sum pairs
+    double2 *d_GD = nullptr;       // [B][lmax][4][4][nd][nhp][2] kappa-folded G-sum pairs (gd_real: one word (G, G'))
     double2 *d_DD = nullptr;       // [3][nq][4][nd][nhp] diagonal operators
     int *d_dtiles = nullptr, *d_dtile_q = nullptr;
     double *d_dtile_k = nullptr;
     int *d_dtile_b = nullptr;      // instance of each tile (tiles never mix instances)
-    int dia_r = 8, dia_p = 1;      // banded tile shape: rows per tile, outputs per lane
-    int dia_hw = 1;                // output halves per banded workgroup (2: both halves share each window)
+    // banded tile shape in use: rows per tile, outputs per lane, output halves per workgroup (2: both halves share
+    // each window).  par_*: what a caller has set or tuned; until then the shape in use is the model's own choice:
+    // 4 rows, 1 output, both halves, fused, the fastest of the shapes at every size measured (apply, us, against the
+    // next shapes fused and the best unfused one: 40 x 110: 20, 22.5, 22; 5 x 60 x 76: 26, 27, 29.5; 400 x 510: 85,
+    // 117, 111)
+    int dia_r = 4, dia_p = 1, dia_hw = 2;
+    int par_r = 8, par_p = 1, par_hw = 1, par_fused = 0;
     // FP64 banded radial phase on the matrix cores: waves of two 8-row halves of one kappa each
     bool mfma_ok = false;          // the banded pattern fits the MFMA kernel (set up)
     int radial_mfma = 0;           // 1: FP64 radial products on MFMA (k_radial_mfma), 0: k_radial_dia (default)
@@ -142,7 +155,7 @@ struct gade_model {
     int *d_mg_rows = nullptr, *d_mg_q = nullptr, *d_mg_b = nullptr;  // [nmg][16], [nmg][2], [nmg]
     double *d_mg_k = nullptr;      // [nmg][2] kappa of each half
     int ang_lb = 2;                // multipoles per angular block
-    int ang_fused = 0;             // 1: the banded radial kernel forms its V windows from x (no V in HBM)
+    int ang_fused = 1;             // 1: the banded radial kernel forms its V windows from x (no V in HBM)
     int psolve_ch = 16;            // preconditioner level height (16 or 32 rows)
     size_t gd_stride = 0;          // GD entries per instance
     double2 *d_V = nullptr;        // [lmax][4][nblk][n]

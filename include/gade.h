@@ -301,8 +301,10 @@ int gade_assembled_get(gade_model_t *m, int *Ap, int *Ai, int *Ai_sub_map, doubl
  *             GADE_GUESS_LEARNED the learned guess;
  *   "dia_rows", "dia_outputs"  banded tile shape: rows per tile and outputs per
  *             lane, (8,1) by default; (4,1), (4,2), (4,4), (8,2), (16,1) also;
- *   "dia_halves"  1 (default): one wave per output half of a tile; 2: both halves
- *             in one two-wave workgroup sharing each staged window;
+ *   "dia_halves"  1 (default): one output half of a tile per workgroup; 2: both halves
+ *             in one workgroup sharing each staged window;
+ *             (until one of these or "ang_fused" is set or tuned, the model runs the
+ *             shape it finds fastest, (4,1) with both halves and the angular phase inside);
  *   "ang_lb"  multipoles per angular block (2 by default; 4, 8);
  *   "ang_list"  1 (default): angular phase over the coupling lists; 0: Hall rows;
  *   "radial_mfma"  1: FP64 banded products on the matrix cores (0 by default);
