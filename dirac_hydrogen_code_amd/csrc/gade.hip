@@ -1307,49 +1307,59 @@ __global__ void k_full_submap(const int *hAp, const int *subAp, const int *fAp, 
     }
 }
 
-// Hfull.Ax in row order: entry e of row (R, a) -> Hall nz p = hAp[R] + e/len, sub entry k
-// (tools/gpu_solver.cu:84-135 evaluated per destination so the stores are coalesced)
+// Hfull.Ax in row order: entry (pos, t) of row (R, a) -> Hall nz p = hAp[R] + pos, sub entry k = subAp[a] + t
+// (tools/gpu_solver.cu:84-135 evaluated per destination so the stores are coalesced).  A workgroup owns two radial rows
+// a (of at most kMaxSlots = 32 entries, one per half wave) and every gridDim.y-th block row R: it stages the 8 LM G-sums
+// of the rows' entries in LDS once, and its waves take the Hall entries of R, each the same one in both halves, so that
+// the couplings come by scalar loads and a multipole with a zero coupling is skipped by the whole wave.  It was one
+// workgroup per (R, a), whose G loads (up to 8 LM of 16 bytes per entry, a radial row apart) came from L2 each time:
+// 388 us for the 13.4 M entries of 104 x 210 with 4 multipoles, now 90 (the stores alone, 215 MB, take about 45).
 template <int LM>
 __global__ __launch_bounds__(256) void k_assemble(const int *__restrict__ hAp, const int *__restrict__ hAi,
                                                   const int *__restrict__ kap, const double2 *__restrict__ coef,
                                                   const int *__restrict__ diag, const int *__restrict__ subAp,
-                                                  const int *__restrict__ ell_pos, const double2 *__restrict__ GE,
-                                                  const double2 *__restrict__ D, const int *__restrict__ blk_q,
-                                                  const int *__restrict__ fAp, int nblk, int n, int ellw, int nq,
-                                                  double2 *__restrict__ fAx) {
-    long long row = blockIdx.x + (long long)blockIdx.y * gridDim.x;
-    if (row >= (long long)nblk * n) return;
-    const int R = (int)(row / n), a = (int)(row % n);
+                                                  const double2 *__restrict__ GE, const double2 *__restrict__ D,
+                                                  const int *__restrict__ blk_q, const int *__restrict__ fAp, int nblk,
+                                                  int n, int ellw, int nq, double2 *__restrict__ fAx) {
+    __shared__ double2 sg[8 * LM][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int a = min(2 * (int)blockIdx.x + (lane >> 5), n - 1), t = lane & 31;
     const int len = subAp[a + 1] - subAp[a];
-    const int nb = hAp[R + 1] - hAp[R];
-    const double ki = kap[R];
+    const bool on = t < len && 2 * (int)blockIdx.x + (lane >> 5) < n;
     const size_t slab = (size_t)ellw * n;
-    const double2 *Dq = D + ((size_t)0 * nq + blk_q[R]) * slab;  // S + ihdt H0: take the H0 part below
-    const double2 *Sq = D + ((size_t)2 * nq + blk_q[R]) * slab;
-    const int base = fAp[row];
-    for (int e = threadIdx.x; e < nb * len; e += blockDim.x) {
-        const int pos = e / len, t = e % len;
-        const int p = hAp[R] + pos;
-        const double kj = kap[hAi[p]];
-        const int k = subAp[a] + t;
-        const size_t ep = (size_t)ell_pos[k];
-        double2 val = make_double2(0, 0);
-        if (diag[p]) val = csub(Dq[ep], Sq[ep]);  // ihdt*(h00 + k h01 + k^2 h02 + k^3 h03)
-        const double2 *cp = coef + (size_t)p * LM * 2;
+    const size_t ep = (size_t)(on ? t : 0) * n + a;
+    for (int lm = wave; lm < 8 * LM; lm += 4) sg[lm][lane] = GE[(size_t)lm * slab + ep];
+    __syncthreads();
+    for (int R = blockIdx.y; R < nblk; R += gridDim.y) {
+        const int p0 = hAp[R], nb = hAp[R + 1] - p0;
+        const double ki = kap[R];
+        double2 *out = fAx + fAp[(size_t)R * n + a] + t;
+        for (int pos = wave; pos < nb; pos += 4) {
+            const int p = p0 + pos;
+            const double kj = kap[hAi[p]];
+            double2 val = make_double2(0, 0);
+            if (diag[p]) {  // ihdt*(h00 + k h01 + k^2 h02 + k^3 h03) = (S + ihdt H0) - S
+                const size_t o = (size_t)blk_q[R] * slab + ep;
+                val = csub(D[o], D[(size_t)2 * nq * slab + o]);
+            }
+            const double2 *cp = coef + (size_t)p * LM * 2;
 #pragma unroll
-        for (int l = 0; l < LM; l++) {
-            const double2 *G = GE + (size_t)(l * 8) * slab + ep;
-            double2 h0 = cp[2 * l], h1 = cp[2 * l + 1];
-            if (cnz(h0)) {
-                double2 g = cadd(cadd(G[0], cscale(G[slab], ki)), cadd(cscale(G[2 * slab], kj), cscale(G[3 * slab], ki * kj)));
-                val = cfma(h0, g, val);
+            for (int l = 0; l < LM; l++) {
+                const double2 h0 = cp[2 * l], h1 = cp[2 * l + 1];
+                if (cnz(h0)) {
+                    const double2 g = cadd(cadd(sg[8 * l][lane], cscale(sg[8 * l + 1][lane], ki)),
+                                           cadd(cscale(sg[8 * l + 2][lane], kj), cscale(sg[8 * l + 3][lane], ki * kj)));
+                    val = cfma(h0, g, val);
+                }
+                if (cnz(h1)) {
+                    const double2 g =
+                        cadd(cadd(sg[8 * l + 4][lane], cscale(sg[8 * l + 5][lane], kj)),
+                             cadd(cscale(sg[8 * l + 6][lane], ki), cscale(sg[8 * l + 7][lane], ki * kj)));
+                    val = cfma(h1, g, val);
+                }
             }
-            if (cnz(h1)) {
-                double2 g = cadd(cadd(G[4 * slab], cscale(G[5 * slab], kj)), cadd(cscale(G[6 * slab], ki), cscale(G[7 * slab], ki * kj)));
-                val = cfma(h1, g, val);
-            }
+            if (on) out[(size_t)pos * len] = val;
         }
-        fAx[base + e] = val;
     }
 }
 
@@ -1407,7 +1417,7 @@ void free_all(gade_model *m) {
                     m->d_hAp, m->d_hAi, m->d_kap, m->d_blk_q, m->d_coef, m->d_diag, m->d_tiles, m->d_tile_q, m->d_tile_k,
                     m->d_V, m->d_ypart, m->d_flag, m->d_dia_src, m->d_gs, m->d_gts, m->d_GD, m->d_DD, m->d_dtiles, m->d_dtile_q, m->d_dtile_k,
                     m->r, m->r0, m->v, m->p, m->y, m->z, m->s, m->t, m->tmp, m->d_sc, m->d_part, m->d_part2,
-                    m->d_fAp, m->d_fAi, m->d_fAx, m->d_SAp, m->d_SAi, m->d_SAx};
+                    m->d_fAp, m->d_fAi, m->d_fAx, m->d_SAp, m->d_SAi, m->d_SAx, m->d_subAp};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (m->h_sc) hipHostFree(m->h_sc);
@@ -3566,23 +3576,22 @@ int gade_assembled_setup(gade_model_t *m) {
 int gade_assembled_timedep_into(gade_model_t *m, const int *Ap_dev, double *Ax_dev) {
     if (!m || !Ap_dev || !Ax_dev) return GADE_EINVAL;
     if (m->radial_kind == 2) GADE_TRY(launch_gsums(m, true));  // the fused path keeps only the DIA layout
-    int *d_subAp = nullptr;
-    GADE_TRY(upload(&d_subAp, m->rad_Ap.data(), m->rad_Ap.size()));
-    const long long N = m->N;
-    dim3 g2((unsigned)std::min<long long>(N, 65535), (unsigned)((N + 65534) / 65535));
+    if (!m->d_subAp) GADE_TRY(upload(&m->d_subAp, m->rad_Ap.data(), m->rad_Ap.size()));
+    // several workgroups per compute unit, each staging its radial rows' G-sums for many block rows
+    const int na = (m->n + 1) / 2;
+    const dim3 grid((unsigned)na, (unsigned)std::max(1, std::min(m->nblk, (4096 + na - 1) / na)));
     {
         Prof pr(m, "assemble", GADE_PROF_ASSEMBLE);
 #define ASM(LM) \
-    case LM: hipLaunchKernelGGL(k_assemble<LM>, g2, dim3(256), 0, m->stream, m->d_hAp, m->d_hAi, m->d_kap, m->d_coef, m->d_diag, d_subAp, m->d_ell_pos, m->d_GE, m->d_D, m->d_blk_q, Ap_dev, m->nblk, m->n, m->ellw, m->nq, (double2 *)Ax_dev); break;
+    case LM: hipLaunchKernelGGL(k_assemble<LM>, grid, dim3(256), 0, m->stream, m->d_hAp, m->d_hAi, m->d_kap, m->d_coef, m->d_diag, m->d_subAp, m->d_GE, m->d_D, m->d_blk_q, Ap_dev, m->nblk, m->n, m->ellw, m->nq, (double2 *)Ax_dev); break;
         switch (m->lmax) {
             ASM(1) ASM(2) ASM(3) ASM(4) ASM(5) ASM(6) ASM(7) ASM(8) ASM(9) ASM(10) ASM(11) ASM(12) ASM(13) ASM(14) ASM(15) ASM(16)
-            default: (void)hipFree(d_subAp); return GADE_EINVAL;
+            default: return GADE_EINVAL;
         }
 #undef ASM
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-    (void)hipFree(d_subAp);
     if (e != hipSuccess) {
         gade::set_error(std::string("k_assemble: ") + hipGetErrorString(e));
         return GADE_EHIP;
@@ -3606,12 +3615,8 @@ int gade_assembled_spmv(gade_model_t *m, const double *x, double *y, double alph
     {
         Prof pr(m, "csr_spmv", GADE_PROF_CSR_SPMV);
         hipLaunchKernelGGL(k_csr_spmv, dim3(grid), dim3(256), 0, m->stream, m->d_fAp, m->d_fAi, m->d_fAx,
-                           (const double2 *)x, N, make_double2(alpha, 0), make_double2(beta, 0), (double2 *)y);
-    }
-    if (with_S) {
-        Prof pr(m, "csr_spmv_S", GADE_PROF_CSR_SPMV);
-        hipLaunchKernelGGL(k_csr_spmv, dim3(grid), dim3(256), 0, m->stream, m->d_SAp, m->d_SAi, m->d_SAx,
-                           (const double2 *)x, N, make_double2(1.0, 0), make_double2(1.0, 0), (double2 *)y);
+                           (const double2 *)x, N, make_double2(alpha, 0), make_double2(beta, 0), (double2 *)y,
+                           with_S ? m->d_SAp : nullptr, m->d_SAi, m->d_SAx);
     }
     GADE_HIP(hipGetLastError());
     GADE_HIP(hipStreamSynchronize(m->stream));

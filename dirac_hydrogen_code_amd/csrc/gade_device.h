@@ -704,14 +704,10 @@ __global__ __launch_bounds__(kRedThreads) void k_bicg_fin(int nparts, const doub
     ctl[CT_PSKIP] = 1;
 }
 
-// y = alpha A x + beta y for a CSR matrix: one wave per row, streaming loads.
-[[maybe_unused]] static __global__ __launch_bounds__(256) void k_csr_spmv(const int *__restrict__ Ap, const int *__restrict__ Ai,
-                                                  const double2 *__restrict__ Ax, const double2 *__restrict__ x,
-                                                  long long nrows, double2 alpha, double2 beta,
-                                                  double2 *__restrict__ y) {
-    const long long row = (blockIdx.x * (long long)blockDim.x + threadIdx.x) >> 6;
-    const int lane = threadIdx.x & 63;
-    if (row >= nrows) return;
+// sum of a CSR row's products over the wave (every lane), streaming loads
+__device__ __forceinline__ double2 csr_row(const int *__restrict__ Ap, const int *__restrict__ Ai,
+                                           const double2 *__restrict__ Ax, const double2 *__restrict__ x, long long row,
+                                           int lane) {
     const int b = Ap[row], e = Ap[row + 1];
     double2 acc0 = make_double2(0, 0), acc1 = make_double2(0, 0);
     int i = b + lane;
@@ -728,14 +724,26 @@ __global__ __launch_bounds__(kRedThreads) void k_bicg_fin(int nparts, const doub
         int c0 = __builtin_nontemporal_load(Ai + i);
         acc0 = cfma(a0, x[c0], acc0);
     }
-    double re = wave_sum(acc0.x + acc1.x), im = wave_sum(acc0.y + acc1.y);
+    return make_double2(wave_sum(acc0.x + acc1.x), wave_sum(acc0.y + acc1.y));
+}
+
+// y = alpha A x + beta y for a CSR matrix, plus B x when B is given: one wave per row.
+[[maybe_unused]] static __global__ __launch_bounds__(256) void k_csr_spmv(
+    const int *__restrict__ Ap, const int *__restrict__ Ai, const double2 *__restrict__ Ax,
+    const double2 *__restrict__ x, long long nrows, double2 alpha, double2 beta, double2 *__restrict__ y,
+    const int *__restrict__ Bp = nullptr, const int *__restrict__ Bi = nullptr, const double2 *__restrict__ Bx = nullptr) {
+    const long long row = (blockIdx.x * (long long)blockDim.x + threadIdx.x) >> 6;
+    const int lane = threadIdx.x & 63;
+    if (row >= nrows) return;
+    const double2 ax = csr_row(Ap, Ai, Ax, x, row, lane);
+    const double2 bx = Bp ? csr_row(Bp, Bi, Bx, x, row, lane) : make_double2(0, 0);
     if (lane == 0) {
-        double2 res = cmul(alpha, make_double2(re, im));
+        double2 res = cmul(alpha, ax);
         if (beta.x != 0.0 || beta.y != 0.0) res = cadd(res, cmul(beta, y[row]));
+        if (Bp) res = cadd(bx, res);
         y[row] = res;
     }
 }
-
 
 // ---------------------------------------------------------------------------
 // preconditioner: banded LU per distinct kappa (interleaved radial order)

@@ -176,6 +176,7 @@ struct gade_model {
     bool asm_ready = false;
     long long nnz_full = 0;
     int *d_fAp = nullptr, *d_fAi = nullptr;
+    int *d_subAp = nullptr;        // radial row pointers
     double2 *d_fAx = nullptr;
     int *d_SAp = nullptr, *d_SAi = nullptr;
     double2 *d_SAx = nullptr;
