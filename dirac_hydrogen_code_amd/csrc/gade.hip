@@ -2507,6 +2507,9 @@ struct GateScope {
 
 }  // namespace
 namespace gade {
+template <class T>
+int launch_tw(const gade_blocklu *lu, const T *F, const T *b, T *x, hipStream_t stream, const int *gate, int gstride,
+              int nblk1);
 // the step graph holds device addresses of the model's buffers: drop it before any of them is replaced
 void drop_step_graph(gade_model *m) {
     // a replay may still be running on the model's stream: let it finish before the executable goes
@@ -2657,11 +2660,7 @@ int psolve32_async(gade_model *m, const float2 *b, float2 *x) {
     Prof pr(m, "psolve_f32", GADE_PROF_PSOLVE);
     const gade_blocklu *lu = m->pre;
     if (lu->d_TW) {
-        hipLaunchKernelGGL((k_psolve_tw<4, float2>), dim3(lu->norder), dim3(128), sizeof(float2) * (size_t)lu->nch * 16,
-                           m->stream, b, x, lu->d_order, lu->d_blk_q, lu->ilv, (const float2 *)m->tw32, lu->n,
-                           lu->nch, lu->tw_m, m->gate, m->gstride, m->nblk1);
-        GADE_HIP(hipGetLastError());
-        return GADE_OK;
+        return gade::launch_tw(lu, (const float2 *)m->tw32, b, x, m->stream, m->gate, m->gstride, m->nblk1);
     }
     // 32-row levels (mixed precision needs 16- or 32-row levels and a band of at most 16)
     const size_t shq = sizeof(float2) * ((size_t)lu->nch * lu->ch + lu->ch);
@@ -4109,6 +4108,18 @@ int twisted_factors(const std::vector<double2> &AB, int nq, int n, int band, std
     return GADE_OK;
 }
 
+// Blocks per workgroup of the twisted solve: one while the blocks do not fill the compute units much more than once,
+// then two, then four.  Measured, us with 1 / 2 / 4 (events; blocks x rows of each):
+//   40 x 110: 8.3 / 9.3 / 12.8        300 x 76: 8.4 / 8.6 / 11.5       400 x 510: 27.5 / 23.3 / 35.1
+//   640 x 110: 14.7 / 11.2 / 13.3     800 x 510: 49 / 31 / 36          1280 x 110: 26 / 15.8 / 15.6
+//   1600 x 510: 87 / 52 / 45          2560 x 110: 45 / 28 / 18.8       3200 x 510: 148 / 91 / 59
+// (fewer where the blocks would not fit 64 KB of LDS together)
+int psolve_blocks(int nblk, int nch) {
+    int nr = nblk <= 320 ? 1 : nblk < 1280 ? 2 : 4;
+    while (nr > 1 && sizeof(double2) * (size_t)nch * 16 * nr > 64 * 1024) nr /= 2;
+    return nr;
+}
+
 int blocklu_build(int nblk, int n, const int *rAp, const int *rAi, int nq, const int *blk_q,
                   const std::vector<double2> &Pq, hipStream_t stream, gade_blocklu **out, int min_ch) {
     const int nnzb = rAp[n];
@@ -4190,7 +4201,10 @@ int blocklu_build(int nblk, int n, const int *rAp, const int *rAi, int nq, const
     lu->npw = (int)wb.size() / G;
     // one block per wave: the blocks of one distinct factor go to one XCD (workgroups are dealt to the 8
     // XCDs round-robin), so each XCD's L2 holds the factors of its own kappa groups only
+    // (the twisted solve takes nr blocks of one factor per workgroup, -1 pads: entries of nr blocks)
     constexpr int kXcd = 8;
+    const int nr = lu->d_TW ? psolve_blocks(nblk, lu->nch) : 1;
+    lu->nr = nr;
     std::vector<std::vector<int>> bins(kXcd);
     {
         std::vector<std::vector<int>> groups(nq);
@@ -4203,20 +4217,40 @@ int blocklu_build(int nblk, int n, const int *rAp, const int *rAi, int nq, const
             for (int x = 1; x < kXcd; x++)
                 if (bins[x].size() < bins[best].size()) best = x;
             bins[best].insert(bins[best].end(), groups[q].begin(), groups[q].end());
+            while (bins[best].size() % nr) bins[best].push_back(-1);
         }
     }
     size_t maxlen = 0;
     for (auto &b : bins) maxlen = std::max(maxlen, b.size());
     std::vector<int> order(maxlen * kXcd, -1);
     for (int x = 0; x < kXcd; x++)
-        for (size_t k = 0; k < bins[x].size(); k++) order[k * kXcd + x] = bins[x][k];
-    lu->norder = (int)order.size();
+        for (size_t k = 0; k < bins[x].size(); k++) order[((k / nr) * kXcd + x) * nr + k % nr] = bins[x][k];
+    lu->norder = (int)order.size() / nr;
     if ((rc = upload(&lu->d_wblocks, wb.data(), wb.size())) || (rc = upload(&lu->d_blk_q, blk_q, (size_t)nblk)) ||
         (rc = upload(&lu->d_order, order.data(), order.size())))
         return fail(rc);
     *out = lu;
     return GADE_OK;
 }
+
+template <class T>
+int launch_tw(const gade_blocklu *lu, const T *F, const T *b, T *x, hipStream_t stream, const int *gate, int gstride,
+              int nblk1) {
+    const size_t sh = sizeof(T) * (size_t)lu->nch * 16 * lu->nr;
+#define TW(PF_, NR_)                                                                                                  \
+    hipLaunchKernelGGL((k_psolve_tw<PF_, T, NR_>), dim3(lu->norder), dim3(128), sh, stream, b, x, lu->d_order,        \
+                       lu->d_blk_q, lu->ilv, F, lu->n, lu->nch, lu->tw_m, gate, gstride, nblk1)
+    switch (lu->nr) {
+        case 1: TW(4, 1); break;
+        case 2: TW(2, 2); break;
+        default: TW(1, 4); break;
+    }
+#undef TW
+    GADE_HIP(hipGetLastError());
+    return GADE_OK;
+}
+template int launch_tw<float2>(const gade_blocklu *, const float2 *, const float2 *, float2 *, hipStream_t, const int *,
+                               int, int);
 
 int blocklu_solve_async(const gade_blocklu *lu, const double2 *b, double2 *x, hipStream_t stream, const int *gate,
                         int gstride, int nblk1) {
@@ -4225,12 +4259,8 @@ int blocklu_solve_async(const gade_blocklu *lu, const double2 *b, double2 *x, hi
         return GADE_EINVAL;
     }
     if (lu->d_TW) {
-        // twisted factorization: one block per workgroup of two waves, meeting at level tw_m
-        const size_t sh = sizeof(double2) * (size_t)lu->nch * 16;
-        hipLaunchKernelGGL((k_psolve_tw<4, double2>), dim3(lu->norder), dim3(128), sh, stream, b, x, lu->d_order,
-                           lu->d_blk_q, lu->ilv, lu->d_TW, lu->n, lu->nch, lu->tw_m, gate, gstride, nblk1);
-        GADE_HIP(hipGetLastError());
-        return GADE_OK;
+        // twisted factorization, meeting at level tw_m
+        return launch_tw(lu, (const double2 *)lu->d_TW, b, x, stream, gate, gstride, nblk1);
     }
     const bool quad = (lu->ch == 16 || lu->ch == 32) && lu->band <= 16;
     if (!quad && gstride != 0) {

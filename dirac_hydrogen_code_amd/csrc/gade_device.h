@@ -970,7 +970,7 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// x = P^{-1} b from the twisted factorization over 16-row levels (twisted_factors): one block per workgroup of
+// x = P^{-1} b from the twisted factorization over 16-row levels (twisted_factors): NR blocks per workgroup of
 // two waves.  Wave 0 runs the top levels (g_c = b_c - X_c g_{c-1}, c = 1..m-1), wave 1 the bottom ones
 // (h_c = b_c - X_c h_{c+1}, c = nch-2..m+1) at the same time; after a barrier wave 0 solves the meeting level
 // x_m = Y_m (b_m - X_m g_{m-1} - W_m h_{m+1}); after another, both run their back sweeps outwards
@@ -979,20 +979,32 @@ __device__ __forceinline__ void wave_lds_sync() {
 // a wave takes terms 4k..4k+3 of row i, summed over the quad with DPP; b, g/h and x share one LDS array in
 // place (a level reads its neighbour's values and then writes its own rows).  The factors of the level PF
 // steps ahead load as soon as a register slot is free; the meeting level's factors load at the start.
-template <int PF, class T = double2>
+// NR blocks of one kappa per workgroup share the factors: each is loaded once for the NR chains, which also fill each
+// other's LDS and FP64 latencies.  The factors of a block (4 nch matrices of 4 KB) come from L2, so with many blocks
+// their traffic is the bound: 3200 blocks of 510 rows read 1.6 GB with NR = 1, 148 us against 59 with NR = 4.  Few
+// blocks are bound by the chain of levels; there NR = 1 has more of them side by side (psolve_blocks).  PF, the levels
+// of factors in flight, is 4, 2 and 1 for NR = 1, 2 and 4: more costs registers and so waves.
+template <int PF, class T, int NR>
 __global__ __launch_bounds__(128) void k_psolve_tw(const T *__restrict__ b, T *__restrict__ xo,
                                                    const int *__restrict__ order, const int *__restrict__ blk_q,
                                                    int ilv, const T *__restrict__ F, int n, int nch, int m,
                                                    const int *gate = nullptr, int gstride = 0, int nblk1 = 1) {
     constexpr int CH = 16, MS = CH * CH;
     extern __shared__ __align__(16) char smem_raw[];
-    T *v = reinterpret_cast<T *>(smem_raw);  // [nch*16], interleaved order
+    T *const v = reinterpret_cast<T *>(smem_raw);  // [NR][nch*16], interleaved order
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane >> 2, k = lane & 3;
-    const int r = order[blockIdx.x];
-    if (r < 0) return;  // padding slot (whole workgroup)
-    GADE_GATED_B(gate, gstride, r / nblk1);
-    const int q = blk_q[r];
     const int ntot = nch * CH;
+    // blocks of this workgroup (-1: padding, or an instance that is gated off); the first one is always there
+    int r[NR];
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < NR; j++) {
+        r[j] = order[blockIdx.x * NR + j];
+        if (r[j] >= 0 && gated(gate, gstride, r[j] / nblk1)) r[j] = -1;
+        any = any || r[j] >= 0;
+    }
+    if (!any) return;
+    const int q = blk_q[order[blockIdx.x * NR]];
     // terms 4k..4k+3 of row i of matrix j of level c
     const T *Fq = F + (size_t)q * nch * 4 * MS + (size_t)(4 * k) * CH + i;
     auto ld4 = [&](int c, int j, T (&f)[4]) {
@@ -1017,33 +1029,55 @@ __global__ __launch_bounds__(128) void k_psolve_tw(const T *__restrict__ b, T *_
     for (int u = 0; u < PF; u++)
         if (u < nf) ld4(fwd_level(u), 0, ff[u]);
     // b: eight loads per thread in flight before the LDS writes
-    const T *bb = b + (size_t)r * n;
-    for (int c0 = 0; c0 < ntot; c0 += 128 * 8) {
-        T t[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int c = c0 + 128 * u + (int)threadIdx.x;
-            t[u] = c < n ? bb[natural_index(c, n, ilv)] : czero<T>();
-        }
+    for (int j = 0; j < NR; j++) {
+        const T *bb = b + (size_t)max(r[j], 0) * n;
+        for (int c0 = 0; c0 < ntot; c0 += 128 * 8) {
+            T t[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int c = c0 + 128 * u + (int)threadIdx.x;
-            if (c < ntot) v[c] = t[u];
+            for (int u = 0; u < 8; u++) {
+                const int c = c0 + 128 * u + (int)threadIdx.x;
+                t[u] = c < n && r[j] >= 0 ? bb[natural_index(c, n, ilv)] : czero<T>();
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int c = c0 + 128 * u + (int)threadIdx.x;
+                if (c < ntot) v[j * ntot + c] = t[u];
+            }
         }
     }
     __syncthreads();
+    // v_c[row i] of every block becomes base - the quad's sum of t
+    auto finish = [&](T (&t)[NR], int c, bool subtract) {
+#pragma unroll
+        for (int j = 0; j < NR; j++) t[j] = quad_sum(t[j]);
+        if (k == 0) {
+#pragma unroll
+            for (int j = 0; j < NR; j++) {
+                T *o = v + j * ntot + c * CH + i;
+                *o = subtract ? csub(*o, t[j]) : t[j];
+            }
+        }
+    };
+    // t[j] += f (x the four terms at level c)
+    auto terms = [&](const T (&f)[4], int c, T (&t)[NR]) {
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) t[j] = cfma(f[e], v[j * ntot + c * CH + 4 * k + e], t[j]);
+    };
     // forward: v_c -= X_c v_{c+dir}
     for (int s0 = 0; s0 < nf; s0 += PF) {
 #pragma unroll
         for (int u = 0; u < PF; u++) {
             const int s = s0 + u;
             if (s >= nf) break;
-            const int c = fwd_level(s), nbr = (c + dir) * CH;
-            T t = czero<T>();
+            const int c = fwd_level(s);
+            T t[NR];
 #pragma unroll
-            for (int e = 0; e < 4; e++) t = cfma(ff[u][e], v[nbr + 4 * k + e], t);
-            t = quad_sum(t);
-            if (k == 0) v[c * CH + i] = csub(v[c * CH + i], t);
+            for (int j = 0; j < NR; j++) t[j] = czero<T>();
+            terms(ff[u], c + dir, t);
+            finish(t, c, true);
             wave_lds_sync();
             if (s + PF < nf) ld4(fwd_level(s + PF), 0, ff[u]);
         }
@@ -1058,23 +1092,17 @@ __global__ __launch_bounds__(128) void k_psolve_tw(const T *__restrict__ b, T *_
     __syncthreads();
     if (wave == 0) {
         // meeting level: v_m = Y_m (v_m - X_m v_{m-1} - W_m v_{m+1})
-        T t = czero<T>();
-        if (m >= 1) {
+        T t[NR];
 #pragma unroll
-            for (int e = 0; e < 4; e++) t = cfma(fm[0][e], v[(m - 1) * CH + 4 * k + e], t);
-        }
-        if (m + 1 < nch) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) t = cfma(fm[1][e], v[(m + 1) * CH + 4 * k + e], t);
-        }
-        t = quad_sum(t);
-        if (k == 0) v[m * CH + i] = csub(v[m * CH + i], t);
+        for (int j = 0; j < NR; j++) t[j] = czero<T>();
+        if (m >= 1) terms(fm[0], m - 1, t);
+        if (m + 1 < nch) terms(fm[1], m + 1, t);
+        finish(t, m, true);
         wave_lds_sync();
-        T y = czero<T>();
 #pragma unroll
-        for (int e = 0; e < 4; e++) y = cfma(fm[2][e], v[m * CH + 4 * k + e], y);
-        y = quad_sum(y);
-        if (k == 0) v[m * CH + i] = y;
+        for (int j = 0; j < NR; j++) t[j] = czero<T>();
+        terms(fm[2], m, t);
+        finish(t, m, false);
     }
     __syncthreads();
     // back: v_c = Y_c v_c - Z_c v_{c-dir}
@@ -1083,14 +1111,16 @@ __global__ __launch_bounds__(128) void k_psolve_tw(const T *__restrict__ b, T *_
         for (int u = 0; u < PF; u++) {
             const int s = s0 + u;
             if (s >= nb) break;
-            const int c = back_level(s), nbr = (c - dir) * CH;
-            T t = czero<T>();
+            const int c = back_level(s);
+            T t[NR];
 #pragma unroll
-            for (int e = 0; e < 4; e++) t = cfma(fb[u][0][e], v[c * CH + 4 * k + e], t);
+            for (int j = 0; j < NR; j++) t[j] = czero<T>();
+            terms(fb[u][0], c, t);
+            T z[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) t = cfma(cx<T>::mk(-fb[u][1][e].x, -fb[u][1][e].y), v[nbr + 4 * k + e], t);
-            t = quad_sum(t);
-            if (k == 0) v[c * CH + i] = t;
+            for (int e = 0; e < 4; e++) z[e] = cx<T>::mk(-fb[u][1][e].x, -fb[u][1][e].y);
+            terms(z, c - dir, t);
+            finish(t, c, false);
             wave_lds_sync();
             if (s + PF < nb) {
                 ld4(back_level(s + PF), 1, fb[u][0]);
@@ -1099,7 +1129,10 @@ __global__ __launch_bounds__(128) void k_psolve_tw(const T *__restrict__ b, T *_
         }
     }
     __syncthreads();
-    for (int c = threadIdx.x; c < n; c += 128) xo[(size_t)r * n + natural_index(c, n, ilv)] = v[c];
+#pragma unroll
+    for (int j = 0; j < NR; j++)
+        if (r[j] >= 0)
+            for (int c = threadIdx.x; c < n; c += 128) xo[(size_t)r[j] * n + natural_index(c, n, ilv)] = v[j * ntot + c];
 }
 
 // x = P^{-1} b: one wave serves 64/CH blocks (preferably of one kappa), lane =

@@ -53,7 +53,8 @@ struct gade_blocklu {
     double2 *d_AB = nullptr, *d_Linv = nullptr, *d_Uinv = nullptr, *d_Loff = nullptr, *d_Uoff = nullptr;
     int *d_blk_q = nullptr, *d_wblocks = nullptr, *d_flag = nullptr;
     int *d_order = nullptr;  // one block per wave, -1 pads; blocks of one factor on one XCD
-    int norder = 0;
+    int norder = 0;          // workgroups
+    int nr = 1;              // blocks per workgroup of the twisted solve
     // twisted factorization over 16-row levels (k_psolve_tw): [q][level][X, Y, Z, W][16 x 16, column-major],
     // meeting level tw_m; null when the levels are not 16 rows or the band exceeds 16
     double2 *d_TW = nullptr;
