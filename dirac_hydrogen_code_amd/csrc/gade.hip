@@ -550,7 +550,11 @@ __global__ __launch_bounds__(256) void k_radial_sum(const T *__restrict__ ypart,
 // at a time.  The per-multipole results go to ypart and are summed in a fixed
 // order.
 // ---------------------------------------------------------------------------
-constexpr int kDiaSegMax = 256; // longest output run of a wave (64 lanes x 4 outputs); nhp is a multiple of it
+// A half's coefficients are padded to nhp, a multiple of 64.  A wave with P outputs per lane may read up to 64 (P - 1)
+// entries past a diagonal's last one, for outputs past the half that are never stored: kDiaSlack more words lie behind
+// the last diagonal.  (Padded to 256, halves of 55 functions held 4.6 times their coefficients: the 64 instances' sums
+// of a dipole scan took 27 us, 11 now.)
+constexpr int kDiaSlack = 2 * 192;
 constexpr int kDiaBW = 7;
 
 // LDS slot of window position p of a run of 64*P outputs: position p at [p % P][p / P], so the lanes' positions
@@ -1694,7 +1698,7 @@ int setup_dia(gade_model *m) {
             if (std::abs(m->rad_Ai[k] % nh - a % nh) > kDiaBW) return GADE_OK;
     m->nh = nh;
     m->nd = 2 * kDiaBW + 1;
-    m->nhp = (nh + kDiaSegMax - 1) / kDiaSegMax * kDiaSegMax;
+    m->nhp = (nh + 63) / 64 * 64;
     const int S = 4 * m->nd * m->nhp;
     std::vector<int> dia_src(S, -1);
     for (int qd = 0; qd < 4; qd++)
@@ -1716,9 +1720,11 @@ int setup_dia(gade_model *m) {
         GADE_TRY(hip_alloc((void **)&m->d_gtsr, sizeof(double) * (size_t)lmax * 12 * S));
     }
     m->gd_stride = (size_t)lmax * 4 * S * 2;
-    GADE_TRY(hip_alloc((void **)&m->d_GD, sizeof(double2) * m->gd_stride * m->B));
-    GADE_HIP(hipMemset(m->d_GD, 0, sizeof(double2) * m->gd_stride * m->B));  // f = 0 until the first set_time
-    GADE_TRY(hip_alloc((void **)&m->d_DD, sizeof(double2) * (size_t)3 * m->nq * S));
+    const size_t gd_words = m->gd_stride * m->B + kDiaSlack, dd_words = (size_t)3 * m->nq * S + kDiaSlack;
+    GADE_TRY(hip_alloc((void **)&m->d_GD, sizeof(double2) * gd_words));
+    GADE_HIP(hipMemset(m->d_GD, 0, sizeof(double2) * gd_words));  // f = 0 until the first set_time
+    GADE_TRY(hip_alloc((void **)&m->d_DD, sizeof(double2) * dd_words));
+    GADE_HIP(hipMemset(m->d_DD, 0, sizeof(double2) * dd_words));
     const long long tg = (long long)lmax * 12 * S, td = (long long)3 * m->nq * S;
     hipLaunchKernelGGL(k_build_gdia, dim3(grid_for(tg, 256)), dim3(256), 0, m->stream, m->d_g, m->d_dia_src, m->d_tmap,
                        lmax, m->nd, m->nhp, m->nnzb, m->d_gs, m->d_gts, m->d_gsr, m->d_gtsr);
@@ -2598,10 +2604,11 @@ int mp_setup(gade_model *m) {
     }
     const size_t N = (size_t)m->N, L = (size_t)m->lmax;
     const size_t S = (size_t)4 * m->nd * m->nhp;
-    const size_t nDD = 3 * (size_t)m->nq * S, nco = (size_t)m->hnnz * L * 2;
+    const size_t nDD = 3 * (size_t)m->nq * S + kDiaSlack, nco = (size_t)m->hnnz * L * 2;
     GADE_TRY(hip_alloc((void **)&m->d_V32, sizeof(float2) * L * 4 * N));
     GADE_TRY(hip_alloc((void **)&m->d_ypart32, sizeof(float2) * L * N));
-    GADE_TRY(hip_alloc((void **)&m->d_GD32, sizeof(float2) * m->gd_stride * m->B));
+    GADE_TRY(hip_alloc((void **)&m->d_GD32, sizeof(float2) * (m->gd_stride * m->B + kDiaSlack)));
+    GADE_HIP(hipMemsetAsync(m->d_GD32, 0, sizeof(float2) * (m->gd_stride * m->B + kDiaSlack), m->stream));
     GADE_TRY(hip_alloc((void **)&m->d_DD32, sizeof(float2) * nDD));
     GADE_TRY(hip_alloc((void **)&m->d_coef32, sizeof(float2) * nco));
     const size_t nacf = 2 * (size_t)m->h_aoff.back();  // (h0, h1) per list entry
