@@ -1604,7 +1604,7 @@ int launch_radial(gade_model *m, const double2 *x, double2 *y, int sel, double c
     if (m->radial_kind == 2) {
         const int lgrid = inter ? m->lmax : 1;
         double2 *yp = inter && lgrid > 1 ? m->d_ypart : nullptr;
-        double2 *yp2 = y2 && yp ? m->d_ypart2 : nullptr;  // allocated with the model when lmax > 1
+        double2 *yp2 = y2 && yp ? m->d_ypart2 : nullptr;
         if (y2) {
             Prof pr(m, "radial_pair", GADE_PROF_RADIAL);
             GADE_TRY((launch_dia64<true>(m, lgrid, x, sel, cH, 0.0, y, yp, y2, yp2, sel2)));
@@ -2165,7 +2165,7 @@ int gade_model_create_batch(const gade_inputs_t *in, int B, double h, double dt,
         (rc = hip_alloc((void **)&m->d_D, sizeof(double2) * (size_t)3 * m->nq * ellw * n)) ||
         (rc = hip_alloc((void **)&m->d_V, sizeof(double2) * (size_t)lmax * 4 * m->N)) ||
         (rc = hip_alloc((void **)&m->d_ypart, sizeof(double2) * (size_t)lmax * m->N)) ||
-        (lmax > 1 && (rc = hip_alloc((void **)&m->d_ypart2, sizeof(double2) * (size_t)lmax * m->N))))
+        (rc = hip_alloc((void **)&m->d_ypart2, sizeof(double2) * (size_t)lmax * m->N)))
         return fail(rc);
     if (hipMemset(m->d_GE, 0, sizeof(double2) * (size_t)lmax * 8 * ellw * n) != hipSuccess)  // f = 0 until set_time
         return fail(GADE_EHIP);
@@ -2303,6 +2303,11 @@ int gade_precond_setup(gade_model_t *m) {
 // ---------------------------------------------------------------------------
 // preconditioner apply, BiCGSTAB, CN stepping
 // ---------------------------------------------------------------------------
+namespace gade {
+template <class T, int PRE>
+int launch_tw(const gade_blocklu *lu, const T *F, const T *b, T *x, hipStream_t stream, const int *gate, int gstride,
+              int nblk1, const PsolveVecs<T> &kv);
+}
 namespace {
 
 int psolve_async(gade_model *m, const double2 *b, double2 *x) {
@@ -2323,14 +2328,15 @@ int bicg_op(gade_model *m, const double2 *b, double2 *x = nullptr) {
     return GADE_OK;
 }
 
-// out = A x followed by the reduction OP (OP_ALPHA: out = v; OP_W: out = t), the radial phase's partial sum
-// and the reduction in one kernel (partials into 'part'); the same results as apply_async then bicg_op<OP>,
-// bit for bit.  Needs the banded radial phase with multipole partials (fused_sums()).  fin: finish the
-// reduction in its own k_bicg_fin (else the next vector step folds it in).
-bool fused_sums(const gade_model *m) { return m->radial_kind == 2 && m->lmax >= 2; }
+// The banded radial phase leaves multipole partials, and the kernel that sums them carries the dot products that follow
+// (apply_dot); the vector steps before a preconditioner solve are formed by the solve (psolve_p, psolve_s), and alpha
+// and w are finished by the kernels that use them.  A body is eight launches: solve, product, sum, solve, product, sum,
+// x and r, finish.
+bool fused_sums(const gade_model *m) { return m->radial_kind == 2; }
 
+// out = A x followed by the partial sums of the reduction OP (OP_ALPHA: out = v; OP_W: out = t) into 'part'
 template <int OP>
-int apply_dot(gade_model *m, const double2 *x, double2 *out, double *part, bool fin) {
+int apply_dot(gade_model *m, const double2 *x, double2 *out, double *part) {
     GADE_TRY(angular_phase(m, x));
     {
         Prof pr(m, "radial", GADE_PROF_RADIAL);
@@ -2340,11 +2346,6 @@ int apply_dot(gade_model *m, const double2 *x, double2 *out, double *part, bool 
     hipLaunchKernelGGL(k_sum_bicg<OP>, dim3(m->red_blocks, m->B), dim3(kRedThreads), 0, m->stream, m->N1, m->N,
                        m->lmax, (const double2 *)m->d_ypart, out, (const double2 *)m->r0, (const double2 *)m->s,
                        part, m->gate, m->gstride);
-    if (fin) {
-        int *ctl = m->ctl_on ? m->d_ctl : nullptr;
-        hipLaunchKernelGGL(k_bicg_fin<OP>, dim3(m->B), dim3(kRedThreads), 0, m->stream, m->red_blocks, part,
-                           m->d_sc, m->gate, m->gstride, ctl);
-    }
     GADE_HIP(hipGetLastError());
     return GADE_OK;
 }
@@ -2364,6 +2365,50 @@ int bicg_op_fold(gade_model *m, const double *fold_part, double2 *x = nullptr) {
     }
     GADE_HIP(hipGetLastError());
     return GADE_OK;
+}
+
+// p = r + beta (p - w v), y = M^-1 p
+int psolve_p(gade_model *m) {
+    if (!m->pre->d_TW) {
+        GADE_TRY(bicg_op<OP_P>(m, m->tmp));
+        return psolve_async(m, m->p, m->y);
+    }
+    Prof pr(m, "psolve", GADE_PROF_PSOLVE);
+    PsolveVecs<double2> kv;
+    kv.r = m->r;
+    kv.p = m->p;
+    kv.v = m->v;
+    kv.sc = m->d_sc;
+    return gade::launch_tw<double2, PRE_P>(m->pre, m->pre->d_TW, nullptr, m->y, m->stream, m->gate, m->gstride,
+                                           m->nblk1, kv);
+}
+
+// alpha from the partials, s = r - alpha v, z = M^-1 s
+int psolve_s(gade_model *m, const double *fold_part) {
+    if (!m->pre->d_TW) {
+        GADE_TRY(bicg_op_fold<OP_S>(m, fold_part));
+        return psolve_async(m, m->s, m->z);
+    }
+    Prof pr(m, "psolve", GADE_PROF_PSOLVE);
+    PsolveVecs<double2> kv;
+    kv.r = m->r;
+    kv.v = m->v;
+    kv.s = m->s;
+    kv.sc = m->d_sc;
+    kv.fold = fold_part;
+    kv.nparts = m->red_blocks;
+    return gade::launch_tw<double2, PRE_S>(m->pre, m->pre->d_TW, nullptr, m->z, m->stream, m->gate, m->gstride,
+                                           m->nblk1, kv);
+}
+
+// one BiCGSTAB body on the current vectors (x: the solution), banded radial phase (w's partials in their own buffer:
+// x/r's reduction reuses d_part while other blocks still read them)
+int bicg_body(gade_model *m, double2 *x) {
+    GADE_TRY(psolve_p(m));
+    GADE_TRY(apply_dot<OP_ALPHA>(m, m->y, m->v, m->d_part));
+    GADE_TRY(psolve_s(m, m->d_part));
+    GADE_TRY(apply_dot<OP_W>(m, m->z, m->t, m->d_part2));
+    return bicg_op_fold<OP_XR>(m, m->d_part2, x);
 }
 
 int read_scalars(gade_model *m) {
@@ -2400,15 +2445,20 @@ int bicg_host_loop(gade_model *m, const double2 *rhs, double2 *x, int i, double 
             GADE_TRY(read_scalars(m));
             r0_sq = m->h_sc[SC_R0SQ];
         }
-        GADE_TRY(bicg_op<OP_P>(m, rhs));                 // p = r + beta (p - w v)
-        GADE_TRY(psolve_async(m, m->p, m->y));           // y = M^-1 p
-        GADE_TRY(applyA(m, m->y, m->v, napply));         // v = A y
-        GADE_TRY(bicg_op<OP_ALPHA>(m, rhs));             // alpha = rho / (r0 . v)
-        GADE_TRY(bicg_op<OP_S>(m, rhs));                 // s = r - alpha v
-        GADE_TRY(psolve_async(m, m->s, m->z));           // z = M^-1 s
-        GADE_TRY(applyA(m, m->z, m->t, napply));         // t = A z
-        GADE_TRY(bicg_op<OP_W>(m, rhs));                 // w = (t . s) / |t|^2
-        GADE_TRY(bicg_op<OP_XR>(m, rhs, x));             // x += alpha y + w z ; r = s - w t
+        if (fused_sums(m)) {
+            GADE_TRY(bicg_body(m, x));
+            if (napply) *napply += 2;
+        } else {
+            GADE_TRY(bicg_op<OP_P>(m, rhs));              // p = r + beta (p - w v)
+            GADE_TRY(psolve_async(m, m->p, m->y));        // y = M^-1 p
+            GADE_TRY(applyA(m, m->y, m->v, napply));      // v = A y
+            GADE_TRY(bicg_op<OP_ALPHA>(m, rhs));          // alpha = rho / (r0 . v)
+            GADE_TRY(bicg_op<OP_S>(m, rhs));              // s = r - alpha v
+            GADE_TRY(psolve_async(m, m->s, m->z));        // z = M^-1 s
+            GADE_TRY(applyA(m, m->z, m->t, napply));      // t = A z
+            GADE_TRY(bicg_op<OP_W>(m, rhs));              // w = (t . s) / |t|^2
+            GADE_TRY(bicg_op<OP_XR>(m, rhs, x));          // x += alpha y + w z ; r = s - w t
+        }
         GADE_TRY(read_scalars(m));
         rnorm2 = m->h_sc[SC_RNORM2];
         rho_next_abs = std::hypot(m->h_sc[SC_RHONEXT], m->h_sc[SC_RHONEXT + 1]);
@@ -2513,9 +2563,6 @@ struct GateScope {
 
 }  // namespace
 namespace gade {
-template <class T>
-int launch_tw(const gade_blocklu *lu, const T *F, const T *b, T *x, hipStream_t stream, const int *gate, int gstride,
-              int nblk1);
 // the step graph holds device addresses of the model's buffers: drop it before any of them is replaced
 void drop_step_graph(gade_model *m) {
     // a replay may still be running on the model's stream: let it finish before the executable goes
@@ -2546,27 +2593,20 @@ int ensure_step_buffers(gade_model *m, int nsteps) {
 // K gated BiCGSTAB iterations on the current step of every instance
 int enqueue_iterations(gade_model *m, double2 *psi, int K) {
     m->gate = m->d_ctl + CT_SKIP;
-    const bool fused = fused_sums(m);
     for (int k = 0; k < K; k++) {
+        if (fused_sums(m)) {
+            GADE_TRY(bicg_body(m, psi));
+            continue;
+        }
         GADE_TRY(bicg_op<OP_P>(m, m->tmp));
         GADE_TRY(psolve_async(m, m->p, m->y));
-        if (fused) {
-            // the radial sums carry the dots; alpha and w are finished by the vector steps that use them (w's
-            // partials in their own buffer: x/r's reduction reuses d_part while other blocks still read them)
-            GADE_TRY(apply_dot<OP_ALPHA>(m, m->y, m->v, m->d_part, false));
-            GADE_TRY(bicg_op_fold<OP_S>(m, m->d_part));
-            GADE_TRY(psolve_async(m, m->s, m->z));
-            GADE_TRY(apply_dot<OP_W>(m, m->z, m->t, m->d_part2, false));
-            GADE_TRY(bicg_op_fold<OP_XR>(m, m->d_part2, psi));
-        } else {
-            GADE_TRY(apply_async(m, m->y, m->v, 1.0, 0.0));
-            GADE_TRY(bicg_op<OP_ALPHA>(m, m->tmp));
-            GADE_TRY(bicg_op<OP_S>(m, m->tmp));
-            GADE_TRY(psolve_async(m, m->s, m->z));
-            GADE_TRY(apply_async(m, m->z, m->t, 1.0, 0.0));
-            GADE_TRY(bicg_op<OP_W>(m, m->tmp));
-            GADE_TRY(bicg_op<OP_XR>(m, m->tmp, psi));
-        }
+        GADE_TRY(apply_async(m, m->y, m->v, 1.0, 0.0));
+        GADE_TRY(bicg_op<OP_ALPHA>(m, m->tmp));
+        GADE_TRY(bicg_op<OP_S>(m, m->tmp));
+        GADE_TRY(psolve_async(m, m->s, m->z));
+        GADE_TRY(apply_async(m, m->z, m->t, 1.0, 0.0));
+        GADE_TRY(bicg_op<OP_W>(m, m->tmp));
+        GADE_TRY(bicg_op<OP_XR>(m, m->tmp, psi));
     }
     return GADE_OK;
 }
@@ -2639,54 +2679,69 @@ int mp_setup(gade_model *m) {
     return GADE_OK;
 }
 
-// y = (S + H) x in FP32 (the FP32 G-sums of the current step)
-int apply32_async(gade_model *m, const float2 *x, float2 *y) {
+// out = (S + H) x in FP32 (the FP32 G-sums of the current step) and the partial sums of the reduction OP into 'part'
+template <int OP>
+int apply_dot32(gade_model *m, const float2 *x, float2 *out, double *part) {
     if (!ang_in_radial<float2>(m)) {
         Prof pr(m, "angular_f32", GADE_PROF_ANGULAR);
         GADE_TRY(launch_angular_t<float2>(m, x, (const float2 *)m->d_coef32, (const float2 *)m->d_acf32,
                                           (const float2 *)m->d_acr32, m->d_V32));
     }
-    const int lgrid = m->lmax;
-    float2 *yp = lgrid > 1 ? m->d_ypart32 : nullptr;
     {
         Prof pr(m, "radial_f32", GADE_PROF_RADIAL);
-        GADE_TRY((launch_dia<false, float2>(m, lgrid, x, (const float2 *)m->d_V32, (const float2 *)m->d_GD32,
-                                            (const float2 *)m->d_DD32, 0, 1.0, 0.0, y, yp, (float2 *)nullptr,
-                                            (float2 *)nullptr, 0)));
+        GADE_TRY((launch_dia<false, float2>(m, m->lmax, x, (const float2 *)m->d_V32, (const float2 *)m->d_GD32,
+                                            (const float2 *)m->d_DD32, 0, 1.0, 0.0, out, m->d_ypart32,
+                                            (float2 *)nullptr, (float2 *)nullptr, 0)));
     }
-    if (yp) {
-        Prof pr(m, "radial_sum_f32", GADE_PROF_RADIAL_SUM);
-        hipLaunchKernelGGL(k_radial_sum<float2>, dim3(grid_for(m->N1, 256, 2048), m->B), dim3(256), 0, m->stream,
-                           yp, lgrid, m->N, 0.0, y, m->gate, m->gstride, m->N1);
-        GADE_HIP(hipGetLastError());
-    }
-    return GADE_OK;
-}
-
-int psolve32_async(gade_model *m, const float2 *b, float2 *x) {
-    Prof pr(m, "psolve_f32", GADE_PROF_PSOLVE);
-    const gade_blocklu *lu = m->pre;
-    if (lu->d_TW) {
-        return gade::launch_tw(lu, (const float2 *)m->tw32, b, x, m->stream, m->gate, m->gstride, m->nblk1);
-    }
-    // 32-row levels (mixed precision needs 16- or 32-row levels and a band of at most 16)
-    const size_t shq = sizeof(float2) * ((size_t)lu->nch * lu->ch + lu->ch);
-    hipLaunchKernelGGL((k_psolve_q<2, float2, 32, 2>), dim3(lu->norder), dim3(64), shq, m->stream, b, x,
-                       lu->d_order, lu->d_blk_q, lu->ilv, m->lu32[0], m->lu32[1], m->lu32[2], m->lu32[3], lu->n,
-                       lu->band, lu->nch, m->gate, m->gstride, m->nblk1);
+    Prof pr(m, "radial_sum_f32", GADE_PROF_RADIAL_SUM);
+    hipLaunchKernelGGL((k_sum_bicg<OP, float2>), dim3(m->red_blocks, m->B), dim3(kRedThreads), 0, m->stream, m->N1, m->N,
+                       m->lmax, (const float2 *)m->d_ypart32, out, (const float2 *)m->mp_r0, (const float2 *)m->mp_s,
+                       part, m->gate, m->gstride);
     GADE_HIP(hipGetLastError());
     return GADE_OK;
 }
 
-template <int OP>
-int bicg32_op(gade_model *m) {
+template <int OP, bool FOLD>
+int bicg32_op(gade_model *m, const double *fold_part) {
     Prof pr(m, "blas1_f32", GADE_PROF_BLAS1);
-    hipLaunchKernelGGL((k_bicg<OP, float2>), dim3(m->red_blocks, m->B), dim3(kRedThreads), 0, m->stream, m->N1,
+    hipLaunchKernelGGL((k_bicg<OP, float2, FOLD>), dim3(m->red_blocks, m->B), dim3(kRedThreads), 0, m->stream, m->N1,
                        (const float2 *)nullptr, m->mp_r, m->mp_r0, m->mp_p, m->mp_v, m->mp_s, m->mp_t, m->mp_y,
-                       m->mp_z, m->mp_d, m->d_sc32, m->d_part, m->gate, m->gstride);
-    if (OP != OP_P && OP != OP_S)
+                       m->mp_z, m->mp_d, m->d_sc32, m->d_part, m->gate, m->gstride, fold_part, m->red_blocks);
+    if (OP == OP_XR)
         hipLaunchKernelGGL((k_bicg_fin<OP, true>), dim3(m->B), dim3(kRedThreads), 0, m->stream, m->red_blocks,
                            m->d_part, m->d_sc32, m->gate, m->gstride, m->d_ctl);
+    GADE_HIP(hipGetLastError());
+    return GADE_OK;
+}
+
+// the solves of the FP32 body with their vector steps: psolve_p, psolve_s in FP32
+template <int PRE>
+int psolve32(gade_model *m) {
+    const gade_blocklu *lu = m->pre;
+    float2 *out = PRE == PRE_P ? m->mp_y : m->mp_z;
+    if (lu->d_TW) {
+        Prof pr(m, "psolve_f32", GADE_PROF_PSOLVE);
+        PsolveVecs<float2> kv;
+        kv.r = m->mp_r;
+        kv.p = m->mp_p;
+        kv.v = m->mp_v;
+        kv.s = m->mp_s;
+        kv.sc = m->d_sc32;
+        kv.fold = m->d_part;
+        kv.nparts = m->red_blocks;
+        return gade::launch_tw<float2, PRE>(lu, m->tw32, nullptr, out, m->stream, m->gate, m->gstride, m->nblk1, kv);
+    }
+    // 32-row levels (mixed precision needs 16- or 32-row levels and a band of at most 16)
+    if (PRE == PRE_P)
+        GADE_TRY((bicg32_op<OP_P, false>(m, nullptr)));
+    else
+        GADE_TRY((bicg32_op<OP_S, true>(m, m->d_part)));
+    Prof pr(m, "psolve_f32", GADE_PROF_PSOLVE);
+    const size_t shq = sizeof(float2) * ((size_t)lu->nch * lu->ch + lu->ch);
+    hipLaunchKernelGGL((k_psolve_q<2, float2, 32, 2>), dim3(lu->norder), dim3(64), shq, m->stream,
+                       (const float2 *)(PRE == PRE_P ? m->mp_p : m->mp_s), out, lu->d_order, lu->d_blk_q, lu->ilv,
+                       m->lu32[0], m->lu32[1], m->lu32[2], m->lu32[3], lu->n, lu->band, lu->nch, m->gate, m->gstride,
+                       m->nblk1);
     GADE_HIP(hipGetLastError());
     return GADE_OK;
 }
@@ -2703,15 +2758,11 @@ int enqueue_sweeps(gade_model *m, double2 *psi, int J) {
         GADE_HIP(hipGetLastError());
         m->gate = m->d_ctl + CT_ISKIP;
         for (int k = 0; k < m->mp_inner_iters; k++) {
-            GADE_TRY(bicg32_op<OP_P>(m));
-            GADE_TRY(psolve32_async(m, m->mp_p, m->mp_y));
-            GADE_TRY(apply32_async(m, m->mp_y, m->mp_v));
-            GADE_TRY(bicg32_op<OP_ALPHA>(m));
-            GADE_TRY(bicg32_op<OP_S>(m));
-            GADE_TRY(psolve32_async(m, m->mp_s, m->mp_z));
-            GADE_TRY(apply32_async(m, m->mp_z, m->mp_t));
-            GADE_TRY(bicg32_op<OP_W>(m));
-            GADE_TRY(bicg32_op<OP_XR>(m));
+            GADE_TRY(psolve32<PRE_P>(m));
+            GADE_TRY(apply_dot32<OP_ALPHA>(m, m->mp_y, m->mp_v, m->d_part));
+            GADE_TRY(psolve32<PRE_S>(m));
+            GADE_TRY(apply_dot32<OP_W>(m, m->mp_z, m->mp_t, m->d_part2));
+            GADE_TRY((bicg32_op<OP_XR, true>(m, m->d_part2)));
         }
         m->gate = m->d_ctl + CT_SKIP;
         hipLaunchKernelGGL(k_mp_update, dim3(grid_for(m->N1, 256, 2048), m->B), dim3(256), 0, m->stream, m->N1, psi,
@@ -2749,22 +2800,35 @@ int enqueue_rhs_ax0(gade_model *m, double2 *psi) {
     return apply_async(m, psi, m->r, 1.0, 0.0);
 }
 
-// the rhs, A x0 and the start of the solve (OP_INIT); with x0 = psi and multipole partials, the paired
-// apply's sums and OP_INIT are one kernel (the same results)
+// the rhs, A x0 and the start of the solve (OP_INIT), which the banded products' sums carry
 int enqueue_rhs_init(gade_model *m, double2 *psi) {
-    if (m->guess_order != 0 || !fused_sums(m)) {
+    if (!fused_sums(m)) {
         GADE_TRY(enqueue_rhs_ax0(m, psi));
         return bicg_op<OP_INIT>(m, m->tmp);
     }
+    const bool pair = m->guess_order == 0;
+    if (!pair) {
+        GADE_TRY(apply_async(m, psi, m->tmp, -1.0, 0.0));
+        GADE_TRY(launch_guess(m, psi));
+    }
     GADE_TRY(angular_phase(m, psi));
-    {
+    if (pair) {
         Prof pr(m, "radial_pair", GADE_PROF_RADIAL);
         GADE_TRY((launch_dia64<true>(m, m->lmax, psi, 1, -1.0, 0.0, m->tmp, m->d_ypart, m->r, m->d_ypart2, 0)));
+    } else {
+        Prof pr(m, "radial", GADE_PROF_RADIAL);
+        GADE_TRY((launch_dia64<false>(m, m->lmax, psi, 0, 1.0, 0.0, m->r, m->d_ypart2, nullptr, nullptr, 0)));
     }
     Prof pr(m, "radial_sum", GADE_PROF_RADIAL_SUM);
-    hipLaunchKernelGGL(k_sum2_init, dim3(m->red_blocks, m->B), dim3(kRedThreads), 0, m->stream, m->N1, m->N, m->lmax,
-                       (const double2 *)m->d_ypart, (const double2 *)m->d_ypart2, m->tmp, m->r, m->r0, m->d_part,
-                       m->gate, m->gstride);
+    const dim3 red(m->red_blocks, m->B);
+    if (pair)
+        hipLaunchKernelGGL(k_sum2_init<false>, red, dim3(kRedThreads), 0, m->stream, m->N1, m->N, m->lmax,
+                           (const double2 *)m->d_ypart, (const double2 *)m->d_ypart2, m->tmp, m->r, m->r0, m->d_part,
+                           m->gate, m->gstride);
+    else
+        hipLaunchKernelGGL(k_sum2_init<true>, red, dim3(kRedThreads), 0, m->stream, m->N1, m->N, m->lmax,
+                           (const double2 *)nullptr, (const double2 *)m->d_ypart2, m->tmp, m->r, m->r0, m->d_part,
+                           m->gate, m->gstride);
     int *ctl = m->ctl_on ? m->d_ctl : nullptr;
     hipLaunchKernelGGL(k_bicg_fin<OP_INIT>, dim3(m->B), dim3(kRedThreads), 0, m->stream, m->red_blocks, m->d_part,
                        m->d_sc, m->gate, m->gstride, ctl);
@@ -2816,20 +2880,15 @@ int launch_gsums_window(gade_model *m) {
 // step words), so the same launches serve every step: the body of the step graph.
 int enqueue_step_window(gade_model *m, double2 *psi, int K, bool per_instance_steps) {
     GateScope gs(m);
-    hipLaunchKernelGGL(k_step_begin, dim3(m->B), dim3(64), 0, m->stream, m->d_ctl, m->d_gctl, -1,
-                       per_instance_steps ? m->d_nsteps : nullptr);
+    hipLaunchKernelGGL(k_step_turn, dim3(1), dim3(256), 0, m->stream, m->B, m->d_ctl, m->d_gctl,
+                       (const double *)m->d_sc, m->steps_cap, m->d_iters, m->d_tols,
+                       (const int *)(per_instance_steps ? m->d_nsteps : nullptr));
     GADE_HIP(hipGetLastError());
     m->gate = m->d_ctl + CT_PSKIP;
     GADE_TRY(launch_gsums_window(m));
     if (m->precision == 1) GADE_TRY(mp_convert_gsums(m));
     GADE_TRY(enqueue_rhs_init(m, psi));
-    GADE_TRY(enqueue_solve(m, psi, K));
-    hipLaunchKernelGGL(k_step_end, dim3(m->B), dim3(64), 0, m->stream, m->d_ctl, m->d_gctl, m->d_sc, -1,
-                       m->steps_cap, m->d_iters, m->d_tols);
-    hipLaunchKernelGGL(k_stall_spread, dim3(m->B), dim3(64), 0, m->stream, m->d_ctl, m->d_gctl);
-    hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(64), 0, m->stream, m->d_gctl);
-    GADE_HIP(hipGetLastError());
-    return GADE_OK;
+    return enqueue_solve(m, psi, K);
 }
 
 // the step graph for this K (captured again when anything it bakes in has changed)
@@ -3028,6 +3087,7 @@ int cn_run_device(gade_model *m, double2 *psi, const double *times, int nsteps, 
                 return rc;
             }
         }
+        if (table) GADE_TRY(enqueue_step_end(m, -1));  // the last step's (the others end as the next one starts)
         GADE_HIP(hipMemcpyAsync(m->h_gctl, m->d_gctl, sizeof(int) * GC_COUNT, hipMemcpyDeviceToHost, m->stream));
         GADE_HIP(hipMemcpyAsync(it_h.data(), m->d_iters, sizeof(int) * B * cap, hipMemcpyDeviceToHost, m->stream));
         GADE_HIP(hipMemcpyAsync(tol_h.data(), m->d_tols, sizeof(double) * B * cap, hipMemcpyDeviceToHost, m->stream));
@@ -4240,13 +4300,13 @@ int blocklu_build(int nblk, int n, const int *rAp, const int *rAi, int nq, const
     return GADE_OK;
 }
 
-template <class T>
+template <class T, int PRE>
 int launch_tw(const gade_blocklu *lu, const T *F, const T *b, T *x, hipStream_t stream, const int *gate, int gstride,
-              int nblk1) {
+              int nblk1, const PsolveVecs<T> &kv) {
     const size_t sh = sizeof(T) * (size_t)lu->nch * 16 * lu->nr;
 #define TW(PF_, NR_)                                                                                                  \
-    hipLaunchKernelGGL((k_psolve_tw<PF_, T, NR_>), dim3(lu->norder), dim3(128), sh, stream, b, x, lu->d_order,        \
-                       lu->d_blk_q, lu->ilv, F, lu->n, lu->nch, lu->tw_m, gate, gstride, nblk1)
+    hipLaunchKernelGGL((k_psolve_tw<PF_, T, NR_, PRE>), dim3(lu->norder), dim3(128), sh, stream, b, x, lu->d_order,   \
+                       lu->d_blk_q, lu->ilv, F, lu->n, lu->nch, lu->tw_m, gate, gstride, nblk1, kv)
     switch (lu->nr) {
         case 1: TW(4, 1); break;
         case 2: TW(2, 2); break;
@@ -4256,8 +4316,11 @@ int launch_tw(const gade_blocklu *lu, const T *F, const T *b, T *x, hipStream_t 
     GADE_HIP(hipGetLastError());
     return GADE_OK;
 }
-template int launch_tw<float2>(const gade_blocklu *, const float2 *, const float2 *, float2 *, hipStream_t, const int *,
-                               int, int);
+#define TWI(T_, P_)                                                                                              \
+    template int launch_tw<T_, P_>(const gade_blocklu *, const T_ *, const T_ *, T_ *, hipStream_t, const int *, \
+                                   int, int, const PsolveVecs<T_> &);
+TWI(double2, PRE_P) TWI(double2, PRE_S) TWI(float2, PRE_NONE) TWI(float2, PRE_P) TWI(float2, PRE_S)
+#undef TWI
 
 int blocklu_solve_async(const gade_blocklu *lu, const double2 *b, double2 *x, hipStream_t stream, const int *gate,
                         int gstride, int nblk1) {
@@ -4267,7 +4330,7 @@ int blocklu_solve_async(const gade_blocklu *lu, const double2 *b, double2 *x, hi
     }
     if (lu->d_TW) {
         // twisted factorization, meeting at level tw_m
-        return launch_tw(lu, (const double2 *)lu->d_TW, b, x, stream, gate, gstride, nblk1);
+        return launch_tw<double2, PRE_NONE>(lu, lu->d_TW, b, x, stream, gate, gstride, nblk1, {});
     }
     const bool quad = (lu->ch == 16 || lu->ch == 32) && lu->band <= 16;
     if (!quad && gstride != 0) {

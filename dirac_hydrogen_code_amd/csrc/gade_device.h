@@ -349,12 +349,11 @@ __global__ __launch_bounds__(kRedThreads) void k_bicg(long long N1, const T *__r
 // multipole partials of the radial phase (in multipole order, as k_radial_sum with beta 0), then for
 // OP_ALPHA the partial r0 . out, for OP_W the partials |out|^2 and out . s (out = t).  The grid and every
 // thread's order of entries are k_bicg's, so out and the partial sums equal the unfused pair's bit for bit.
-template <int OP>
+template <int OP, class T = double2>
 __global__ __launch_bounds__(kRedThreads) void k_sum_bicg(long long N1, long long N, int lgrid,
-                                                           const double2 *__restrict__ ypart,
-                                                           double2 *__restrict__ out, const double2 *__restrict__ r0,
-                                                           const double2 *__restrict__ s, double *__restrict__ part0,
-                                                           const int *gate, int gstride) {
+                                                           const T *__restrict__ ypart, T *__restrict__ out,
+                                                           const T *__restrict__ r0, const T *__restrict__ s,
+                                                           double *__restrict__ part0, const int *gate, int gstride) {
     static_assert(OP == OP_ALPHA || OP == OP_W, "fused sums: alpha or w");
     const int inst = blockIdx.y;
     GADE_GATED_B(gate, gstride, inst);
@@ -364,16 +363,17 @@ __global__ __launch_bounds__(kRedThreads) void k_sum_bicg(long long N1, long lon
     double acc[4] = {0, 0, 0, 0};
     for (long long j = blockIdx.x * (long long)blockDim.x + threadIdx.x; j < N1; j += (long long)gridDim.x * blockDim.x) {
         const long long i = o + j;
-        double2 v = ypart[i];
-        for (int l = 1; l < lgrid; l++) v = cadd(v, ypart[(size_t)l * N + i]);
-        out[i] = v;
+        T vT = ypart[i];
+        for (int l = 1; l < lgrid; l++) vT = cadd(vT, ypart[(size_t)l * N + i]);
+        out[i] = vT;
+        const double2 v = to_f64(vT);  // the dot products accumulate in double
         if (OP == OP_ALPHA) {
-            double2 d = cfmaconj(r0[i], v, make_double2(acc[0], acc[1]));
+            double2 d = cfmaconj(to_f64(r0[i]), v, make_double2(acc[0], acc[1]));
             acc[0] = d.x;
             acc[1] = d.y;
         } else {
             acc[0] = fma(v.x, v.x, fma(v.y, v.y, acc[0]));
-            double2 d = cfmaconj(v, s[i], make_double2(acc[1], acc[2]));
+            double2 d = cfmaconj(v, to_f64(s[i]), make_double2(acc[1], acc[2]));
             acc[1] = d.x;
             acc[2] = d.y;
         }
@@ -387,7 +387,9 @@ __global__ __launch_bounds__(kRedThreads) void k_sum_bicg(long long N1, long lon
 // ax = sum of ypart2 (A x0 = (S + H) x), r = r0 = b - ax, partials |r|^2 and |b|^2.  Each sum runs in
 // multipole order and the grid and every thread's order of entries are k_bicg's: the same results as two
 // k_radial_sum launches then k_bicg<OP_INIT>, bit for bit.
-[[maybe_unused]] static __global__ __launch_bounds__(kRedThreads) void k_sum2_init(long long N1, long long N, int lgrid,
+// GIVEN_B: b holds the rhs already (ypart unused), and only A x0 is summed.
+template <bool GIVEN_B>
+__global__ __launch_bounds__(kRedThreads) void k_sum2_init(long long N1, long long N, int lgrid,
                                                             const double2 *__restrict__ ypart,
                                                             const double2 *__restrict__ ypart2,
                                                             double2 *__restrict__ b, double2 *__restrict__ r,
@@ -401,12 +403,12 @@ __global__ __launch_bounds__(kRedThreads) void k_sum_bicg(long long N1, long lon
     double acc[4] = {0, 0, 0, 0};
     for (long long j = blockIdx.x * (long long)blockDim.x + threadIdx.x; j < N1; j += (long long)gridDim.x * blockDim.x) {
         const long long i = o + j;
-        double2 bs = ypart[i], ax = ypart2[i];
+        double2 bs = GIVEN_B ? b[i] : ypart[i], ax = ypart2[i];
         for (int l = 1; l < lgrid; l++) {
-            bs = cadd(bs, ypart[(size_t)l * N + i]);
+            if (!GIVEN_B) bs = cadd(bs, ypart[(size_t)l * N + i]);
             ax = cadd(ax, ypart2[(size_t)l * N + i]);
         }
-        b[i] = bs;
+        if (!GIVEN_B) b[i] = bs;
         const double2 ri = csub(bs, ax);
         r[i] = ri;
         r0[i] = ri;
@@ -667,6 +669,47 @@ __global__ __launch_bounds__(kRedThreads) void k_bicg_fin(int nparts, const doub
     }
 }
 
+// Start of a window's next step (one workgroup): k_step_end of the step before it (if it is not the window's first),
+// the stall marked for every instance, the run-wide step words advanced and k_step_begin, in one launch instead of
+// four.  k_window_begin precedes the first step, k_step_end and k_stall_spread follow the last one.
+[[maybe_unused]] static __global__ __launch_bounds__(256) void k_step_turn(int B, int *ctl0, int *gctl,
+                                                                         const double *__restrict__ sc0,
+                                                                         int nsteps_cap, int *iters, double *tols,
+                                                                         const int *__restrict__ nsteps) {
+    __shared__ int stalled;
+    const int prev = gctl[GC_STEP], slot = gctl[GC_WSLOT], was = gctl[GC_STALLED];
+    if (threadIdx.x == 0) stalled = was;
+    __syncthreads();
+    if (!was && slot >= 0)
+        for (int b = threadIdx.x; b < B; b += blockDim.x) {
+            const int *ctl = ctl0 + (size_t)b * CT_STRIDE;
+            const double *sc = sc0 + (size_t)b * SC_STRIDE;
+            if (ctl[CT_PSKIP] != 0) continue;
+            const int st = ctl[CT_STATUS];
+            if (st == 1 || st == 3) {
+                iters[(size_t)b * nsteps_cap + prev] = ctl[CT_ITER];
+                tols[(size_t)b * nsteps_cap + prev] = sqrt(sc[SC_RNORM2] / sc[SC_RHSSQ]);
+            } else {
+                stalled = 1;  // every unfinished instance writes the same value
+            }
+        }
+    __syncthreads();
+    for (int b = threadIdx.x; b < B; b += blockDim.x) {
+        int *ctl = ctl0 + (size_t)b * CT_STRIDE;
+        const int idle = stalled != 0 || (nsteps != nullptr && prev + 1 >= nsteps[b]);
+        ctl[CT_PSKIP] = idle;
+        if (idle) ctl[CT_SKIP] = 1;
+    }
+    if (threadIdx.x == 0) {
+        if (stalled && !was) {
+            gctl[GC_STALLED] = 1;
+            gctl[GC_STALL_STEP] = prev;
+        }
+        gctl[GC_STEP] = prev + 1;
+        gctl[GC_WSLOT] = slot + 1;
+    }
+}
+
 // End of the extra iterations the host enqueues for a stalled step: record every decided solve.
 [[maybe_unused]] static __global__ void k_step_end_resume(int *ctl0, int *gctl, const double *__restrict__ sc0,
                                                           int step, int nsteps_cap, int *iters, double *tols) {
@@ -682,17 +725,11 @@ __global__ __launch_bounds__(kRedThreads) void k_bicg_fin(int nparts, const doub
     (void)gctl;
 }
 
-// Next step of a window (after k_stall_spread): advances the run-wide step words.
-[[maybe_unused]] static __global__ void k_step_advance(int *gctl) {
-    if (threadIdx.x == 0) {
-        gctl[GC_STEP] += 1;
-        gctl[GC_WSLOT] += 1;
-    }
-}
+// Before a window's first step (k_step_turn advances to it).
 [[maybe_unused]] static __global__ void k_window_begin(int *gctl, int step) {
     if (threadIdx.x == 0) {
-        gctl[GC_STEP] = step;
-        gctl[GC_WSLOT] = 0;
+        gctl[GC_STEP] = step - 1;
+        gctl[GC_WSLOT] = -1;
     }
 }
 
@@ -984,11 +1021,25 @@ __device__ __forceinline__ void wave_lds_sync() {
 // their traffic is the bound: 3200 blocks of 510 rows read 1.6 GB with NR = 1, 148 us against 59 with NR = 4.  Few
 // blocks are bound by the chain of levels; there NR = 1 has more of them side by side (psolve_blocks).  PF, the levels
 // of factors in flight, is 4, 2 and 1 for NR = 1, 2 and 4: more costs registers and so waves.
-template <int PF, class T, int NR>
+// PRE: the solve's right-hand side is formed from the BiCGSTAB vectors as it is staged, by the vector step before it
+// (its entries belong to the block): PRE_P: p = r + beta (p - w v), beta from the scalars, p stored; PRE_S: alpha
+// finished from the previous reduction's partials, s = r - alpha v, s stored (and alpha, rho recorded by the workgroup
+// of the instance's first block).  At 400 x 510 the two vector kernels took 4.9 and 6.7 us a body besides the gaps
+// around them; the solves take 25.2 and 27.9 us with the steps inside and 23.3 without.
+enum PsolvePre { PRE_NONE = 0, PRE_P, PRE_S };
+template <class T>
+struct PsolveVecs {  // the vectors and scalars of PRE (fold: [instance][nparts][4])
+    const T *r = nullptr, *v = nullptr;
+    T *p = nullptr, *s = nullptr;
+    double *sc = nullptr;
+    const double *fold = nullptr;
+    int nparts = 0;
+};
+template <int PF, class T, int NR, int PRE>
 __global__ __launch_bounds__(128) void k_psolve_tw(const T *__restrict__ b, T *__restrict__ xo,
                                                    const int *__restrict__ order, const int *__restrict__ blk_q,
                                                    int ilv, const T *__restrict__ F, int n, int nch, int m,
-                                                   const int *gate = nullptr, int gstride = 0, int nblk1 = 1) {
+                                                   const int *gate, int gstride, int nblk1, PsolveVecs<T> kv) {
     constexpr int CH = 16, MS = CH * CH;
     extern __shared__ __align__(16) char smem_raw[];
     T *const v = reinterpret_cast<T *>(smem_raw);  // [NR][nch*16], interleaved order
@@ -1028,21 +1079,81 @@ __global__ __launch_bounds__(128) void k_psolve_tw(const T *__restrict__ b, T *_
 #pragma unroll
     for (int u = 0; u < PF; u++)
         if (u < nf) ld4(fwd_level(u), 0, ff[u]);
+    double2 alpha[NR];  // PRE_S
+    if constexpr (PRE == PRE_S) {
+        __shared__ double red[2][2];
+#pragma unroll
+        for (int j = 0; j < NR; j++) {
+            alpha[j] = make_double2(0, 0);
+            if (r[j] < 0) continue;
+            const int inst = r[j] / nblk1;
+            if (j > 0 && r[j - 1] >= 0 && r[j - 1] / nblk1 == inst) {
+                alpha[j] = alpha[j - 1];
+                continue;
+            }
+            const double *fp = kv.fold + (size_t)inst * kv.nparts * 4;
+            double t0 = 0, t1 = 0;
+            for (int u = threadIdx.x; u < kv.nparts; u += 128) {
+                t0 += fp[(size_t)u * 4];
+                t1 += fp[(size_t)u * 4 + 1];
+            }
+            t0 = wave_sum(t0);
+            t1 = wave_sum(t1);
+            __syncthreads();
+            if (lane == 0) {
+                red[wave][0] = t0;
+                red[wave][1] = t1;
+            }
+            __syncthreads();
+            const double *sc = kv.sc + (size_t)inst * SC_STRIDE;
+            alpha[j] = cdiv(make_double2(sc[SC_RHONEXT], sc[SC_RHONEXT + 1]),
+                            make_double2(red[0][0] + red[1][0], red[0][1] + red[1][1]));
+        }
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+            if (r[j] >= 0 && r[j] % nblk1 == 0 && threadIdx.x == 0) {
+                double *sc = kv.sc + (size_t)(r[j] / nblk1) * SC_STRIDE;
+                sc[SC_ALPHA] = alpha[j].x;
+                sc[SC_ALPHA + 1] = alpha[j].y;
+                sc[SC_RHO] = sc[SC_RHONEXT];
+                sc[SC_RHO + 1] = sc[SC_RHONEXT + 1];
+            }
+    }
     // b: eight loads per thread in flight before the LDS writes
 #pragma unroll
     for (int j = 0; j < NR; j++) {
-        const T *bb = b + (size_t)max(r[j], 0) * n;
-        for (int c0 = 0; c0 < ntot; c0 += 128 * 8) {
-            T t[8];
+        const size_t o = (size_t)max(r[j], 0) * n;
+        T beta = czero<T>(), w = czero<T>(), al = czero<T>();
+        if constexpr (PRE == PRE_P) {
+            // beta = (rho_new / rho_old) * (alpha / w), as k_bicg<OP_P>
+            const double *sc = kv.sc + (size_t)(max(r[j], 0) / nblk1) * SC_STRIDE;
+            const double2 w2 = make_double2(sc[SC_W], sc[SC_W + 1]);
+            beta = from_f64<T>(cmul(cdiv(make_double2(sc[SC_RHONEXT], sc[SC_RHONEXT + 1]),
+                                         make_double2(sc[SC_RHO], sc[SC_RHO + 1])),
+                                    cdiv(make_double2(sc[SC_ALPHA], sc[SC_ALPHA + 1]), w2)));
+            w = from_f64<T>(w2);
+        }
+        if constexpr (PRE == PRE_S) al = from_f64<T>(alpha[j]);
+        constexpr int LU = PRE == PRE_NONE ? 8 : 4;  // loads in flight (of up to three vectors)
+        for (int c0 = 0; c0 < ntot; c0 += 128 * LU) {
+            T t[LU];
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
+            for (int u = 0; u < LU; u++) {
                 const int c = c0 + 128 * u + (int)threadIdx.x;
-                t[u] = c < n && r[j] >= 0 ? bb[natural_index(c, n, ilv)] : czero<T>();
+                t[u] = czero<T>();
+                if (c < n && r[j] >= 0) {
+                    const size_t g = o + natural_index(c, n, ilv);
+                    if constexpr (PRE == PRE_NONE) t[u] = b[g];
+                    if constexpr (PRE == PRE_P) t[u] = cadd(kv.r[g], cmul(beta, csub(kv.p[g], cmul(w, kv.v[g]))));
+                    if constexpr (PRE == PRE_S) t[u] = csub(kv.r[g], cmul(al, kv.v[g]));
+                }
             }
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
+            for (int u = 0; u < LU; u++) {
                 const int c = c0 + 128 * u + (int)threadIdx.x;
                 if (c < ntot) v[j * ntot + c] = t[u];
+                if (PRE != PRE_NONE && c < n && r[j] >= 0)
+                    (PRE == PRE_P ? kv.p : kv.s)[o + natural_index(c, n, ilv)] = t[u];
             }
         }
     }
