@@ -1428,6 +1428,8 @@ void free_all(gade_model *m) {
     if (m->h_ctl) hipHostFree(m->h_ctl);
     if (m->h_gctl) hipHostFree(m->h_gctl);
     if (m->h_cfwin) hipHostFree(m->h_cfwin);
+    if (m->h_iters) hipHostFree(m->h_iters);
+    if (m->h_tols) hipHostFree(m->h_tols);
     gade::lg_free(m->lg);
     m->lg = nullptr;
     if (m->d_cfwin) hipFree(m->d_cfwin);
@@ -1441,7 +1443,7 @@ void free_all(gade_model *m) {
                     (void *)m->lu32[2], (void *)m->lu32[3], (void *)m->tw32, (void *)m->mp_r, (void *)m->mp_r0, (void *)m->mp_p,
                     (void *)m->mp_v, (void *)m->mp_y, (void *)m->mp_z, (void *)m->mp_s, (void *)m->mp_t,
                     (void *)m->mp_d, (void *)m->d_mp_ax, (void *)m->d_sc32, (void *)m->d_aoff, (void *)m->d_ack,
-                    (void *)m->d_acf, (void *)m->d_acf32, (void *)m->d_acr, (void *)m->d_acr32, (void *)m->d_gsr, (void *)m->d_gtsr, (void *)m->d_GF, (void *)m->d_DF, (void *)m->d_mg_rows,
+                    (void *)m->d_acf, (void *)m->d_acf32, (void *)m->d_psi, (void *)m->d_acr, (void *)m->d_acr32, (void *)m->d_gsr, (void *)m->d_gtsr, (void *)m->d_GF, (void *)m->d_DF, (void *)m->d_mg_rows,
                     (void *)m->d_mg_q, (void *)m->d_mg_b, (void *)m->d_mg_k})
         if (p) hipFree(p);
     resolve_pending(m);
@@ -2581,11 +2583,15 @@ int ensure_step_buffers(gade_model *m, int nsteps) {
     drop_step_graph(m);  // it writes the per-step outputs being replaced
     if (m->d_iters) (void)hipFree(m->d_iters);
     if (m->d_tols) (void)hipFree(m->d_tols);
-    m->d_iters = nullptr;
-    m->d_tols = nullptr;
+    if (m->h_iters) (void)hipHostFree(m->h_iters);
+    if (m->h_tols) (void)hipHostFree(m->h_tols);
+    m->d_iters = m->h_iters = nullptr;
+    m->d_tols = m->h_tols = nullptr;
     m->steps_cap = 0;
     GADE_TRY(hip_alloc((void **)&m->d_iters, sizeof(int) * (size_t)m->B * nsteps));
     GADE_TRY(hip_alloc((void **)&m->d_tols, sizeof(double) * (size_t)m->B * nsteps));
+    GADE_HIP(hipHostMalloc((void **)&m->h_iters, sizeof(int) * (size_t)m->B * nsteps, hipHostMallocDefault));
+    GADE_HIP(hipHostMalloc((void **)&m->h_tols, sizeof(double) * (size_t)m->B * nsteps, hipHostMallocDefault));
     m->steps_cap = nsteps;
     return GADE_OK;
 }
@@ -2900,7 +2906,7 @@ int step_graph(gade_model *m, double2 *psi, int K, bool per_instance_steps) {
     // on growth also drop the graph themselves)
     intptr_t tol_bits = 0;
     memcpy(&tol_bits, &m->mp_inner_tol, sizeof(double) < sizeof(intptr_t) ? sizeof(double) : sizeof(intptr_t));
-    const void *key[12] = {psi,      (const void *)(intptr_t)K, (const void *)(intptr_t)m->guess_order,
+    const void *key[11] = {(const void *)(intptr_t)K, (const void *)(intptr_t)m->guess_order,
                            (const void *)(intptr_t)(per_instance_steps ? 1 : 0), m->d_iters,
                            (const void *)(intptr_t)m->steps_cap, m->d_cfwin, m->d_hist,
                            (const void *)(intptr_t)m->precision, (const void *)(intptr_t)m->mp_inner_iters,
@@ -2939,9 +2945,7 @@ int ensure_cfwin(gade_model *m, int slots) {
 }
 
 // The run stalled at 'step': finish it for every instance from the device state.
-// it_h/tol_h: [B][steps_cap] host copies of the per-step outputs.
-int finish_stalled_step(gade_model *m, double2 *psi, int step, int K, std::vector<int> &it_h,
-                        std::vector<double> &tol_h) {
+int finish_stalled_step(gade_model *m, double2 *psi, int step, int K) {
     const int B = m->B;
     for (int round = 0;; round++) {
         GADE_HIP(hipMemcpyAsync(m->h_ctl, m->d_ctl, sizeof(int) * B * CT_STRIDE, hipMemcpyDeviceToHost, m->stream));
@@ -3002,9 +3006,9 @@ int finish_stalled_step(gade_model *m, double2 *psi, int step, int K, std::vecto
         hipLaunchKernelGGL(k_step_end_resume, dim3(B), dim3(64), 0, m->stream, m->d_ctl, m->d_gctl, m->d_sc, step,
                            m->steps_cap, m->d_iters, m->d_tols);
         GADE_HIP(hipGetLastError());
-        GADE_HIP(hipMemcpyAsync(it_h.data(), m->d_iters, sizeof(int) * B * m->steps_cap, hipMemcpyDeviceToHost,
+        GADE_HIP(hipMemcpyAsync(m->h_iters, m->d_iters, sizeof(int) * B * m->steps_cap, hipMemcpyDeviceToHost,
                                 m->stream));
-        GADE_HIP(hipMemcpyAsync(tol_h.data(), m->d_tols, sizeof(double) * B * m->steps_cap, hipMemcpyDeviceToHost,
+        GADE_HIP(hipMemcpyAsync(m->h_tols, m->d_tols, sizeof(double) * B * m->steps_cap, hipMemcpyDeviceToHost,
                                 m->stream));
         if (!more) {
             GADE_HIP(hipStreamSynchronize(m->stream));
@@ -3018,17 +3022,18 @@ int finish_stalled_step(gade_model *m, double2 *psi, int step, int K, std::vecto
 // Steps 0..nsteps-1 for every instance at the given times; params [B][4] = (E0, omega, cycles, cep) of
 // each instance's pulse; nsteps_b [B] (null: every instance runs all steps).  psi [B][N1] is x0 and
 // result.  iters/tol_out [B][nsteps] (entries past an instance's pulse are left untouched).
-int cn_run_device(gade_model *m, double2 *psi, const double *times, int nsteps, const double *params,
-                  const int *nsteps_b, double tol, int maxit, int *iters, double *tol_out, double *usec) {
-    if (nsteps == 0) return GADE_OK;
+int run_steps(gade_model *m, double2 *psi, const double *times, int nsteps, const double *params, const int *nsteps_b,
+              double tol, int maxit, int *iters, double *tol_out, double *usec) {
     const int B = m->B;
     GADE_TRY(gade_precond_setup(m));
     if (m->precision == 1) GADE_TRY(mp_setup(m));
     GADE_TRY(ensure_step_buffers(m, nsteps));
     if (m->guess_order == GADE_GUESS_LEARNED || m->lg_features) GADE_TRY(gade::lg_prepare(m));
     const size_t cap = (size_t)m->steps_cap;
-    std::vector<int> it_h((size_t)B * cap, 0);
-    std::vector<double> tol_h((size_t)B * cap, 0.0);
+    int *const it_h = m->h_iters;  // pinned copies of the per-step outputs, [B][steps_cap]
+    double *const tol_h = m->h_tols;
+    std::fill(it_h, it_h + (size_t)B * cap, 0);
+    std::fill(tol_h, tol_h + (size_t)B * cap, 0.0);
     GADE_HIP(hipMemsetAsync(m->d_iters, 0, sizeof(int) * B * cap, m->stream));
     GADE_HIP(hipMemsetAsync(m->d_tols, 0, sizeof(double) * B * cap, m->stream));
     if (nsteps_b) GADE_HIP(hipMemcpyAsync(m->d_nsteps, nsteps_b, sizeof(int) * B, hipMemcpyHostToDevice, m->stream));
@@ -3089,24 +3094,32 @@ int cn_run_device(gade_model *m, double2 *psi, const double *times, int nsteps, 
         }
         if (table) GADE_TRY(enqueue_step_end(m, -1));  // the last step's (the others end as the next one starts)
         GADE_HIP(hipMemcpyAsync(m->h_gctl, m->d_gctl, sizeof(int) * GC_COUNT, hipMemcpyDeviceToHost, m->stream));
-        GADE_HIP(hipMemcpyAsync(it_h.data(), m->d_iters, sizeof(int) * B * cap, hipMemcpyDeviceToHost, m->stream));
-        GADE_HIP(hipMemcpyAsync(tol_h.data(), m->d_tols, sizeof(double) * B * cap, hipMemcpyDeviceToHost, m->stream));
+        GADE_HIP(hipMemcpy2DAsync(it_h + s, sizeof(int) * cap, m->d_iters + s, sizeof(int) * cap, sizeof(int) * W, B,
+                                  hipMemcpyDeviceToHost, m->stream));
+        GADE_HIP(hipMemcpy2DAsync(tol_h + s, sizeof(double) * cap, m->d_tols + s, sizeof(double) * cap,
+                                  sizeof(double) * W, B, hipMemcpyDeviceToHost, m->stream));
         GADE_HIP(hipStreamSynchronize(m->stream));
         int done = s + W;
-        if (m->h_gctl[GC_STALLED]) {
+        const bool stalled = m->h_gctl[GC_STALLED] != 0;
+        if (stalled) {
             done = m->h_gctl[GC_STALL_STEP];
             if (done < s || done >= s + W) {
                 gade::set_error("device-driven stepping: inconsistent stall record");
                 return GADE_EHIP;
             }
-            GADE_TRY(finish_stalled_step(m, psi, done, K, it_h, tol_h));
+            GADE_TRY(finish_stalled_step(m, psi, done, K));
             GADE_HIP(hipStreamSynchronize(m->stream));
             done += 1;
         }
         int kmax = 0;
         for (int b = 0; b < B; b++)
             for (int w = s; w < done; w++) kmax = std::max(kmax, it_h[(size_t)b * cap + w] + 1);
-        m->last_k = std::min(std::max(kmax + 1, 2), 16);
+        // The iterations the window needed, at least two, and one more for a while after a step needed more than were
+        // enqueued: a body too many costs its gated launches on every step (20 of 148 us at 40 x 110), a body too few
+        // voids the rest of a window, but hardly ever happens as the count moves slowly along a pulse.
+        if (stalled) m->slack_windows = 8;
+        const int slack = m->slack_windows > 0 ? (m->slack_windows--, 1) : 0;
+        m->last_k = std::min(std::max(kmax + slack, 2), 16);
         if (usec) {
             for (int w = 0; w < done - s; w++) {
                 float ms = 0;
@@ -3126,6 +3139,25 @@ int cn_run_device(gade_model *m, double2 *psi, const double *times, int nsteps, 
             if (tol_out) tol_out[(size_t)b * nsteps + w] = tol_h[(size_t)b * cap + w];
         }
     }
+    return GADE_OK;
+}
+
+// The same on a state of the model's own when the steps are replayed from a graph, which holds its address: a caller
+// with another psi (a new state, the next pulse) copies it in and out, and the graph is not captured again (0.3 ms).
+int cn_run_device(gade_model *m, double2 *psi, const double *times, int nsteps, const double *params,
+                  const int *nsteps_b, double tol, int maxit, int *iters, double *tol_out, double *usec) {
+    if (nsteps == 0) return GADE_OK;
+    if (m->radial_kind != 2 || !m->use_graph || m->profile != 0)
+        return run_steps(m, psi, times, nsteps, params, nsteps_b, tol, maxit, iters, tol_out, usec);
+    if (!m->d_psi) GADE_TRY(hip_alloc((void **)&m->d_psi, sizeof(double2) * m->N));
+    const dim3 grid(grid_for(m->N, 256, 8192));
+    hipLaunchKernelGGL(k_copy, grid, dim3(256), 0, m->stream, (const double2 *)psi, m->d_psi, m->N);
+    GADE_HIP(hipGetLastError());
+    const int rc = run_steps(m, m->d_psi, times, nsteps, params, nsteps_b, tol, maxit, iters, tol_out, usec);
+    hipLaunchKernelGGL(k_copy, grid, dim3(256), 0, m->stream, (const double2 *)m->d_psi, psi, m->N);
+    const hipError_t e = hipStreamSynchronize(m->stream);
+    GADE_TRY(rc);  // (the state goes back as far as it got)
+    GADE_HIP(e);
     return GADE_OK;
 }
 

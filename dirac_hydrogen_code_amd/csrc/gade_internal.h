@@ -193,6 +193,9 @@ struct gade_model {
     int *d_nsteps = nullptr;       // [B] steps of each instance's pulse
     int *d_iters = nullptr;        // [B][steps_cap]
     double *d_tols = nullptr;      // [B][steps_cap]
+    int *h_iters = nullptr;        // pinned mirrors
+    double *h_tols = nullptr;
+    double2 *d_psi = nullptr;      // the state that replayed step graphs run on
     int steps_cap = 0;
     const int *gate = nullptr;     // gate passed to every model launch (null: ungated)
     int gstride = 0;               // ints between the gate words of consecutive instances
@@ -201,6 +204,7 @@ struct gade_model {
     int window = 8;                // steps enqueued per host synchronization
     int iter_batch = 0;            // iterations enqueued per step (0: adaptive)
     int last_k = 2;                // adaptive iterations per step
+    int slack_windows = 0;         // windows that enqueue one iteration more (after a step that needed it)
     int guess_order = 0;           // initial guess: 0 psi_n (the reference), p: extrapolation of order p
     // per-step pulse coefficients of a window on the device ([slot][B] x 6 complex) and the step graph
     double2 *d_cfwin = nullptr, *h_cfwin = nullptr;
@@ -209,7 +213,7 @@ struct gade_model {
     hipStream_t cap_stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
-    const void *graph_key[12] = {};  // what the captured step depends on
+    const void *graph_key[11] = {};  // what the captured step depends on
     double2 *d_hist = nullptr;     // [kHistSlots][N] history ring of previous solutions (per instance)
     gade_lg *lg = nullptr;         // learned initial guess
     int lg_features = 0;           // compute the learned guess's inputs every step (training data)
