@@ -26,76 +26,118 @@ using gade::set_error;
 
 namespace {
 
-// per block r: w = S(k_r) psi_r (staged in LDS), c_j = sum_i conj(v_j[i]) w_i,
-// out[r] = (sum over classes of |c_j|^2, then psi_r^H S psi_r)
-__global__ __launch_bounds__(256) void k_eigproj(const double2 *__restrict__ x, const double2 *__restrict__ D,
-                                                 const int *__restrict__ ell_col, const int *__restrict__ blk_q,
-                                                 const double2 *__restrict__ VT, const double *__restrict__ E,
-                                                 int n, int ellw, int nq, double csq, double *__restrict__ out) {
+// per block r: w = S(k_r) psi_r (staged in LDS), then c_j = v_j . w for every eigenpair j of its kappa.
+// COEF false: out[r][blockIdx.y] = (sums of |c_j|^2 over the classes for this workgroup's eigenpairs, psi_r^H S
+// psi_r for the first); out may be pinned host memory.
+// COEF true: out[r][j] = c_j, complex (the amplitudes behind the populations).
+//
+// One workgroup per block leaves most of the chip idle at the usual 60 to 500 blocks, and the work of one block
+// is a chain of dependent memory reads, so latency bounds it: 256 threads with a thread per eigenpair and two
+// loads in flight took 36.8 us at 104 blocks of 210 rows (57 us for the call).  Here 1024 threads take eight
+// eigenpairs per wave, the sum over the rows split over eight lanes (64-byte row segments of V, the partial sums
+// met by lane exchanges), and the first kBatch rows of each lane are read before w is formed, as they do not
+// depend on it.  The rows of S are likewise split over eight lanes.  The eigenvectors are real and are stored so.
+// Measured there: 17.6 us, and 30 us for the call with no copy and no allocation left in it (32 us with one
+// workgroup per block, so that two passes follow each other).
+constexpr int kLanes = 8;   // lanes that share one eigenpair's sum, or one row of S
+constexpr int kBatch = 8;   // rows of V a lane holds in flight
+constexpr int kEigThreads = 1024;
+constexpr int kItems = kEigThreads / kLanes;
+// workgroups per block: a pass of kItems eigenpairs each, while the blocks alone leave CUs without a workgroup
+inline int eig_split(int nblk, int n) {
+    return std::max(1, std::min((n + kItems - 1) / kItems, 512 / std::max(1, nblk)));
+}
+template <bool COEF>
+__global__ __launch_bounds__(kEigThreads) void k_eigproj(const double2 *__restrict__ x, const double2 *__restrict__ D,
+                                                         const int *__restrict__ ell_col,
+                                                         const int *__restrict__ blk_q, const double *__restrict__ VT,
+                                                         const double *__restrict__ E, int n, int ellw, int nq,
+                                                         double csq, double *__restrict__ out) {
     extern __shared__ double2 w[];
-    __shared__ double sh[4 * 16];
+    __shared__ double sh[4 * (kEigThreads / 64)];
     const int r = blockIdx.x;
     const int q = blk_q[r];
+    const int lane = threadIdx.x & 63, part = lane >> 3;
+    const int item = (threadIdx.x >> 6) * 8 + (lane & 7);  // eigenpair (or row of S) of this lane's group
+    const double *V = VT + (size_t)q * n * n;
+    const int jf = blockIdx.y * kItems;  // first pass of this workgroup
+    double v0[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; u++) {
+        const int i = part + kLanes * u;
+        v0[u] = (i < n && jf + item < n) ? V[(size_t)i * n + jf + item] : 0.0;
+    }
     const double2 *Sq = D + ((size_t)2 * nq + q) * ellw * n;  // S(k) in ELL layout
     const double2 *xr = x + (size_t)r * n;
     double acc[4] = {0, 0, 0, 0};
-    for (int a = threadIdx.x; a < n; a += blockDim.x) {
-        double2 sx = make_double2(0, 0);
-        for (int sl = 0; sl < ellw; sl++) sx = cfma(Sq[(size_t)sl * n + a], xr[ell_col[(size_t)sl * n + a]], sx);
-        w[a] = sx;
-        const double2 xa = xr[a];
-        acc[3] += xa.x * sx.x + xa.y * sx.y;
+    for (int a0 = 0; a0 < n; a0 += kItems) {
+        const int a = a0 + item;
+        double sx = 0, sy = 0;
+        if (a < n) {
+            double2 t = make_double2(0, 0);
+            for (int sl = part; sl < ellw; sl += kLanes)
+                t = cfma(Sq[(size_t)sl * n + a], xr[ell_col[(size_t)sl * n + a]], t);
+            sx = t.x;
+            sy = t.y;
+        }
+#pragma unroll
+        for (int o = 8; o < 64; o <<= 1) {
+            sx += __shfl_xor(sx, o, 64);
+            sy += __shfl_xor(sy, o, 64);
+        }
+        if (a < n && part == 0) {
+            w[a] = make_double2(sx, sy);
+            if (!COEF && blockIdx.y == 0) {
+                const double2 xa = xr[a];
+                acc[3] += xa.x * sx + xa.y * sy;
+            }
+        }
     }
     __syncthreads();
-    const double2 *V = VT + (size_t)q * n * n;
-    const double *Eq = E + (size_t)q * n;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        double2 c0 = make_double2(0, 0), c1 = make_double2(0, 0);
-        int i = 0;
-        for (; i + 1 < n; i += 2) {
-            c0 = cfma(V[(size_t)i * n + j], w[i], c0);
-            c1 = cfma(V[(size_t)(i + 1) * n + j], w[i + 1], c1);
+    for (int j0 = jf; j0 < n; j0 += gridDim.y * kItems) {
+        const int j = j0 + item;
+        double cx = 0, cy = 0;
+        if (j < n) {
+            for (int i0 = 0; i0 < n; i0 += kLanes * kBatch) {
+                if (i0 > 0 || j0 != jf) {
+#pragma unroll
+                    for (int u = 0; u < kBatch; u++) {
+                        const int i = i0 + part + kLanes * u;
+                        v0[u] = i < n ? V[(size_t)i * n + j] : 0.0;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kBatch; u++) {
+                    const int i = i0 + part + kLanes * u;
+                    if (i < n) {
+                        const double2 wi = w[i];
+                        cx = fma(v0[u], wi.x, cx);
+                        cy = fma(v0[u], wi.y, cy);
+                    }
+                }
+            }
         }
-        if (i < n) c0 = cfma(V[(size_t)i * n + j], w[i], c0);
-        const double2 c = cadd(c0, c1);
-        const double p = c.x * c.x + c.y * c.y;
-        const double e = Eq[j];
-        if (e < -csq) acc[0] += p;
-        else if (e < 0) acc[1] += p;
-        else acc[2] += p;
-    }
-    block_sum<4>(acc, sh);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < 4; k++) out[(size_t)r * 4 + k] = acc[k];
-}
-
-// per block r: c_j = v_j^H S(k_r) psi_r for every eigenpair j of its kappa (the amplitudes behind the
-// populations); out [nblk][n] complex
-__global__ __launch_bounds__(256) void k_eigcoef(const double2 *__restrict__ x, const double2 *__restrict__ D,
-                                                 const int *__restrict__ ell_col, const int *__restrict__ blk_q,
-                                                 const double2 *__restrict__ VT, int n, int ellw, int nq,
-                                                 double2 *__restrict__ out) {
-    extern __shared__ double2 w[];
-    const int r = blockIdx.x;
-    const int q = blk_q[r];
-    const double2 *Sq = D + ((size_t)2 * nq + q) * ellw * n;
-    const double2 *xr = x + (size_t)r * n;
-    for (int a = threadIdx.x; a < n; a += blockDim.x) {
-        double2 sx = make_double2(0, 0);
-        for (int sl = 0; sl < ellw; sl++) sx = cfma(Sq[(size_t)sl * n + a], xr[ell_col[(size_t)sl * n + a]], sx);
-        w[a] = sx;
-    }
-    __syncthreads();
-    const double2 *V = VT + (size_t)q * n * n;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        double2 c0 = make_double2(0, 0), c1 = make_double2(0, 0);
-        int i = 0;
-        for (; i + 1 < n; i += 2) {
-            c0 = cfma(V[(size_t)i * n + j], w[i], c0);
-            c1 = cfma(V[(size_t)(i + 1) * n + j], w[i + 1], c1);
+#pragma unroll
+        for (int o = 8; o < 64; o <<= 1) {
+            cx += __shfl_xor(cx, o, 64);
+            cy += __shfl_xor(cy, o, 64);
         }
-        if (i < n) c0 = cfma(V[(size_t)i * n + j], w[i], c0);
-        out[(size_t)r * n + j] = cadd(c0, c1);
+        if (j < n && part == 0) {
+            if (COEF) {
+                reinterpret_cast<double2 *>(out)[(size_t)r * n + j] = make_double2(cx, cy);
+            } else {
+                const double p = cx * cx + cy * cy;
+                const double e = E[(size_t)q * n + j];
+                if (e < -csq) acc[0] += p;
+                else if (e < 0) acc[1] += p;
+                else acc[2] += p;
+            }
+        }
+    }
+    if (!COEF) {
+        block_sum<4>(acc, sh);
+        if (threadIdx.x == 0)
+            for (int k = 0; k < 4; k++) out[((size_t)r * gridDim.y + blockIdx.y) * 4 + k] = acc[k];
     }
 }
 
@@ -141,16 +183,15 @@ int gade_eig_setup(gade_model_t *m) {
                       (rcs[q] == GADE_EINVAL ? " failed: S is not positive definite" : " did not converge"));
             return rcs[q];
         }
-    // VT[q][i][j] = conj(v_j[i]); the eigenvectors are real
-    std::vector<double2> vt((size_t)nq * nn);
-    for (size_t idx = 0; idx < vt.size(); idx++) vt[idx] = make_double2(V[idx], 0.0);
-    double *d_eval = nullptr;
-    double2 *d_evec = nullptr;
+    // V[q][i][j] = v_j[i], as stored; h_eig receives the populations of every block
+    double *d_eval = nullptr, *d_evec = nullptr, *h_eig = nullptr;
     GADE_TRY(gade::hip_alloc((void **)&d_eval, sizeof(double) * nq * n));
-    int rc = gade::hip_alloc((void **)&d_evec, sizeof(double2) * vt.size());
+    int rc = gade::hip_alloc((void **)&d_evec, sizeof(double) * V.size());
     hipError_t e = hipSuccess;
     if (rc == GADE_OK) e = hipMemcpy(d_eval, E.data(), sizeof(double) * E.size(), hipMemcpyHostToDevice);
-    if (rc == GADE_OK && e == hipSuccess) e = hipMemcpy(d_evec, vt.data(), sizeof(double2) * vt.size(), hipMemcpyHostToDevice);
+    if (rc == GADE_OK && e == hipSuccess) e = hipMemcpy(d_evec, V.data(), sizeof(double) * V.size(), hipMemcpyHostToDevice);
+    if (rc == GADE_OK && e == hipSuccess)
+        e = hipHostMalloc((void **)&h_eig, sizeof(double) * 4 * m->nblk * eig_split(m->nblk, n), hipHostMallocDefault);
     if (rc != GADE_OK || e != hipSuccess) {
         (void)hipFree(d_eval);
         if (d_evec) (void)hipFree(d_evec);
@@ -158,6 +199,7 @@ int gade_eig_setup(gade_model_t *m) {
         set_error(std::string("gade_eig_setup: ") + hipGetErrorString(e));
         return GADE_EHIP;
     }
+    m->h_eig = h_eig;
     m->d_eval = d_eval;
     m->d_evec = d_evec;
     return GADE_OK;
@@ -177,31 +219,31 @@ int gade_populations(gade_model_t *m, const double *x, double *norm, double *bou
                      double *per_block) {
     if (!m || !x) return GADE_EINVAL;
     GADE_TRY(gade_eig_setup(m));
-    double *d_out = nullptr;
-    GADE_TRY(gade::hip_alloc((void **)&d_out, sizeof(double) * 4 * m->nblk));
     const double csq = gade::kSoL * gade::kSoL;
-    hipLaunchKernelGGL(k_eigproj, dim3(m->nblk), dim3(256), sizeof(double2) * m->n, m->stream, (const double2 *)x,
-                       m->d_D, m->d_ell_col, m->d_blk_q, m->d_evec, m->d_eval, m->n, m->ellw, m->nq, csq, d_out);
-    std::vector<double> out((size_t)4 * m->nblk);
+    // the sums go straight to pinned host memory: four numbers per workgroup, read once the stream is done
+    const int ny = eig_split(m->nblk, m->n);
+    hipLaunchKernelGGL(k_eigproj<false>, dim3(m->nblk, ny), dim3(kEigThreads), sizeof(double2) * m->n, m->stream,
+                       (const double2 *)x, m->d_D, m->d_ell_col, m->d_blk_q, m->d_evec, m->d_eval, m->n, m->ellw,
+                       m->nq, csq, m->h_eig);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(out.data(), d_out, sizeof(double) * out.size(), hipMemcpyDeviceToHost, m->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-    (void)hipFree(d_out);
     if (e != hipSuccess) {
         set_error(std::string("gade_populations: ") + hipGetErrorString(e));
         return GADE_EHIP;
     }
     double tb = 0, ti = 0, tn = 0;
     for (int r = 0; r < m->nblk; r++) {
-        tb += out[(size_t)r * 4 + 1];
-        ti += out[(size_t)r * 4 + 2];
-        tn += out[(size_t)r * 4 + 3];
+        double sum[4] = {0, 0, 0, 0};
+        for (int y = 0; y < ny; y++)
+            for (int k = 0; k < 4; k++) sum[k] += m->h_eig[((size_t)r * ny + y) * 4 + k];
+        tb += sum[1];
+        ti += sum[2];
+        tn += sum[3];
+        if (per_block) memcpy(per_block + (size_t)r * 4, sum, sizeof sum);
     }
     if (norm) *norm = tn;
     if (bound) *bound = tb;
     if (ionised) *ionised = ti;
-    if (per_block) memcpy(per_block, out.data(), sizeof(double) * out.size());
     return GADE_OK;
 }
 
@@ -211,8 +253,9 @@ int gade_psiev(gade_model_t *m, const double *x, double *psiev) {
     const size_t cnt = (size_t)m->nblk * m->n;
     double2 *d_out = nullptr;
     GADE_TRY(gade::hip_alloc((void **)&d_out, sizeof(double2) * cnt));
-    hipLaunchKernelGGL(k_eigcoef, dim3(m->nblk), dim3(256), sizeof(double2) * m->n, m->stream, (const double2 *)x,
-                       m->d_D, m->d_ell_col, m->d_blk_q, m->d_evec, m->n, m->ellw, m->nq, d_out);
+    hipLaunchKernelGGL(k_eigproj<true>, dim3(m->nblk, eig_split(m->nblk, m->n)), dim3(kEigThreads), sizeof(double2) * m->n, m->stream,
+                       (const double2 *)x, m->d_D, m->d_ell_col, m->d_blk_q, m->d_evec, m->d_eval, m->n, m->ellw,
+                       m->nq, 0.0, (double *)d_out);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(psiev, d_out, sizeof(double2) * cnt, hipMemcpyDeviceToHost, m->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
@@ -249,17 +292,18 @@ int gade_eig_write(gade_model_t *m, const char *dir) {
     const int n = m->n, nq = m->nq;
     const size_t nn = (size_t)n * n;
     std::vector<double> E((size_t)nq * n);
-    std::vector<double2> VT((size_t)nq * nn), evc(nn);
+    std::vector<double> VT((size_t)nq * nn);
+    std::vector<double2> evc(nn);
     GADE_HIP(hipMemcpy(E.data(), m->d_eval, sizeof(double) * E.size(), hipMemcpyDeviceToHost));
-    GADE_HIP(hipMemcpy(VT.data(), m->d_evec, sizeof(double2) * VT.size(), hipMemcpyDeviceToHost));
+    GADE_HIP(hipMemcpy(VT.data(), m->d_evec, sizeof(double) * VT.size(), hipMemcpyDeviceToHost));
     for (int q = 0; q < nq; q++) {
         const int kappa = m->kap_q[q];
         GADE_TRY(dense_write(std::string(dir) + "/evl" + std::to_string(kappa) + ".mat", n, 1, E.data() + (size_t)q * n,
                              sizeof(double)));
-        // column j = eigenvector j: evc[j * n + i] = v_j[i] = conj(VT[q][i][j])
-        const double2 *V = VT.data() + (size_t)q * nn;
+        // column j = eigenvector j: evc[j * n + i] = v_j[i] (the files hold complex numbers)
+        const double *V = VT.data() + (size_t)q * nn;
         for (int i = 0; i < n; i++)
-            for (int j = 0; j < n; j++) evc[(size_t)j * n + i] = make_double2(V[(size_t)i * n + j].x, -V[(size_t)i * n + j].y);
+            for (int j = 0; j < n; j++) evc[(size_t)j * n + i] = make_double2(V[(size_t)i * n + j], -0.0);
         GADE_TRY(dense_write(std::string(dir) + "/evc" + std::to_string(kappa) + ".mat", n, n, evc.data(),
                              sizeof(double2)));
     }

@@ -1428,6 +1428,7 @@ void free_all(gade_model *m) {
     if (m->h_ctl) hipHostFree(m->h_ctl);
     if (m->h_gctl) hipHostFree(m->h_gctl);
     if (m->h_cfwin) hipHostFree(m->h_cfwin);
+    if (m->h_eig) hipHostFree(m->h_eig);
     if (m->h_iters) hipHostFree(m->h_iters);
     if (m->h_tols) hipHostFree(m->h_tols);
     gade::lg_free(m->lg);

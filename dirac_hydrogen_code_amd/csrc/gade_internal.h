@@ -181,10 +181,11 @@ struct gade_model {
     double2 *d_fAx = nullptr;
     int *d_SAp = nullptr, *d_SAi = nullptr;
     double2 *d_SAx = nullptr;
-    // eigen-projection: per distinct kappa, S-orthonormal eigenvectors (conjugate-transposed,
-    // [q][i][j] = conj(v_j[i])) and energies [q][j] of H0(k) v = E S(k) v
-    double2 *d_evec = nullptr;
+    // eigen-projection: per distinct kappa, S-orthonormal real eigenvectors (transposed,
+    // [q][i][j] = v_j[i]) and energies [q][j] of H0(k) v = E S(k) v
+    double *d_evec = nullptr;
     double *d_eval = nullptr;
+    double *h_eig = nullptr;       // pinned: the populations of every block, per workgroup
     // device-driven CN stepping: control words, per-step outputs, launch gate
     int *d_ctl = nullptr;          // [B][CT_STRIDE] per-instance words
     int *h_ctl = nullptr;          // pinned mirror
