@@ -82,49 +82,45 @@ __device__ __forceinline__ float gelu_d(float z) {
 }
 
 // ---------------------------------------------------------------------------
-// BF16 MFMA GEMM: C(m,n) = sum_k A(m,k) B(k,n), FP32 accumulation, with
-// A(m,k) = a[m*sam + k*sak], B(k,n) = b[k*sbk + n*sbn] (bf16 bits).  One block
-// per 16x16 tile of C (v_mfma_f32_16x16x16_bf16: lane l holds A[l%16][4(l/16)..+3],
-// B[4(l/16)..+3][l%16] and C[4(l/16)+i][l%16]).  The block's KS waves take the
-// 16-wide k steps in turn (wave w: steps w, w + KS, ...) and their accumulators
-// are added in wave order; KS = 1 for the training sizes, KS = 4 for the few
-// rows of inference (short per-wave chains).  M, N, K multiples of 16.
+// BF16 MFMA GEMM of the network's forward layers: C(m,n) = sum_k A[m][k] W[n][k] + bias[n], FP32 accumulation
+// (bf16 bits, both operands contiguous along k, so each lane's four k are one 8-byte load).  One block per 16x16
+// tile of C (v_mfma_f32_16x16x16_bf16: lane l holds A[l%16][4(l/16)..+3], B[4(l/16)..+3][l%16] and
+// C[4(l/16)+i][l%16]).  The block's KS waves take the 16-wide k steps in turn (wave w: steps w, w + KS, ...) and
+// their accumulators are added in wave order; KS = 4 for the few rows of inference (short per-wave chains), 1 for
+// more rows.  M, N, K multiples of 16.
 // ---------------------------------------------------------------------------
 typedef short bf4 __attribute__((ext_vector_type(4)));
 typedef float fl4 __attribute__((ext_vector_type(4)));
-enum { EPI_STORE = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2 };
+enum { EPI_BIAS = 1, EPI_BIAS_GELU = 2 };
 
 template <int EPI, int KS = 1>
-__global__ __launch_bounds__(64 * KS) void k_gemm_bf16(int M, int N, int K, const uint16_t *__restrict__ a, long sam,
-                                                       long sak, const uint16_t *__restrict__ b, long sbk, long sbn,
-                                                       float *__restrict__ c, int ldc, const float *__restrict__ bias,
+__global__ __launch_bounds__(64 * KS) void k_gemm_bf16(int M, int N, int K, const uint16_t *__restrict__ a,
+                                                       const uint16_t *__restrict__ b, float *__restrict__ c, int ldc, const float *__restrict__ bias,
                                                        uint16_t *__restrict__ act, int ldact) {
     const int tiles_n = N / 16;
     const int tm = blockIdx.x / tiles_n, tn = blockIdx.x % tiles_n;
     if (tm * 16 >= M) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-    const uint16_t *ap = a + (long)(tm * 16 + r) * sam;
-    const uint16_t *bp = b + (long)(tn * 16 + r) * sbn;
+    const uint16_t *ap = a + (long)(tm * 16 + r) * K;
+    const uint16_t *bp = b + (long)(tn * 16 + r) * K;
     fl4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (sak == 1 && sbk == 1) {
-        // both operands contiguous along k (the forward layers): each lane's four k are one 8-byte load
-        for (int k0 = 16 * w; k0 < K; k0 += 16 * KS) {
-            bf4 av, bv;
-            __builtin_memcpy(&av, reinterpret_cast<const uint2 *>(ap + k0 + 4 * g), sizeof(bf4));
-            __builtin_memcpy(&bv, reinterpret_cast<const uint2 *>(bp + k0 + 4 * g), sizeof(bf4));
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
-        }
-    } else {
-        for (int k0 = 16 * w; k0 < K; k0 += 16 * KS) {
-            bf4 av, bv;
+    // loads of six steps in flight (the whole chain of a wave at KS = 4)
+    for (int k0 = 16 * w; k0 < K; k0 += 6 * 16 * KS) {
+        uint2 au[6], bu[6];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const long kk = k0 + 4 * g + j;
-                av[j] = (short)ap[kk * sak];
-                bv[j] = (short)bp[kk * sbk];
-            }
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
+        for (int u = 0; u < 6; u++) {
+            const int k = min(k0 + 16 * KS * u, K - 16) + 4 * g;
+            au[u] = *reinterpret_cast<const uint2 *>(ap + k);
+            bu[u] = *reinterpret_cast<const uint2 *>(bp + k);
         }
+#pragma unroll
+        for (int u = 0; u < 6; u++)
+            if (k0 + 16 * KS * u < K) {
+                bf4 av, bv;
+                __builtin_memcpy(&av, &au[u], sizeof av);
+                __builtin_memcpy(&bv, &bu[u], sizeof bv);
+                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
+            }
     }
     if constexpr (KS > 1) {
         __shared__ fl4 red[KS][64];
@@ -137,8 +133,7 @@ __global__ __launch_bounds__(64 * KS) void k_gemm_bf16(int M, int N, int K, cons
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int m = tm * 16 + 4 * g + i, n = tn * 16 + r;
-        float v = acc[i];
-        if (EPI != EPI_STORE) v += bias[n];
+        const float v = acc[i] + bias[n];
         c[(long)m * ldc + n] = v;
         if (EPI == EPI_BIAS_GELU) act[(long)m * ldact + n] = f2bf(gelu(v));
     }
@@ -640,15 +635,6 @@ __global__ void k_lg_snap(long long N1, long long Ntot, const double2 *__restric
 // ---------------------------------------------------------------------------
 // training kernels
 // ---------------------------------------------------------------------------
-// X[m] = standardized bf16 inputs of sample idx[m]
-__global__ void k_lg_gather(const float *__restrict__ samples, const int *__restrict__ idx, const float *mean,
-                            const float *stdv, uint16_t *__restrict__ X) {
-    const int m = blockIdx.x;
-    const float *s = samples + (size_t)idx[m] * kSample;
-    for (int t = threadIdx.x; t < kIn; t += blockDim.x)
-        X[(size_t)m * kIn + t] = t < F_END ? f2bf((s[S_FEAT + t] - mean[t]) / stdv[t]) : (uint16_t)0;
-}
-
 // X[m] = standardized bf16 inputs of raw row m (stride kIn)
 __global__ void k_lg_gather_rows(const float *__restrict__ x, const float *mean, const float *stdv,
                                  uint16_t *__restrict__ X) {
@@ -657,100 +643,350 @@ __global__ void k_lg_gather_rows(const float *__restrict__ x, const float *mean,
         X[(size_t)m * kIn + t] = t < F_END ? f2bf((x[(size_t)m * kIn + t] - mean[t]) / stdv[t]) : (uint16_t)0;
 }
 
-// per sample: loss L = |e_hat - D w - U c|^2 / beta (the quadratic form) and dL/dY / M
-__global__ __launch_bounds__(64) void k_lg_loss(const float *__restrict__ Y, const float *__restrict__ samples,
-                                                const int *__restrict__ idx, int M, float *__restrict__ dY,
-                                                float *__restrict__ loss) {
-    const int m = blockIdx.x, t = threadIdx.x;
-    const float *y = Y + (size_t)m * kOut;
-    const float *s = samples + (size_t)idx[m] * kSample;
-    __shared__ float w[6], pw[2 * kPod], part[64];
-    if (t < 6) w[t] = y[t];
-    __syncthreads();
-    const float beta = s[S_BETA];
-    const float ib = beta > 0 ? 1.0f / beta : 0.0f;
-    float contrib = 0;
-    // POD part, one coefficient per lane
-    {
-        const int q = t;
-        float pr = 0, pi = 0;
-        for (int k = 0; k < 6; k++) {
-            pr += s[S_P + (q * 6 + k) * 2] * w[k];
-            pi += s[S_P + (q * 6 + k) * 2 + 1] * w[k];
+// The weights in the order in which the training kernel's lanes read them, next to the row-major copy: a 16-wide
+// step of a 16-wide tile is 64 lanes times four bf16, 512 contiguous bytes.
+//   fw[l]: the forward operand, tile n/16, step k/16, lane ((k/4)%4)*16 + n%16, element k%4
+//   bw[l]: the operand of dA = dZ W, tile k/16, step n/16, lane ((n/4)%4)*16 + k%16, element n%4
+template <int K, int N>
+__device__ __forceinline__ void lg_put_w(int j, uint16_t v, uint16_t *__restrict__ fw, uint16_t *__restrict__ bw) {
+    const int n = j / K, k = j % K;
+    fw[(((n >> 4) * (K / 16) + (k >> 4)) * 64 + ((k >> 2) & 3) * 16 + (n & 15)) * 4 + (k & 3)] = v;
+    bw[(((k >> 4) * (N / 16) + (n >> 4)) * 64 + ((n >> 2) & 3) * 16 + (k & 15)) * 4 + (n & 3)] = v;
+}
+__device__ __forceinline__ void lg_put(int i, uint16_t v, uint16_t *__restrict__ pbf, uint16_t *__restrict__ pfw,
+                                       uint16_t *__restrict__ pbw) {
+    pbf[i] = v;
+    if (i < (int)P_B1) lg_put_w<kIn, kHid>(i, v, pfw, pbw);
+    else if (i >= (int)P_W2 && i < (int)P_B2) lg_put_w<kHid, kHid>(i - P_W2, v, pfw + P_W2, pbw + P_W2);
+    else if (i >= (int)P_W3 && i < (int)P_B3) lg_put_w<kHid, kHid>(i - P_W3, v, pfw + P_W3, pbw + P_W3);
+    else if (i >= (int)P_W4 && i < (int)P_B4) lg_put_w<kHid, kOut>(i - P_W4, v, pfw + P_W4, pbw + P_W4);
+}
+
+// every bf16 copy of the FP32 parameters
+__global__ void k_lg_tobf(const float *__restrict__ p, uint16_t *__restrict__ pbf, uint16_t *__restrict__ pfw,
+                          uint16_t *__restrict__ pbw) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < (int)P_TOTAL; i += gridDim.x * blockDim.x)
+        lg_put(i, f2bf(p[i]), pbf, pfw, pbw);
+}
+
+// ---------------------------------------------------------------------------
+// One training batch in two launches.
+//
+// k_lg_batch: ROWS samples per workgroup, the whole way there and back: standardized inputs, four layers, the loss
+// and dL/dY, and the three products dA = dZ W with gelu' between them.  Sixteen waves, a 16-wide tile of the
+// layer's outputs each.  The work of 256 samples is 0.25 GFLOP of bf16 and 0.8 MB of weights, microseconds at most,
+// so the chain of dependent steps bounds it: as eighteen launches (a GEMM a layer, gelu', conversions, column sums
+// each on their own) it took 163 us of kernels and 212 us a call at 256 samples.  Activations and gradients pass
+// between the layers in LDS, gelu' stays in registers (its erf is the forward's), and the weights of the next layer
+// are asked for before the barrier that ends this one, in the packed order of lg_put.
+// ROWS = 16 fills the rows of the matrix instruction.  ROWS = 4 repeats its four rows four times there, so that a
+// lane finds every row of its column in its accumulator and takes one: the matrix work is far from its bound, and
+// erf, exp and the sixteen waves' other vector work spread over four times as many CUs.
+// Each product keeps the order of sums of a tile-by-tile GEMM over k (KS = 4: four interleaved chains, for few
+// rows), as its result is rounded to bf16 for the next layer.
+// Left for k_lg_grad: the inputs, activations and gradients of all samples in operand order (tile of 16 columns,
+// step of 16 samples, lane, four samples: what a lane holds of its tile of C is what the next product reads), the
+// sums of dZ over this workgroup's samples, and every sample's loss.
+// Measured at 256 samples: 22 us (34 us with ROWS = 16), and 36 us for the call with k_lg_grad's 4.2 us.
+// ---------------------------------------------------------------------------
+constexpr int kMaxSteps = kIn / 16;
+static_assert(kHid == 256 && kOut <= kHid && kPod == 64 && kIn >= kHid, "tiles of k_lg_batch: sixteen waves");
+constexpr int kSX = kIn + 16, kSH = kHid + 16, kSY = kOut + 4;  // LDS row strides: rows on different banks
+constexpr int kDb = 3 * kHid + kOut;                            // bias gradients, layer by layer
+
+template <int STEPS>
+__device__ __forceinline__ void lg_load(uint2 (&b)[kMaxSteps], const uint16_t *__restrict__ w, int tile, int lane) {
+    const uint2 *p = reinterpret_cast<const uint2 *>(w) + (size_t)tile * STEPS * 64 + lane;
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) b[s] = p[s * 64];
+}
+// row: this lane's row of the A operand in LDS, at its four k of the first step
+template <int STEPS, int KS>
+__device__ __forceinline__ fl4 lg_mma(const uint16_t *row, const uint2 (&b)[kMaxSteps]) {
+    fl4 acc[KS];
+#pragma unroll
+    for (int q = 0; q < KS; q++) acc[q] = fl4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+        bf4 av, bv;
+        __builtin_memcpy(&av, row + 16 * s, sizeof av);
+        __builtin_memcpy(&bv, &b[s], sizeof bv);
+        acc[s % KS] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[s % KS], 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 1; q < KS; q++) acc[0] += acc[q];
+    return acc[0];
+}
+// a lane's values of a tile (ROWS = 16: rows 4g .. 4g+3 of column r; 4: row g) into the LDS rows and, four rows of a
+// column together, into memory
+template <int ROWS>
+__device__ __forceinline__ void lg_keep(const float (&v)[ROWS / 4], uint16_t *lds, int stride, int col, int g,
+                                        uint16_t *__restrict__ out, size_t at) {
+    if constexpr (ROWS == 16) {
+        uint16_t h[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            h[i] = f2bf(v[i]);
+            if (lds) lds[(4 * g + i) * stride + col] = h[i];
         }
-        pw[2 * q] = pr;
-        pw[2 * q + 1] = pi;
-        const float cr = y[6 + 2 * q], ci = y[7 + 2 * q];
-        const float qr = s[S_Q + 2 * q], qi = s[S_Q + 2 * q + 1];
+        reinterpret_cast<uint2 *>(out)[at] = make_uint2(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16);
+    } else {
+        const uint32_t h = f2bf(v[0]);
+        if (lds) lds[g * stride + col] = (uint16_t)h;
+        const uint32_t two = h | (uint32_t)__shfl_xor((int)h, 16, 64) << 16;
+        const uint32_t next = (uint32_t)__shfl_xor((int)two, 32, 64);
+        if (g == 0) reinterpret_cast<uint2 *>(out)[at] = make_uint2(two, next);
+    }
+}
+// rows of bf16 in LDS (cols columns) into memory, four rows of a column together
+template <int ROWS>
+__device__ __forceinline__ void lg_pack(const uint16_t *lds, int stride, int cols, int t0, int nt, int blk, int steps,
+                                        uint16_t *__restrict__ out) {
+    constexpr int Q = ROWS / 4;
+    for (int e = t0; e < cols * Q; e += nt) {
+        const int c = e / Q, q = e % Q, grp = blk * Q + q;  // groups of four samples: four to a step
+        const uint16_t *h = lds + 4 * q * stride + c;
+        reinterpret_cast<uint2 *>(out)[((size_t)(c >> 4) * steps + (grp >> 2)) * 64 + (grp & 3) * 16 + (c & 15)] =
+            make_uint2(h[0] | (uint32_t)h[stride] << 16, h[2 * stride] | (uint32_t)h[3 * stride] << 16);
+    }
+}
+
+struct LgBatch {  // device pointers of a batch of M samples
+    const float *samples;
+    const int *idx;
+    const float *mean, *stdv, *p;
+    const uint16_t *fw, *bw;
+    uint16_t *x, *a[3], *g[4];  // packed operands of k_lg_grad
+    float *db, *loss;           // [M/ROWS][kDb], [M]
+};
+
+template <int KS, int ROWS>
+__global__ __launch_bounds__(1024) void k_lg_batch(LgBatch P, int M) {
+    constexpr int E = ROWS / 4;  // values a lane holds of its tile
+    constexpr int kRowBytes = 16 * (kSX + kSH) * 2, kPodBytes = ROWS * kPod * 12 * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char pool[kPodBytes > kRowBytes ? kPodBytes : kRowBytes];
+    __shared__ float Y[ROWS][kSY];
+    uint16_t *const bx = reinterpret_cast<uint16_t *>(pool), *const bh = bx + 16 * kSX;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const int ra = ROWS == 16 ? r : r & 3;  // this lane's row of the A operand
+    const int blk = blockIdx.x, steps = M / 16, n = w * 16 + r, ws = w % ROWS, m = blk * ROWS + ws;
+    // where this lane's four samples of tile w go
+    const size_t at = ROWS == 16 ? ((size_t)w * steps + blk) * 64 + lane
+                                 : ((size_t)w * steps + (blk >> 2)) * 64 + (blk & 3) * 16 + r;
+    const float *s = P.samples + (size_t)P.idx[m] * kSample;
+    uint2 b[kMaxSteps];
+    lg_load<kIn / 16>(b, P.fw, w, lane);
+    for (int t = lane + 64 * (w / ROWS); t < kIn; t += 64 * (16 / ROWS))
+        bx[ws * kSX + t] = t < F_END ? f2bf((s[S_FEAT + t] - P.mean[t]) / P.stdv[t]) : (uint16_t)0;
+    __syncthreads();
+    lg_pack<ROWS>(bx, kSX, kIn, threadIdx.x, 1024, blk, steps, P.x);
+    float dg[3][E], v[E];  // gelu' of the pre-activations, the values on their way
+    fl4 acc = lg_mma<kIn / 16, KS>(bx + ra * kSX + 4 * g, b);
+    auto forward = [&](int l, float bias, uint16_t *dst, int stride) {
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            const float z = (ROWS == 16 ? acc[i] : g == 0 ? acc[0] : g == 1 ? acc[1] : g == 2 ? acc[2] : acc[3]) + bias;
+            v[i] = gelu(z);
+            dg[l][i] = gelu_d(z);
+        }
+        lg_keep<ROWS>(v, dst, stride, n, g, P.a[l], at);
+    };
+    lg_load<kHid / 16>(b, P.fw + P_W2, w, lane);
+    forward(0, P.p[P_B1 + n], bh, kSH);
+    __syncthreads();
+    acc = lg_mma<kHid / 16, KS>(bh + ra * kSH + 4 * g, b);
+    lg_load<kHid / 16>(b, P.fw + P_W3, w, lane);
+    forward(1, P.p[P_B2 + n], bx, kSX);
+    __syncthreads();
+    acc = lg_mma<kHid / 16, KS>(bx + ra * kSX + 4 * g, b);
+    if (w < kOut / 16) lg_load<kHid / 16>(b, P.fw + P_W4, w, lane);
+    forward(2, P.p[P_B3 + n], bh, kSH);
+    // the terms of sample w of this workgroup in the loss: lane q those of POD coefficient q, lanes below 6 a row of G
+    float pk[12], gl[6];
+    const int t6 = lane < 6 ? lane : 0;
+#pragma unroll
+    for (int k = 0; k < 12; k++) pk[k] = s[S_P + lane * 12 + k];
+#pragma unroll
+    for (int k = 0; k < 6; k++) gl[k] = s[S_G + t6 * 6 + k];
+    const float sa = s[S_A + t6], beta = s[S_BETA], qr = s[S_Q + 2 * lane], qi = s[S_Q + 2 * lane + 1];
+    __syncthreads();
+    if (w < kOut / 16) {
+        acc = lg_mma<kHid / 16, KS>(bh + ra * kSH + 4 * g, b);
+        const float bias = P.p[P_B4 + n];
+        if (ROWS == 16) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) Y[(4 * g + i) % ROWS][n] = acc[i] + bias;
+        } else if (g == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) Y[i][n] = acc[i] + bias;
+        }
+    }
+    lg_load<kOut / 16>(b, P.bw + P_W4, w, lane);
+    __syncthreads();
+    // loss L = |e_hat - D w - U c|^2 / beta (the quadratic form) and dL/dY / M
+    float *pod = reinterpret_cast<float *>(pool) + ws * kPod * 12;
+    const float *y = Y[ws];
+    const float ib = beta > 0 ? 1.0f / beta : 0.0f;
+    float contrib = 0, d0 = 0, d1 = 0, dw = 0;
+    if (w < ROWS) {
+        float pr = 0, pi = 0;
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            pr += pk[2 * k] * y[k];
+            pi += pk[2 * k + 1] * y[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 12; k++) pod[lane * 12 + k] = pk[k];
+        const float cr = y[6 + 2 * lane], ci = y[7 + 2 * lane];
         contrib += -2.f * (cr * qr + ci * qi) + cr * cr + ci * ci + 2.f * (cr * pr + ci * pi);
-        dY[(size_t)m * kOut + 6 + 2 * q] = 2.f * ib * (cr - qr + pr) / M;
-        dY[(size_t)m * kOut + 7 + 2 * q] = 2.f * ib * (ci - qi + pi) / M;
+        d0 = 2.f * ib * (cr - qr + pr) / M;
+        d1 = 2.f * ib * (ci - qi + pi) / M;
     }
     __syncthreads();
-    if (t < 6) {
-        float gw = 0;
-        for (int l = 0; l < 6; l++) gw += s[S_G + t * 6 + l] * w[l];
-        float pc = 0;
-        for (int q = 0; q < kPod; q++) pc += s[S_P + (q * 6 + t) * 2] * y[6 + 2 * q] + s[S_P + (q * 6 + t) * 2 + 1] * y[7 + 2 * q];
-        contrib += -2.f * w[t] * s[S_A + t] + w[t] * gw;
-        dY[(size_t)m * kOut + t] = 2.f * ib * (-s[S_A + t] + gw + pc) / M;
+    if (w < ROWS) {
+        if (lane < 6) {
+            float gw = 0;
+#pragma unroll
+            for (int l = 0; l < 6; l++) gw += gl[l] * y[l];
+            float pc = 0;
+#pragma unroll 8
+            for (int q = 0; q < kPod; q++)
+                pc += pod[(q * 6 + lane) * 2] * y[6 + 2 * q] + pod[(q * 6 + lane) * 2 + 1] * y[7 + 2 * q];
+            contrib += -2.f * y[lane] * sa + y[lane] * gw;
+            dw = 2.f * ib * (-sa + gw + pc) / M;
+        }
+        const double tot = wave_sum((double)contrib);
+        if (lane == 0) P.loss[m] = beta > 0 ? 1.0f + (float)tot * ib : 0.f;
     }
-    if (t < kOut - (6 + 2 * kPod)) dY[(size_t)m * kOut + 6 + 2 * kPod + t] = 0.f;  // padding outputs
-    part[t] = contrib;
+    __syncthreads();  // every read of Y and of the POD terms is done
+    if (w < ROWS) {
+        Y[ws][6 + 2 * lane] = d0;
+        Y[ws][7 + 2 * lane] = d1;
+        bx[ws * kSX + 6 + 2 * lane] = f2bf(d0);
+        bx[ws * kSX + 7 + 2 * lane] = f2bf(d1);
+        if (lane < 6) {
+            Y[ws][lane] = dw;
+            bx[ws * kSX + lane] = f2bf(dw);
+        } else if (lane < kOut - 2 * kPod) {  // padding outputs
+            Y[ws][2 * kPod + lane] = 0.f;
+            bx[ws * kSX + 2 * kPod + lane] = 0;
+        }
+    }
     __syncthreads();
-    if (t == 0) {
-        float tot = 0;
-        for (int k = 0; k < 64; k++) tot += part[k];
-        loss[m] = beta > 0 ? 1.0f + tot * ib : 0.f;
+    float *db = P.db + (size_t)blk * kDb;
+    if (threadIdx.x < kOut) {
+        float c = 0;
+#pragma unroll
+        for (int k = 0; k < ROWS; k++) c += Y[k][threadIdx.x];
+        db[3 * kHid + threadIdx.x] = c;
+    } else if (threadIdx.x >= 256) {
+        lg_pack<ROWS>(bx, kSX, kOut, threadIdx.x - 256, 768, blk, steps, P.g[3]);
+    }
+    // dZ_l = (dZ_{l+1} W_{l+1}) gelu'(Z_l)
+    acc = lg_mma<kOut / 16, 1>(bx + ra * kSX + 4 * g, b);
+#pragma unroll
+    for (int l = 2; l >= 0; l--) {
+        if (l == 2) lg_load<kHid / 16>(b, P.bw + P_W3, w, lane);
+        if (l == 1) lg_load<kHid / 16>(b, P.bw + P_W2, w, lane);
+        float c = 0;
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            v[i] = (ROWS == 16 ? acc[i] : g == 0 ? acc[0] : g == 1 ? acc[1] : g == 2 ? acc[2] : acc[3]) * dg[l][i];
+            c += v[i];
+        }
+        uint16_t *const dst = l == 2 ? bh : l == 1 ? bx : (uint16_t *)nullptr;
+        lg_keep<ROWS>(v, dst, l == 1 ? kSX : kSH, n, g, P.g[l], at);
+        c += __shfl_xor(c, 16, 64);
+        c += __shfl_xor(c, 32, 64);
+        if (g == 0) db[l * kHid + n] = c;
+        if (l > 0) {
+            __syncthreads();
+            acc = lg_mma<kHid / 16, 1>(dst + ra * (l == 1 ? kSX : kSH) + 4 * g, b);
+        }
     }
 }
 
-// mean of loss[0..M) into out[0]
-__global__ void k_lg_mean(const float *__restrict__ loss, int M, float *__restrict__ out) {
-    __shared__ float sh[256];
-    float s = 0;
-    for (int m = threadIdx.x; m < M; m += blockDim.x) s += loss[m];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = 0;
-        for (int k = 0; k < (int)blockDim.x; k++) t += sh[k];
-        out[0] = t / M;
+// Gradients of the batch from what k_lg_batch left: a block per 16x16 tile of every dW[n][k] = sum_m dZ[m][n]
+// A[m][k] (four waves, the steps of 16 samples in turn, added in wave order), then blocks of 64 bias gradients,
+// then one block for the mean loss.  4.2 us at 256 samples (the seven launches before it: 94 us).
+constexpr int kTiles0 = (kHid / 16) * (kIn / 16), kTiles1 = (kHid / 16) * (kHid / 16), kTiles3 = (kOut / 16) * (kHid / 16);
+constexpr int kGradTiles = kTiles0 + 2 * kTiles1 + kTiles3, kGradBias = (kDb + 63) / 64;
+__global__ __launch_bounds__(256) void k_lg_grad(LgBatch P, int M, int nparts, float *__restrict__ grad,
+                                                float *__restrict__ mean) {
+    __shared__ fl4 red[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, g = lane >> 4, steps = M / 16;
+    int tile = blockIdx.x;
+    if (tile < kGradTiles) {
+        int l = 0, K = kIn;
+        size_t wo = P_W1;
+        if (tile >= kTiles0) {
+            tile -= kTiles0;
+            l = 1 + tile / kTiles1;
+            tile %= kTiles1;
+            K = kHid;
+            wo = l == 1 ? P_W2 : l == 2 ? P_W3 : P_W4;
+        }
+        const int tn = tile / (K / 16), tk = tile % (K / 16);
+        const uint16_t *A = l == 0 ? P.x : l == 1 ? P.a[0] : l == 2 ? P.a[1] : P.a[2];
+        const uint16_t *G = l == 0 ? P.g[0] : l == 1 ? P.g[1] : l == 2 ? P.g[2] : P.g[3];
+        const uint2 *ap = reinterpret_cast<const uint2 *>(G) + (size_t)tn * steps * 64 + lane;
+        const uint2 *bp = reinterpret_cast<const uint2 *>(A) + (size_t)tk * steps * 64 + lane;
+        fl4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int s0 = w; s0 < steps; s0 += 16) {
+            uint2 au[4], bu[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const size_t s = min(s0 + 4 * u, steps - 1);
+                au[u] = ap[s * 64];
+                bu[u] = bp[s * 64];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (s0 + 4 * u < steps) {
+                    bf4 av, bv;
+                    __builtin_memcpy(&av, &au[u], sizeof av);
+                    __builtin_memcpy(&bv, &bu[u], sizeof bv);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
+                }
+        }
+        red[w][lane] = acc;
+        __syncthreads();
+        if (w != 0) return;
+#pragma unroll
+        for (int q = 1; q < 4; q++) acc += red[q][lane];
+#pragma unroll
+        for (int i = 0; i < 4; i++) grad[wo + (size_t)(tn * 16 + 4 * g + i) * K + tk * 16 + r] = acc[i];
+    } else if (tile < kGradTiles + kGradBias) {
+        float *sh = reinterpret_cast<float *>(&red[0][0]);
+        const int c = (tile - kGradTiles) * 64 + lane;
+        float s = 0;
+        if (c < kDb)
+            for (int k0 = w; k0 < nparts; k0 += 64) {
+                float t[16];
+#pragma unroll
+                for (int u = 0; u < 16; u++) t[u] = P.db[(size_t)min(k0 + 4 * u, nparts - 1) * kDb + c];
+#pragma unroll
+                for (int u = 0; u < 16; u++) s += k0 + 4 * u < nparts ? t[u] : 0.f;
+            }
+        sh[w * 64 + lane] = s;
+        __syncthreads();
+        if (w == 0 && c < kDb) {
+            const int l = c / kHid;
+            const size_t bo = l == 0 ? P_B1 : l == 1 ? P_B2 : l == 2 ? P_B3 : P_B4;
+            grad[bo + c - l * kHid] = (sh[lane] + sh[64 + lane]) + (sh[128 + lane] + sh[192 + lane]);
+        }
+    } else {
+        double t[1] = {0};
+        for (int k = threadIdx.x; k < M; k += 256) t[0] += P.loss[k];
+        block_sum<1>(t, reinterpret_cast<double *>(&red[0][0]));
+        if (threadIdx.x == 0) mean[0] = (float)(t[0] / M);
     }
-}
-
-// bf16 copy of an FP32 matrix
-__global__ void k_lg_tobf(long n, const float *__restrict__ x, uint16_t *__restrict__ y) {
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) y[i] = f2bf(x[i]);
-}
-
-// dZ = dA * gelu'(Z), and its bf16 copy
-__global__ void k_lg_gelu_back(long n, const float *__restrict__ dA, const float *__restrict__ Z, float *__restrict__ dZ,
-                               uint16_t *__restrict__ G) {
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const float v = dA[i] * gelu_d(Z[i]);
-        dZ[i] = v;
-        G[i] = f2bf(v);
-    }
-}
-
-// column sums db[n] = sum_m dZ[m][n]: 64 columns per block, 4 row groups
-__global__ __launch_bounds__(256) void k_lg_colsum(int M, int N, const float *__restrict__ dZ, float *__restrict__ db) {
-    __shared__ float sh[4][64];
-    const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
-    const int n = blockIdx.x * 64 + c;
-    float s = 0;
-    if (n < N)
-        for (int m = g; m < M; m += 4) s += dZ[(size_t)m * N + n];
-    sh[g][c] = s;
-    __syncthreads();
-    if (g == 0 && n < N) db[n] = (sh[0][c] + sh[1][c]) + (sh[2][c] + sh[3][c]);
 }
 
 // Adam step on the FP32 parameters, refreshing the bf16 weights
 __global__ void k_lg_adam(long n, float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m1,
                           float *__restrict__ m2, float lr, float b1, float b2, float eps, float c1, float c2,
-                          uint16_t *__restrict__ pbf) {
+                          uint16_t *__restrict__ pbf, uint16_t *__restrict__ pfw, uint16_t *__restrict__ pbw) {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         const float gi = g[i];
         const float a = b1 * m1[i] + (1.f - b1) * gi;
@@ -759,7 +995,7 @@ __global__ void k_lg_adam(long n, float *__restrict__ p, const float *__restrict
         m2[i] = v;
         const float pi = p[i] - lr * (a / c1) / (sqrtf(v / c2) + eps);
         p[i] = pi;
-        pbf[i] = f2bf(pi);
+        lg_put((int)i, f2bf(pi), pbf, pfw, pbw);
     }
 }
 
@@ -795,11 +1031,13 @@ struct gade_lg {
     bool net = false;
     float *p = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr;  // [P_TOTAL]
     uint16_t *pbf = nullptr;      // bf16 copy (weights)
+    uint16_t *pfw = nullptr, *pbw = nullptr;  // the weights again, in the training kernel's operand orders
+    float *h_loss = nullptr;      // pinned: the mean loss of gade_lg_grad
     long adam_t = 0;
     // training buffers (batch Mt)
     int Mt = 0;
     uint16_t *xt = nullptr, *at[3] = {}, *gt[4] = {};
-    float *zt[3] = {}, *yt = nullptr, *dy = nullptr, *da = nullptr, *dz = nullptr, *loss = nullptr;
+    float *zt[3] = {}, *yt = nullptr, *db = nullptr, *loss = nullptr;
 };
 
 namespace gade {
@@ -808,8 +1046,8 @@ void lg_free(gade_lg *lg) {
     if (!lg) return;
     std::vector<void *> ptrs = {lg->U, lg->U32, lg->UT32, lg->ppart, lg->V, lg->part, lg->gram, lg->proj, lg->lres, lg->feat, lg->mean, lg->stdv,
                                 lg->zmax, lg->oor, lg->uses,
-                                lg->xin, lg->yi, lg->p, lg->g, lg->m1, lg->m2, lg->pbf, lg->xt, lg->yt, lg->dy,
-                                lg->da, lg->dz, lg->loss};
+                                lg->xin, lg->yi, lg->p, lg->g, lg->m1, lg->m2, lg->pbf, lg->pfw, lg->pbw, lg->xt, lg->yt,
+                                lg->db, lg->loss};
     for (int k = 0; k < 3; k++) {
         ptrs.push_back(lg->zi[k]);
         ptrs.push_back(lg->ai[k]);
@@ -819,6 +1057,7 @@ void lg_free(gade_lg *lg) {
     for (int k = 0; k < 4; k++) ptrs.push_back(lg->gt[k]);
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
+    if (lg->h_loss) (void)hipHostFree(lg->h_loss);
     delete lg;
 }
 
@@ -882,7 +1121,8 @@ int lg_ensure(gade_model *m) {
 int lg_net_alloc(gade_lg *lg) {
     if (lg->net) return GADE_OK;
     for (float **q : {&lg->p, &lg->g, &lg->m1, &lg->m2}) GADE_TRY(hip_alloc((void **)q, sizeof(float) * P_TOTAL));
-    GADE_TRY(hip_alloc((void **)&lg->pbf, sizeof(uint16_t) * P_TOTAL));
+    for (uint16_t **q : {&lg->pbf, &lg->pfw, &lg->pbw}) GADE_TRY(hip_alloc((void **)q, sizeof(uint16_t) * P_TOTAL));
+    GADE_HIP(hipHostMalloc((void **)&lg->h_loss, sizeof(float), hipHostMallocDefault));
     GADE_HIP(hipMemset(lg->g, 0, sizeof(float) * P_TOTAL));
     lg->net = true;
     return GADE_OK;
@@ -890,7 +1130,7 @@ int lg_net_alloc(gade_lg *lg) {
 
 int lg_train_alloc(gade_lg *lg, int Mt) {
     if (lg->Mt >= Mt) return GADE_OK;
-    for (void *q : {(void *)lg->xt, (void *)lg->yt, (void *)lg->dy, (void *)lg->da, (void *)lg->dz, (void *)lg->loss})
+    for (void *q : {(void *)lg->xt, (void *)lg->yt, (void *)lg->db, (void *)lg->loss})
         if (q) (void)hipFree(q);
     for (int k = 0; k < 3; k++) {
         if (lg->at[k]) (void)hipFree(lg->at[k]);
@@ -901,9 +1141,7 @@ int lg_train_alloc(gade_lg *lg, int Mt) {
     lg->Mt = Mt;
     GADE_TRY(hip_alloc((void **)&lg->xt, sizeof(uint16_t) * Mt * kIn));
     GADE_TRY(hip_alloc((void **)&lg->yt, sizeof(float) * Mt * kOut));
-    GADE_TRY(hip_alloc((void **)&lg->dy, sizeof(float) * Mt * kOut));
-    GADE_TRY(hip_alloc((void **)&lg->da, sizeof(float) * Mt * kHid));
-    GADE_TRY(hip_alloc((void **)&lg->dz, sizeof(float) * Mt * kHid));
+    GADE_TRY(hip_alloc((void **)&lg->db, sizeof(float) * (Mt / 4) * kDb));
     GADE_TRY(hip_alloc((void **)&lg->loss, sizeof(float) * Mt));
     for (int k = 0; k < 3; k++) {
         GADE_TRY(hip_alloc((void **)&lg->at[k], sizeof(uint16_t) * Mt * kHid));
@@ -942,45 +1180,38 @@ void mlp_forward(const gade_lg *lg, hipStream_t st, int M, const uint16_t *X, fl
         const float *bias = lg->p + kBoff[l];
         if (M <= kSplitKRows) {
             if (l < 3)
-                hipLaunchKernelGGL((k_gemm_bf16<EPI_BIAS_GELU, 4>), grid, dim3(256), 0, st, M, N, K, in, (long)K, 1L,
-                                   W, 1L, (long)K, Z[l], N, bias, A[l], N);
+                hipLaunchKernelGGL((k_gemm_bf16<EPI_BIAS_GELU, 4>), grid, dim3(256), 0, st, M, N, K, in, W, Z[l], N,
+                                   bias, A[l], N);
             else
-                hipLaunchKernelGGL((k_gemm_bf16<EPI_BIAS, 4>), grid, dim3(256), 0, st, M, N, K, in, (long)K, 1L, W,
-                                   1L, (long)K, Y, N, bias, (uint16_t *)nullptr, 0);
+                hipLaunchKernelGGL((k_gemm_bf16<EPI_BIAS, 4>), grid, dim3(256), 0, st, M, N, K, in, W, Y, N, bias,
+                                   (uint16_t *)nullptr, 0);
         } else if (l < 3) {
-            hipLaunchKernelGGL(k_gemm_bf16<EPI_BIAS_GELU>, grid, dim3(64), 0, st, M, N, K, in, (long)K, 1L, W, 1L,
-                               (long)K, Z[l], N, bias, A[l], N);
+            hipLaunchKernelGGL(k_gemm_bf16<EPI_BIAS_GELU>, grid, dim3(64), 0, st, M, N, K, in, W, Z[l], N, bias, A[l],
+                               N);
         } else {
-            hipLaunchKernelGGL(k_gemm_bf16<EPI_BIAS>, grid, dim3(64), 0, st, M, N, K, in, (long)K, 1L, W, 1L, (long)K,
-                               Y, N, bias, (uint16_t *)nullptr, 0);
+            hipLaunchKernelGGL(k_gemm_bf16<EPI_BIAS>, grid, dim3(64), 0, st, M, N, K, in, W, Y, N, bias,
+                               (uint16_t *)nullptr, 0);
         }
         if (l < 3) in = A[l];
     }
 }
 
-// backward of M rows from dY (FP32 [M][kOut]): gradients of every parameter into lg->g
-void mlp_backward(gade_lg *lg, hipStream_t st, int M, const uint16_t *X) {
-    hipLaunchKernelGGL(k_lg_tobf, dim3(64), dim3(256), 0, st, (long)M * kOut, (const float *)lg->dy, lg->gt[3]);
-    const float *dZ = lg->dy;
-    for (int l = kLayers - 1; l >= 0; l--) {
-        const int K = kLin[l], N = kLout[l];
-        const uint16_t *Gl = lg->gt[l];
-        const uint16_t *Ain = l > 0 ? lg->at[l - 1] : X;
-        // dW[n][k] = sum_m dZ[m][n] A[m][k]
-        hipLaunchKernelGGL(k_gemm_bf16<EPI_STORE>, dim3((N / 16) * (K / 16)), dim3(64), 0, st, N, K, M, Gl, 1L,
-                           (long)N, Ain, (long)K, 1L, lg->g + kWoff[l], K, (const float *)nullptr,
-                           (uint16_t *)nullptr, 0);
-        hipLaunchKernelGGL(k_lg_colsum, dim3((N + 63) / 64), dim3(256), 0, st, M, N, dZ, lg->g + kBoff[l]);
-        if (l > 0) {
-            // dA[m][k] = sum_n dZ[m][n] W[n][k], then dZ_{l-1} = dA * gelu'(Z_{l-1})
-            hipLaunchKernelGGL(k_gemm_bf16<EPI_STORE>, dim3((M / 16) * (K / 16)), dim3(64), 0, st, M, K, N, Gl,
-                               (long)N, 1L, lg->pbf + kWoff[l], (long)K, 1L, lg->da, K, (const float *)nullptr,
-                               (uint16_t *)nullptr, 0);
-            hipLaunchKernelGGL(k_lg_gelu_back, dim3(64), dim3(256), 0, st, (long)M * K, (const float *)lg->da,
-                               (const float *)lg->zt[l - 1], lg->dz, lg->gt[l - 1]);
-            dZ = lg->dz;
-        }
-    }
+// Four samples a workgroup while every workgroup finds a CU of its own (256), sixteen beyond: a call takes 36 and
+// 47 us at 256 samples, 44 and 54 at 1024, 64 and 57 at 1536, 203 and 119 at 8192.
+constexpr int kFewRows = 1024;
+// loss and gradient of the batch idx [M] of samples: the mean loss into mean, the gradient into grad [P_TOTAL]
+// (the forward sums in the order that mlp_forward uses for as many rows)
+void lg_batch(gade_lg *lg, hipStream_t st, const float *samples, const int *idx, int M, float *grad, float *mean) {
+    const LgBatch P = {samples, idx, lg->mean, lg->stdv, lg->p, lg->pfw, lg->pbw, lg->xt,
+                       {lg->at[0], lg->at[1], lg->at[2]}, {lg->gt[0], lg->gt[1], lg->gt[2], lg->gt[3]}, lg->db, lg->loss};
+    const int rows = M <= kFewRows ? 4 : 16;
+    if (M <= kSplitKRows)
+        hipLaunchKernelGGL((k_lg_batch<4, 4>), dim3(M / 4), dim3(1024), 0, st, P, M);
+    else if (rows == 4)
+        hipLaunchKernelGGL((k_lg_batch<1, 4>), dim3(M / 4), dim3(1024), 0, st, P, M);
+    else
+        hipLaunchKernelGGL((k_lg_batch<1, 16>), dim3(M / 16), dim3(1024), 0, st, P, M);
+    hipLaunchKernelGGL(k_lg_grad, dim3(kGradTiles + kGradBias + 1), dim3(256), 0, st, P, M, M / rows, grad, mean);
 }
 
 }  // namespace
@@ -1266,7 +1497,7 @@ int gade_lg_set_params(gade_model_t *m, const float *params) {
     GADE_HIP(hipMemset(lg->m1, 0, sizeof(float) * P_TOTAL));
     GADE_HIP(hipMemset(lg->m2, 0, sizeof(float) * P_TOTAL));
     lg->adam_t = 0;
-    hipLaunchKernelGGL(k_lg_tobf, dim3(256), dim3(256), 0, m->stream, (long)P_TOTAL, (const float *)lg->p, lg->pbf);
+    hipLaunchKernelGGL(k_lg_tobf, dim3(256), dim3(256), 0, m->stream, (const float *)lg->p, lg->pbf, lg->pfw, lg->pbw);
     GADE_HIP(hipGetLastError());
     GADE_HIP(hipStreamSynchronize(m->stream));
     return GADE_OK;
@@ -1314,22 +1545,11 @@ int gade_lg_grad(gade_model_t *m, const float *samples, const int *idx, int M, f
     if (!m->lg || !m->lg->net) return GADE_EINVAL;
     gade_lg *lg = m->lg;
     GADE_TRY(lg_train_alloc(lg, M));
-    float *d_mean = nullptr;
-    GADE_TRY(hip_alloc((void **)&d_mean, sizeof(float)));
-    hipLaunchKernelGGL(k_lg_gather, dim3(M), dim3(64), 0, m->stream, samples, idx, (const float *)lg->mean,
-                       (const float *)lg->stdv, lg->xt);
-    mlp_forward(lg, m->stream, M, lg->xt, lg->zt, lg->at, lg->yt);
-    hipLaunchKernelGGL(k_lg_loss, dim3(M), dim3(64), 0, m->stream, (const float *)lg->yt, samples, idx, M, lg->dy,
-                       lg->loss);
-    hipLaunchKernelGGL(k_lg_mean, dim3(1), dim3(256), 0, m->stream, (const float *)lg->loss, M, d_mean);
-    mlp_backward(lg, m->stream, M, lg->xt);
+    // the gradient goes straight to the caller's buffer, the loss to pinned host memory
+    lg_batch(lg, m->stream, samples, idx, M, grad ? grad : lg->g, lg->h_loss);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && grad)
-        e = hipMemcpyAsync(grad, lg->g, sizeof(float) * P_TOTAL, hipMemcpyDeviceToDevice, m->stream);
-    if (e == hipSuccess && loss_out)
-        e = hipMemcpyAsync(loss_out, d_mean, sizeof(float), hipMemcpyDeviceToHost, m->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-    (void)hipFree(d_mean);
+    if (e == hipSuccess && loss_out) *loss_out = *lg->h_loss;
     if (e != hipSuccess) {
         set_error(std::string("gade_lg_grad: ") + hipGetErrorString(e));
         return GADE_EHIP;
@@ -1354,17 +1574,11 @@ int gade_lg_train(gade_model_t *m, const float *samples, const int *idx, int M, 
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     for (int k = 0; k < nsteps; k++) {
         const int *ik = idx + (size_t)k * M;
-        hipLaunchKernelGGL(k_lg_gather, dim3(M), dim3(64), 0, m->stream, samples, ik, (const float *)lg->mean,
-                           (const float *)lg->stdv, lg->xt);
-        mlp_forward(lg, m->stream, M, lg->xt, lg->zt, lg->at, lg->yt);
-        hipLaunchKernelGGL(k_lg_loss, dim3(M), dim3(64), 0, m->stream, (const float *)lg->yt, samples, ik, M, lg->dy,
-                           lg->loss);
-        hipLaunchKernelGGL(k_lg_mean, dim3(1), dim3(256), 0, m->stream, (const float *)lg->loss, M, d_hist + k);
-        mlp_backward(lg, m->stream, M, lg->xt);
+        lg_batch(lg, m->stream, samples, ik, M, lg->g, d_hist + k);
         lg->adam_t++;
         const float c1 = 1.f - std::pow(b1, (float)lg->adam_t), c2 = 1.f - std::pow(b2, (float)lg->adam_t);
         hipLaunchKernelGGL(k_lg_adam, dim3(256), dim3(256), 0, m->stream, (long)P_TOTAL, lg->p, (const float *)lg->g,
-                           lg->m1, lg->m2, lr, b1, b2, eps, c1, c2, lg->pbf);
+                           lg->m1, lg->m2, lr, b1, b2, eps, c1, c2, lg->pbf, lg->pfw, lg->pbw);
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && loss_hist)
