@@ -260,14 +260,14 @@ constexpr int kAngListU = 4;
 // products of the complex form (cf: h0, then h1).
 template <bool RC, class T>
 __device__ __forceinline__ void ang_terms(const T xv, const int kc, const T *__restrict__ cf, T &z0, T &z2, T &w0,
-                                          T &w1) {
+                                          T &w1, const bool has_z2 = true, const bool has_w1 = true) {
     using Rt = typename cx<T>::R;
     if constexpr (RC) {
         const T h = cf[0], hk = cf[1];
         z0 = rfma(h.x, xv, z0);
-        z2 = rfma(hk.x, xv, z2);
+        if (has_z2) z2 = rfma(hk.x, xv, z2);
         w0 = rfma(h.y, xv, w0);
-        w1 = rfma(hk.y, xv, w1);
+        if (has_w1) w1 = rfma(hk.y, xv, w1);
     } else {
         z0 = cfma(cf[0], xv, z0);
         z2 = cfma(cscale(cf[0], (Rt)kc), xv, z2);
@@ -626,6 +626,60 @@ __global__ __launch_bounds__(256) void k_gsums_dia(const E *__restrict__ gs, con
     }
 }
 
+// The zero pattern of a dual-kinetic-balance basis (KB).  A function of the first output half has no kappa in the
+// component that the row (first) index of a coupling g_n takes, one of the second half is linear in kappa there; for
+// the column index it is the other way round.  With g_n the coefficient of kappa^i kappa'^j, n = i + 2 j, the quadrants
+// (h, hp) of g_0 are all filled, g_1 has h = 1 only, g_2 hp = 0 only and g_3 (1, 0) only.  So of the eight (v, hp)
+// products of a pair, (1, 1) and (3, 0) vanish, and of the two output halves of the six others one has no kappa part
+// (h = 0 for v < 2, h = 1 for v >= 2): a quarter of the products and of the windows and 44 % of the coefficient bytes
+// need not exist.  kb_unit numbers the six; GD then holds per (l, unit) the half with pairs, then the other's sums as
+// single numbers, each [d][ip]: kb_words words.
+__host__ __device__ constexpr int kb_unit(int v, int hp) { return 3 * (v >> 1) + ((v & 1) ? 2 : hp); }
+__host__ __device__ inline size_t kb_words(int nd, int nhp) { return (size_t)nd * nhp * 3 / 2; }
+
+// k_gsums_dia<true> for that pattern, from the same terms in the same order
+__global__ __launch_bounds__(256) void k_gsums_kb(const double *__restrict__ gs, const double *__restrict__ gts,
+                                                  CoefGroup cg, int b0, size_t gd_stride, int lmax, int nd, int nhp,
+                                                  double2 *__restrict__ GD0, const int *gate, int gstride,
+                                                  const Coef6 *__restrict__ cf_dev, const int *__restrict__ gctl,
+                                                  int B) {
+    const int b = b0 + blockIdx.y;
+    GADE_GATED_B(gate, gstride, b);
+    const Coef6 cf = cf_dev ? cf_dev[(size_t)gctl[GC_WSLOT] * B + b] : cg.c[blockIdx.y];
+    double c_even[3], c_odd[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        c_even[j] = cf.c[2 * j + 1].y;
+        c_odd[j] = cf.c[2 * j].y;
+    }
+    double2 *__restrict__ GD = GD0 + (size_t)b * gd_stride;
+    const int Q = nd * nhp, S = 4 * Q;
+    const long long total = (long long)lmax * 12 * Q;
+    for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
+         idx += (long long)gridDim.x * blockDim.x) {
+        const int t = (int)(idx / Q);  // (l, unit, half without kappa)
+        const int e = (int)(idx - (long long)t * Q);
+        const int l = t / 12, u = (t >> 1) % 6, single = t & 1;
+        const int u3 = u % 3, v = 2 * (u / 3) + (u3 == 2), hp = u3 == 2 ? (u == 5) : u3;
+        const int h = (v < 2) != (single != 0);
+        const double *src = v < 2 ? gs : gts;
+        const int n1 = v == 0 ? 0 : v == 1 ? 2 : v == 2 ? 0 : 1, n2 = v == 0 ? 1 : v == 1 ? 3 : v == 2 ? 2 : 3;
+        double G1 = 0, G2 = 0;
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const double c = (l % 2 == 0) ? c_even[j] : c_odd[j];
+            const size_t o = (size_t)(l * 3 + j) * 4 * S + (size_t)(2 * h + hp) * Q + e;
+            G1 = fma(c, src[o + (size_t)n1 * S], G1);
+            if (!single) G2 = fma(c, src[o + (size_t)n2 * S], G2);
+        }
+        double2 *out = GD + (size_t)(t >> 1) * kb_words(nd, nhp);
+        if (single)
+            reinterpret_cast<double *>(out + Q)[e] = G1;
+        else
+            out[e] = make_double2(G1, G2);
+    }
+}
+
 // gs/gts gathered into DIA order once at setup; dia_src[(qd*nd+d)*nhp+ip] is
 // the radial CSR index of that entry or -1.
 __global__ void k_build_gdia(const double2 *__restrict__ g, const int *__restrict__ dia_src,
@@ -683,9 +737,9 @@ __global__ void k_build_DD(const double2 *__restrict__ D, const int *__restrict_
 // two operators), D = d(hp=0) + d(hp=1), and y = D + cH G.  Every (R, P, HV) runs these sums in the same order.
 // One wave per half running all four parts in turn (the form before) was a chain of ten staged windows: 31 us at 40
 // blocks of 110 functions, where nothing else fills the chip, and 72 us at 400 blocks of 510 after 42 us of angular
-// kernel.  This form (4 rows, both halves, FUSED, RC) takes 11 and 70 us with no angular kernel before it.  At 400 x
-// 510 it is bound by vector issue (2.0e7 wave instructions, about half the time) and by its loads' way through L1 (the
-// coefficients, then the gathered x): with neither loads nor LDS reads the same instructions take 52 us.
+// kernel.  This form (4 rows, both halves, FUSED, RC, KB) takes 11.5 and 60 us with no angular kernel before it.  At
+// 400 x 510 it is bound by vector and LDS issue, then by the coefficients' way through L1: with neither coefficient nor
+// x loads the same kernel takes 73 % of its time (66 % for eight instances), with the x loads alone 86 % (81 %).
 // FUSED: no V input.  The windows of V_{l,v} (all four parts of a half hp) are formed from x by the coupling
 // lists of phase A (aoff, ack, acf: the lists of k_angular_list), with the same terms in the same order as
 // k_angular_list forms V, so the results are bit-identical to the two-kernel form and V never goes to HBM.
@@ -694,7 +748,11 @@ __global__ void k_build_DD(const double2 *__restrict__ D, const int *__restrict_
 // four and half the coefficient bytes; the factor i (rot 2) or i*i (rot 1) is applied to the finished sum G.  The
 // terms left out are products with zero, so the results equal the complex form's bit for bit.  At 400 x 510 and 4 rows
 // the complex form takes 93 us where the real one takes 58 (both without FUSED), 16 and 11 us at 40 x 110.
-template <int BW, bool DUAL, class T, int R, int P, int HV, bool FUSED, bool RC>
+// KB (with RC): the zero pattern of kb_unit.  Waves 1 and 3 have one source half, the windows of the vanishing products
+// are neither formed nor staged, and the half without a kappa part takes single coefficients; the terms left out are
+// products with zero.  4 rows, both halves, FUSED: 400 x 510 67 us without and 60 with it, eight such instances 470 and
+// 388, 64 of 40 x 110 20 and 18; one of 40 x 110 is a chain of latencies, 11.7 and 11.5.
+template <int BW, bool DUAL, class T, int R, int P, int HV, bool FUSED, bool RC, bool KB>
 __global__ __launch_bounds__(256) void k_radial_dia(
     const T *__restrict__ x, const T *__restrict__ V, const T *__restrict__ GD, const T *__restrict__ DD,
     const int *__restrict__ tiles, const int *__restrict__ tile_q, const double *__restrict__ tile_k, int nblk, int n,
@@ -705,8 +763,12 @@ __global__ __launch_bounds__(256) void k_radial_dia(
     constexpr int SEG = 64 * P, ND = 2 * BW + 1, W = SEG + 2 * BW, RW = R / 4;
     constexpr int WS = P * dia_wp<P>();  // LDS slots of a window
     static_assert(R % 4 == 0, "each of the four waves finishes R/4 rows");
+    static_assert(RC || !KB, "the zero pattern's coefficients are real");
     using Rt = typename cx<T>::R;
-    __shared__ T sm[4 * 2 * R * WS];  // a window set per wave; reused for the sums over the waves
+    constexpr int SH = 2 * R * P * 64;  // a wave's share of the sums over the waves
+    constexpr int SETS = KB ? 6 : 8;    // window sets (part v of V, source half)
+    __shared__ T sm[SETS * R * WS > 4 * SH ? SETS * R * WS : 4 * SH];  // windows, reused for the sums
+    auto set_of = [](int v, int hp) { return KB ? kb_unit(v, hp) : 2 * v + hp; };
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     // (segment, tile range, multipole, tile [, half]) with tiles fastest, in XCD order: an XCD works through the
@@ -721,7 +783,7 @@ __global__ __launch_bounds__(256) void k_radial_dia(
     const int rng = min(rest / (lgrid * tc), (nt2 - 1) / tc);
     rest -= rng * lgrid * tc;
     const int tn = min(tc, nt2 - rng * tc);
-    const int l = rest / tn;
+    const int lo = rest / tn, l = lo == 0 ? 0 : lgrid - lo;  // the longest first: l = 0 has D, then the longest lists
     const int t2 = rng * tc + rest % tn;
     const int h0 = HV == 2 ? 0 : (t2 & 1);
     const int tile = HV == 2 ? t2 : t2 >> 1;
@@ -736,8 +798,6 @@ __global__ __launch_bounds__(256) void k_radial_dia(
     for (int i = 0; i < R; i++) rows[i] = tiles[tile * R + i];
     const size_t plane = (size_t)nblk * n;
     const int S = 4 * ND * nhp;
-    T *const win = sm + wave * 2 * R * WS;
-
     T acc[HV][R][P];
     auto clear = [&]() {
 #pragma unroll
@@ -748,14 +808,14 @@ __global__ __launch_bounds__(256) void k_radial_dia(
                 for (int j = 0; j < P; j++) acc[hh][i][j] = czero<T>();
     };
 
-    // This wave's windows of half hs of 'src' for every row of the tile into window set ws: position p <-> half index
+    // This wave's windows of half hs of 'src' for every row of the tile into the window set win: position p <-> half index
     // i0 - BW + p, clamped into the half (the coefficients are zero where a position lies outside it); padding rows
     // read row 0 of the vector and are never stored.  The loads of RB rows are in flight together.
     constexpr int NC = (W + 63) / 64;
     unsigned bc[NC];
 #pragma unroll
     for (int c = 0; c < NC; c++) bc[c] = min(max(i0 - BW + c * 64 + lane, 0), nh - 1);
-    auto stage = [&](const T *src, int hs, int ws) {
+    auto stage = [&](const T *src, int hs, T *win) {
         constexpr int RB = R < 8 ? R : (P == 1 ? 8 : 4);
         wave_lds_sync();
 #pragma unroll
@@ -776,26 +836,30 @@ __global__ __launch_bounds__(256) void k_radial_dia(
 #pragma unroll
                 for (int c = 0; c < NC; c++) {
                     const int p = c * 64 + lane;
-                    if (p < W) win[(ws * R + i1 + i) * WS + dia_slot<P>(p)] = cx<T>::mk(tr[i][c], ti[i][c]);
+                    if (p < W) win[(i1 + i) * WS + dia_slot<P>(p)] = cx<T>::mk(tr[i][c], ti[i][c]);
                 }
         }
         wave_lds_sync();
     };
     // FUSED: the windows of V_{l,v} (v = 0..3) for both halves of every row into the waves' window sets, each entry the
     // sums Z0 = sum_e h0_e x_{c_e}, Z2 = sum_e h0_e k_{c_e} x_{c_e}, W0, W1 likewise with h1, over the row's list (l) in
-    // list order from +0, as k_angular_list forms them.  Wave w takes rows w, w + 4, ...; the two halves' windows are
-    // one run of 2 W positions over the lanes.  The list entries are wave-uniform (scalar loads); each x value is
+    // list order from +0, as k_angular_list forms them.  Wave w takes rows w, w + 4, ...; a lane has P positions of the
+    // first half, P of the second and one of the 2 * BW beyond each half's 64 P.  The list entries are wave-uniform (scalar loads); each x value is
     // loaded once for the four sums.
     auto gather = [&]() {
-        constexpr int NCG = (2 * W + 63) / 64;
+        constexpr int NCG = 2 * P + 1;
+        static_assert(4 * BW <= 64, "the positions beyond both halves' runs fit the lanes");
         constexpr int U = kAngListU;
         const T *xh = x + (size_t)inst * nblk1 * n;
+        int gh[NCG], gp[NCG];  // half and position of the lane's c-th entry
         unsigned gc[NCG];
 #pragma unroll
         for (int c = 0; c < NCG; c++) {
-            const int p = c * 64 + lane, hs = p >= W;
-            gc[c] = (hs ? nh : 0) + min(max(i0 - BW + p - (hs ? W : 0), 0), nh - 1);
+            gh[c] = c < 2 * P ? c / P : lane >= 2 * BW;
+            gp[c] = c < 2 * P ? (c % P) * 64 + lane : 64 * P + lane - (lane >= 2 * BW ? 2 * BW : 0);
+            gc[c] = gh[c] * nh + min(max(i0 - BW + gp[c], 0), nh - 1);
         }
+        auto has = [&](int v, int c) { return !KB || v == 0 || v == 2 || (v == 1 ? c < P || c == 2 * P : c >= P); };
 #pragma unroll
         for (int k = 0; k < RW; k++) {
             const int i = wave + 4 * k;
@@ -822,17 +886,17 @@ __global__ __launch_bounds__(256) void k_radial_dia(
 #pragma unroll
                         for (int c = 0; c < NCG; c++)
                             ang_terms<RC>(xv[u][c], ack[e + u].y, acf + 2 * (e + u), z[0][c], z[1][c], z[2][c],
-                                          z[3][c]);
+                                          z[3][c], has(1, c), has(3, c));
                     }
                 }
             }
 #pragma unroll
             for (int c = 0; c < NCG; c++) {
-                const int p = c * 64 + lane, hs = p >= W;
-                if (p < 2 * W) {
+                if (c < 2 * P || lane < 4 * BW) {
 #pragma unroll
                     for (int v = 0; v < 4; v++)
-                        sm[((v * 2 + hs) * R + i) * WS + dia_slot<P>(p - (hs ? W : 0))] = z[v][c];
+                        if (!KB || v == 0 || v == 2 || gh[c] == (v == 1 ? 0 : 1))
+                            sm[(set_of(v, gh[c]) * R + i) * WS + dia_slot<P>(gp[c])] = z[v][c];
                 }
             }
         }
@@ -841,8 +905,7 @@ __global__ __launch_bounds__(256) void k_radial_dia(
     // acc[hh][i][j] += sum_d M^{hh}_d[i0 + P*lane + j] * win[i][P*lane + j + d] for NH output halves whose
     // coefficients start hstep apart; with pairs M = C1 + kap*C2, else M = C1.  Coefficients are fetched PF - 1
     // diagonals ahead.
-    auto sweep = [&](auto nh_tag, int ws, const T *C, size_t hstep, auto pair_tag) {
-        const T *const wn = win + ws * R * WS;
+    auto sweep = [&](auto nh_tag, const T *wn, const T *C, size_t hstep, auto pair_tag) {
         constexpr int NH = decltype(nh_tag)::value;
         constexpr bool PAIR = decltype(pair_tag)::value;
         constexpr int PF = P >= 4 ? 2 : P == 2 ? 3 : (NH * R <= 16 ? 4 : 3);
@@ -900,19 +963,69 @@ __global__ __launch_bounds__(256) void k_radial_dia(
             }
         }
     };
-    // the waves' sums of NH halves side by side in LDS (each in its own window sets)
-    auto share = [&](auto nh_tag) {
+    // the same for the G products of a unit of the zero pattern: with NH = 2 the half with pairs (acc[1]) and the one
+    // without (acc[0]) of a unit, with NH = 1 the half that PAIR says; C is the unit's coefficients
+    auto sweep_kb = [&](auto nh_tag, const T *wn, const T *C, auto pair_tag) {
+        constexpr int NH = decltype(nh_tag)::value;
+        constexpr bool SINGLE = NH == 2 || !decltype(pair_tag)::value, PAIR = NH == 2 || decltype(pair_tag)::value;
+        constexpr int PF = P >= 4 ? 2 : P == 2 ? 3 : (NH * R <= 16 ? 4 : 3);
+        const unsigned lo = P * lane;
+        T w[R][P];
+#pragma unroll
+        for (int i = 0; i < R; i++)
+#pragma unroll
+            for (int j = 0; j < P; j++) w[i][j] = wn[i * WS + (j % P) * dia_wp<P>() + j / P + lane];
+        T cp[PF][P];
+        Rt cs[PF][P];
+        const Rt *const C1 = reinterpret_cast<const Rt *>(C + (size_t)ND * nhp);
+        auto fetch = [&](int d) {
+#pragma unroll
+            for (int j = 0; j < P; j++) {
+                if constexpr (PAIR) cp[d % PF][j] = ld_off(C + (size_t)d * nhp + i0, lo + j);
+                if constexpr (SINGLE) cs[d % PF][j] = ld_off(C1 + (size_t)d * nhp + i0, lo + j);
+            }
+        };
+#pragma unroll
+        for (int d = 0; d < PF - 1; d++) fetch(d);
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            if (d + PF - 1 < ND) fetch(d + PF - 1);
+            Rt M[NH][P];
+#pragma unroll
+            for (int j = 0; j < P; j++) {
+                if constexpr (SINGLE) M[0][j] = cs[d % PF][j];
+                if constexpr (PAIR) M[NH - 1][j] = fma(kap, cp[d % PF][j].y, cp[d % PF][j].x);
+            }
+#pragma unroll
+            for (int i = 0; i < R; i++) {
+#pragma unroll
+                for (int a = 0; a < NH; a++)
+#pragma unroll
+                    for (int j = 0; j < P; j++) acc[a][i][j] = rfma(M[a][j], w[i][j], acc[a][i][j]);
+                if (d + 1 < ND) {
+#pragma unroll
+                    for (int j = 0; j + 1 < P; j++) w[i][j] = w[i][j + 1];
+                    w[i][P - 1] = wn[i * WS + ((P + d) % P) * dia_wp<P>() + (P + d) / P + lane];
+                }
+            }
+        }
+    };
+    // the waves' sums of NH halves side by side in LDS; flip: acc[0] is the second half's
+    auto share = [&](auto nh_tag, int flip) {
+        constexpr int NH = decltype(nh_tag)::value;
+        T *const mine = sm + wave * SH;
         __syncthreads();
 #pragma unroll
-        for (int hh = 0; hh < decltype(nh_tag)::value; hh++)
+        for (int hh = 0; hh < NH; hh++)
 #pragma unroll
             for (int i = 0; i < R; i++)
 #pragma unroll
-                for (int j = 0; j < P; j++) win[((hh * R + i) * P + j) * 64 + lane] = acc[hh][i][j];
+                for (int j = 0; j < P; j++)
+                    mine[((((NH == 2 ? hh ^ flip : hh) * R) + i) * P + j) * 64 + lane] = acc[hh][i][j];
         __syncthreads();
     };
     auto shared_of = [&](int w, int hh, int i, int j) {
-        return sm[w * 2 * R * WS + ((hh * R + i) * P + j) * 64 + lane];
+        return sm[w * SH + ((hh * R + i) * P + j) * 64 + lane];
     };
     // output (or multipole partial) of this wave's row k, output j, half hh
     auto emit = [&](T *YO, T *YPO, int k, int j, int hh, T r) {
@@ -937,18 +1050,30 @@ __global__ __launch_bounds__(256) void k_radial_dia(
             for (int j = 0; j < P; j++) g[hh][k][j] = czero<T>();
     if (cH != 0.0) {
         clear();
+        constexpr std::integral_constant<int, HV> halves{};
+        const int hp0 = KB ? wave == 3 : 0, hp1 = KB ? wave != 1 : 1;  // source halves of this wave's part of V
         if constexpr (FUSED) {
             gather();
         } else {
-            stage(V + (size_t)(l * 4 + wave) * plane, 0, 0);
-            stage(V + (size_t)(l * 4 + wave) * plane, 1, 1);
+            for (int hp = hp0; hp <= hp1; hp++)
+                stage(V + (size_t)(l * 4 + wave) * plane, hp, sm + set_of(wave, hp) * R * WS);
         }
 #pragma unroll 1
-        for (int hp = 0; hp < 2; hp++)
-            sweep(std::integral_constant<int, HV>{}, hp,
-                  GD + ((size_t)(l * 4 + wave) * S + (size_t)(2 * h0 + hp) * ND * nhp) * (RC ? 1 : 2),
-                  (size_t)2 * ND * nhp * (RC ? 1 : 2), std::true_type{});
-        share(std::integral_constant<int, HV>{});
+        for (int hp = hp0; hp <= hp1; hp++) {
+            const T *const wn = sm + set_of(wave, hp) * R * WS;
+            if constexpr (KB) {
+                const T *const C = GD + (size_t)(l * 6 + set_of(wave, hp)) * kb_words(ND, nhp);
+                if (HV == 2 || (h0 == 1) == (wave < 2))
+                    sweep_kb(halves, wn, C, std::true_type{});
+                else
+                    sweep_kb(halves, wn, C, std::false_type{});
+            } else {
+                sweep(halves, wn,
+                      GD + ((size_t)(l * 4 + wave) * S + (size_t)(2 * h0 + hp) * ND * nhp) * (RC ? 1 : 2),
+                      (size_t)2 * ND * nhp * (RC ? 1 : 2), std::true_type{});
+            }
+        }
+        share(halves, KB && wave >= 2);
 #pragma unroll
         for (int hh = 0; hh < HV; hh++)
 #pragma unroll
@@ -981,14 +1106,15 @@ __global__ __launch_bounds__(256) void k_radial_dia(
     __syncthreads();  // the reads of the shared sums are done
     clear();
     if (DUAL || HV == 2 || part == 0) {
-        stage(x, hpD, 0);
+        T *const win = sm + wave * R * WS;
+        stage(x, hpD, win);
         const int hD = DUAL || HV == 1 ? h0 : part;
         const int sD = DUAL && part == 1 ? sel2 : sel;
-        sweep(std::integral_constant<int, NHD>{}, 0,
+        sweep(std::integral_constant<int, NHD>{}, win,
               DD + ((size_t)(sD * nq + q) * S + (size_t)(2 * hD + hpD) * ND * nhp), (size_t)2 * ND * nhp,
               std::false_type{});
     }
-    share(std::integral_constant<int, NHD>{});
+    share(std::integral_constant<int, NHD>{}, 0);
 #pragma unroll
     for (int hh = 0; hh < HV; hh++) {
         const int w0 = DUAL ? 0 : 2 * hh, hs = DUAL ? hh : 0;  // waves (two source halves) and set that hold D
@@ -1547,18 +1673,23 @@ int launch_dia(gade_model *m, int lgrid, const T *x, const T *V, const T *GD, co
         gade::set_error("the fused angular + radial form needs at most 2 outputs per lane");
         return GADE_EINVAL;
     }
-#define GADE_DIA1(R_, P_, HV_, F_, RC_, CF_)                                                                     \
-    hipLaunchKernelGGL((k_radial_dia<kDiaBW, DUAL, T, R_, P_, HV_, F_, RC_>), grid, dim3(256), 0, m->stream, x, V, \
+#define GADE_DIA1(R_, P_, HV_, F_, RC_, KB_, CF_)                                                                   \
+    hipLaunchKernelGGL((k_radial_dia<kDiaBW, DUAL, T, R_, P_, HV_, F_, RC_, KB_>), grid, dim3(256), 0, m->stream, x, V, \
                        GD, DD, m->d_dtiles, m->d_dtile_q, m->d_dtile_k, m->nblk, m->n, m->nh, m->nhp, nseg, lgrid, \
                        m->nq, sel, cH, beta, y, yp, m->gate, m->gstride, m->d_dtile_b, m->gd_stride, y2, yp2, sel2, \
                        m->d_aoff, (const int2 *)m->d_ack, CF_, m->lmax, m->nblk1, m->h_rot)
 #define GADE_DIA(R_, P_, F_)                         \
     if (!m->gd_real) {                               \
-        GADE_DIA1(R_, P_, 2, false, false, nullptr); \
+        GADE_DIA1(R_, P_, 2, false, false, false, nullptr); \
+    } else if (m->g_kb) {                            \
+        if (hv == 2)                                 \
+            GADE_DIA1(R_, P_, 2, F_, true, true, acr);  \
+        else                                         \
+            GADE_DIA1(R_, P_, 1, F_, true, true, acr);  \
     } else if (hv == 2) {                            \
-        GADE_DIA1(R_, P_, 2, F_, true, acr);         \
+        GADE_DIA1(R_, P_, 2, F_, true, false, acr);  \
     } else {                                         \
-        GADE_DIA1(R_, P_, 1, F_, true, acr);         \
+        GADE_DIA1(R_, P_, 1, F_, true, false, acr);  \
     }
 #define GADE_DIAF(R_, P_)           \
     if (fused) {                    \
@@ -1688,6 +1819,23 @@ int kappa_tiles(const gade_model *m, int R, int **d_tiles, int **d_tq, double **
 }
 
 int build_tiles(gade_model *m) { return kappa_tiles(m, m->tile_r, &m->d_tiles, &m->d_tile_q, &m->d_tile_k, &m->ntiles); }
+
+// whether the radial couplings g[alpha*4*lmax + l*4 + n] are real and zero outside the quadrants of kb_unit's pattern
+bool kb_pattern(const gade_model *m, const double *const *g) {
+    if (!m->g_real || m->n % 2) return false;
+    const int nh = m->n / 2;
+    for (int i = 0; i < 24 * m->lmax; i++) {
+        const int n = i % 4;
+        if (n == 0) continue;
+        for (int a = 0; a < m->n; a++)
+            for (int k = m->rad_Ap[a]; k < m->rad_Ap[a + 1]; k++) {
+                const int h = a / nh, hp = m->rad_Ai[k] / nh;
+                const bool filled = (n == 2 || h == 1) && (n == 1 || hp == 0);
+                if (!filled && g[i][2 * k] != 0.0) return false;
+            }
+    }
+    return true;
+}
 
 // Banded form of the radial pattern: n even, every entry (h*nh+i, h'*nh+j)
 // with |i-j| <= kDiaBW.  Builds the DIA maps and the static DIA operators.
@@ -1843,7 +1991,10 @@ void set_form(gade_model *m, bool real) {
 }
 
 void run_gsums_dia(gade_model *m, dim3 grid, const CoefGroup &cg, int b0, const Coef6 *table, const int *gctl) {
-    if (m->gd_real)
+    if (m->gd_real && m->g_kb)
+        hipLaunchKernelGGL(k_gsums_kb, grid, dim3(256), 0, m->stream, m->d_gsr, m->d_gtsr, cg, b0, m->gd_stride, m->lmax,
+                           m->nd, m->nhp, m->d_GD, m->gate, m->gstride, table, gctl, m->B);
+    else if (m->gd_real)
         hipLaunchKernelGGL((k_gsums_dia<true, double>), grid, dim3(256), 0, m->stream, m->d_gsr, m->d_gtsr, cg, b0,
                            m->gd_stride, m->lmax, m->nd, m->nhp, m->d_GD, m->gate, m->gstride, table, gctl, m->B);
     else
@@ -2093,6 +2244,7 @@ int gade_model_create_batch(const gade_inputs_t *in, int B, double h, double dt,
     m->g_real = true;
     for (int i = 0; i < 24 * lmax && m->g_real; i++)
         for (int k = 0; k < m->nnzb && m->g_real; k++) m->g_real = in->g[i][2 * k + 1] == 0.0;
+    m->g_kb = kb_pattern(m, in->g);
     if (ack.empty()) {  // no coupling: one unread entry keeps the uploads non-empty
         ack.push_back(make_int2(0, 0));
         acf.assign(4, 0.0);
@@ -2786,7 +2938,10 @@ int enqueue_sweeps(gade_model *m, double2 *psi, int J) {
 
 // the FP32 G-sums of the step (after the FP64 ones), per instance under the step-prologue gate
 int mp_convert_gsums(gade_model *m) {
-    const long long n = (long long)m->gd_stride / (m->gd_real ? 2 : 1);  // words of an instance in use
+    // words of an instance in use
+    const long long n = !m->gd_real ? (long long)m->gd_stride
+                        : m->g_kb   ? (long long)(m->lmax * 6 * kb_words(m->nd, m->nhp))
+                                    : (long long)m->gd_stride / 2;
     hipLaunchKernelGGL(k_to_f32, dim3(grid_for(n, 256, 4096), m->B), dim3(256), 0, m->stream, n, m->gd_stride,
                        (const double2 *)m->d_GD, m->d_GD32, m->gate, m->gstride);
     GADE_HIP(hipGetLastError());

@@ -117,6 +117,7 @@ struct gade_model {
     // is real, 0 otherwise; the lists without that factor, (h0, h1), (h0 k, h1 k) per entry; g_real: every radial coupling is real
     int h_rot = 0;
     bool g_real = false;
+    bool g_kb = false;             // real, and with the zero quadrants of a dual-kinetic-balance basis
     double2 *d_acr = nullptr;
     float2 *d_acr32 = nullptr;
     bool gd_real = false;          // form of the current G-sums d_GD, and so of the banded products
@@ -134,7 +135,8 @@ struct gade_model {
     int nh = 0, nhp = 0, nd = 0, ndtiles = 0;
     int *d_dia_src = nullptr;      // [4][nd][nhp] radial CSR index or -1
     double2 *d_gs = nullptr, *d_gts = nullptr;  // [lmax][3][4][4][nd][nhp] DIA-ordered couplings
-    double2 *d_GD = nullptr;       // [B][lmax][4][4][nd][nhp][2] kappa-folded G-sum pairs (gd_real: one word (G, G'))
+    double2 *d_GD = nullptr;       // [B][lmax][4][4][nd][nhp][2] kappa-folded G-sum pairs (gd_real: one word (G, G'); with g_kb
+                                   // [B][lmax][6] units of kb_words words)
     double2 *d_DD = nullptr;       // [3][nq][4][nd][nhp] diagonal operators
     int *d_dtiles = nullptr, *d_dtile_q = nullptr;
     double *d_dtile_k = nullptr;
