@@ -115,7 +115,7 @@ def kernel_models(gp):
 
 # device kernels behind each timed family (the names rocprofv3 reports)
 KERNEL_NAMES = {"radial": "k_radial_dia<7, false, double2>", "radial_pair": "k_radial_dia<7, true, double2>",
-                "angular": "k_angular<4, double2>", "psolve": "k_psolve_tw<4, double2>", "gsums": "k_gsums_dia",
+                "angular": "k_angular<4, double2>", "psolve": "k_psolve_tw<2, double2, 2, 1>", "gsums": "k_gsums_kb",
                 "blas1": "k_bicg", "csr_spmv": "k_csr_spmv"}
 
 
@@ -563,11 +563,10 @@ def main():
     else:
         fused = gp.get_param("ang_fused")
         rp = f"{gp.get_param('dia_rows')}, {gp.get_param('dia_outputs')}"
-        KERNEL_NAMES["radial"] = (f"k_radial_dia<7, false, double2, {rp}, {gp.get_param('dia_halves')}, "
-                                  f"{'true' if fused else 'false'}>")
-        # the paired two-kernel form always runs one wave per output half
-        KERNEL_NAMES["radial_pair"] = (f"k_radial_dia<7, true, double2, {rp}, "
-                                       f"{gp.get_param('dia_halves') if fused else 1}, {'true' if fused else 'false'}>")
+        # the generated couplings run the real form with the zero quadrants left out (the last two flags)
+        form = f"{rp}, {gp.get_param('dia_halves')}, {'true' if fused else 'false'}, true, true>"
+        KERNEL_NAMES["radial"] = f"k_radial_dia<7, false, double2, {form}"
+        KERNEL_NAMES["radial_pair"] = f"k_radial_dia<7, true, double2, {form}"
     ang = "k_angular_list" if gp.get_param("ang_list") else "k_angular"
     KERNEL_NAMES["angular"] = f"{ang}<{gp.get_param('ang_lb')}, double2>"
 
