@@ -93,10 +93,13 @@ def kernel_models(gp):
             vals = np.asarray(D[perm[rows], perm[Hall["Ai"]]]).ravel()
             ang_nnz += int(np.count_nonzero(vals))
     nnz_full = gp.hall_nnz * nnzb
-    radial = 8.0 * nb * nnzb * (4 * L + 1)
-    angular = 8.0 * 2 * ang_nnz * n
-    # the fused form does the angular contraction inside the radial kernel
-    fused = gp.get_param("ang_fused") and gp.get_param("radial") == 2 and not gp.get_param("radial_mfma")
+    # the banded kernel runs the generated couplings on real coefficients (4 flops a product instead of 8) and leaves
+    # out a quarter of the G products, zero in their basis; the stationary operator is complex
+    real = gp.get_param("radial") == 2 and not gp.get_param("radial_mfma")
+    radial = nb * nnzb * ((12.0 if real else 32.0) * L + 8.0)
+    # the fused form does the angular contraction inside the radial kernel, without the vanishing products' windows
+    fused = gp.get_param("ang_fused") and real
+    angular = (6.0 if fused else 8.0 if real else 16.0) * ang_nnz * n
     return {
         # fused radial SpMM: per block, 4 kappa-folded radial products per l + the diagonal operator (and the
         # angular contraction with ang_fused)
@@ -109,7 +112,7 @@ def kernel_models(gp):
         "blas1": dict(bound="hbm", bytes=4.0 * N * 16.0),
         # per-multipole partial outputs summed in a fixed order
         "radial_sum": dict(bound="hbm", bytes=(L + 1) * N * 16.0 + N * 16.0),
-        "gsums": dict(bound="hbm", bytes=8.0 * L * nnzb * 16.0 + 12.0 * L * nnzb * 16.0),
+        "gsums": dict(bound="hbm", bytes=L * nnzb * (144.0 if real else 320.0)),
     }
 
 
