@@ -1957,12 +1957,10 @@ int setup_mfma(gade_model *m) {
     return GADE_OK;
 }
 
-// G-sums of the current f(t) in the layout of the active radial kernel
-// pulse coefficients c_alpha = SoL * (i h dt/2) * f_alpha of instance b
-Coef6 coef_of(const gade_model *m, int b) {
+// pulse coefficients c_alpha = SoL * (i h dt/2) * f_alpha of an instance
+Coef6 coef_of(const gade_model *m, const double *ft) {
     Coef6 cf;
     const double hd = kSoL * m->h * m->dt / 2;
-    const double *ft = m->ft.data() + (size_t)12 * b;
     for (int a = 0; a < 6; a++) cf.c[a] = make_double2(-hd * ft[2 * a + 1], hd * ft[2 * a]);
     return cf;
 }
@@ -1976,14 +1974,17 @@ bool dia_gsums_needed(const gade_model *m) { return !m->radial_mfma || m->precis
 // f(t)).  It holds half the coefficient bytes and half the products of the complex form, which runs otherwise; the
 // results are the same.  The Hall-row angular kernel and the matrix-core kernel have the complex form only.
 // ft: [..][12] pulse coefficients of every instance (and step) concerned
-bool real_form(const gade_model *m, const std::vector<double> &ft) {
-    if (!m->g_real || !m->h_rot || !m->ang_list || m->radial_mfma) return false;
-    for (size_t i = 1; i < ft.size(); i += 2)
+bool real_ft(const double *ft, size_t len) {
+    for (size_t i = 1; i < len; i += 2)
         if (ft[i] != 0.0) return false;
     return true;
 }
+bool real_form(const gade_model *m, const std::vector<double> &ft) {
+    return m->g_real && m->h_rot && m->ang_list && !m->radial_mfma && real_ft(ft.data(), ft.size());
+}
 
-// the banded G-sums that follow are written, and every product until the next ones runs, in this form
+// The banded G-sums that follow are written, and every product until the next ones runs, in this form: one for all
+// instances, so whoever changes it writes every instance's sums again (dia_gsums) unless they are about to be.
 void set_form(gade_model *m, bool real) {
     if (m->gd_real == real) return;
     drop_step_graph(m);  // its launches are of the other form
@@ -2002,31 +2003,49 @@ void run_gsums_dia(gade_model *m, dim3 grid, const CoefGroup &cg, int b0, const 
                            m->gd_stride, m->lmax, m->nd, m->nhp, m->d_GD, m->gate, m->gstride, table, gctl, m->B);
 }
 
+// banded G-sums of f(t) = ft [B][12] for every instance (no gate), in the current form
+int dia_gsums(gade_model *m, const std::vector<double> &ft) {
+    long long total = (long long)m->lmax * 16 * m->nd * m->nhp;  // (l, v, qd, d, ip)
+    const long long totf = (long long)m->lmax * 16 * m->nmi * 5 * kMfmaFrag;
+    for (int b0 = 0; b0 < m->B; b0 += kCoefGroup) {
+        const int nb = std::min(kCoefGroup, m->B - b0);
+        CoefGroup cg{};
+        for (int k = 0; k < nb; k++) cg.c[k] = coef_of(m, ft.data() + (size_t)12 * (b0 + k));
+        if (dia_gsums_needed(m))
+            run_gsums_dia(m, dim3(grid_for(total, 256, 4096), nb), cg, b0, nullptr, nullptr);
+        if (m->radial_mfma)
+            hipLaunchKernelGGL(k_gsums_frag, dim3(grid_for(totf, 256, 4096), nb), dim3(256), 0, m->stream,
+                               m->d_gs, m->d_gts, cg, b0, m->gf_stride, m->lmax, m->nd, m->nhp, m->nmi, m->d_GF,
+                               m->gate, m->gstride, (const Coef6 *)nullptr, (const int *)nullptr, m->B);
+    }
+    GADE_HIP(hipGetLastError());
+    m->gd_ft = ft;
+    return GADE_OK;
+}
+
 // G-sums of the current f(t) of every instance in the layout of the active radial kernel
 int launch_gsums(gade_model *m, bool ell) {
     Prof pr(m, "gsums", GADE_PROF_GSUMS);
-    if (ell) {
-        long long total = (long long)m->lmax * 8 * m->ellw * m->n;
-        hipLaunchKernelGGL(k_gsums, dim3(grid_for(total, 256)), dim3(256), 0, m->stream, m->d_g, m->d_ell_src,
-                           m->d_tmap, coef_of(m, 0), m->lmax, m->ellw, m->n, m->nnzb, m->d_GE, m->gate);
-    } else {
-        long long total = (long long)m->lmax * 16 * m->nd * m->nhp;  // (l, v, qd, d, ip)
-        const long long totf = (long long)m->lmax * 16 * m->nmi * 5 * kMfmaFrag;
+    if (!ell) {
         set_form(m, real_form(m, m->ft));
-        for (int b0 = 0; b0 < m->B; b0 += kCoefGroup) {
-            const int nb = std::min(kCoefGroup, m->B - b0);
-            CoefGroup cg{};
-            for (int k = 0; k < nb; k++) cg.c[k] = coef_of(m, b0 + k);
-            if (dia_gsums_needed(m))
-                run_gsums_dia(m, dim3(grid_for(total, 256, 4096), nb), cg, b0, nullptr, nullptr);
-            if (m->radial_mfma)
-                hipLaunchKernelGGL(k_gsums_frag, dim3(grid_for(totf, 256, 4096), nb), dim3(256), 0, m->stream,
-                                   m->d_gs, m->d_gts, cg, b0, m->gf_stride, m->lmax, m->nd, m->nhp, m->nmi, m->d_GF,
-                                   m->gate, m->gstride, (const Coef6 *)nullptr, (const int *)nullptr, m->B);
-        }
+        return dia_gsums(m, m->ft);
     }
+    long long total = (long long)m->lmax * 8 * m->ellw * m->n;
+    hipLaunchKernelGGL(k_gsums, dim3(grid_for(total, 256)), dim3(256), 0, m->stream, m->d_g, m->d_ell_src, m->d_tmap,
+                       coef_of(m, m->ft.data()), m->lmax, m->ellw, m->n, m->nnzb, m->d_GE, m->gate);
     GADE_HIP(hipGetLastError());
     return GADE_OK;
+}
+
+// The form of a run's window with f(t) = ft [..][12].  An instance without a step in the run (nsteps_b) keeps the
+// G-sums it has: complex ones keep the whole batch in the complex form, and a change of form writes the kept ones anew.
+int window_form(gade_model *m, const std::vector<double> &ft, const int *nsteps_b) {
+    bool real = real_form(m, ft);
+    for (int b = 0; nsteps_b && b < m->B; b++)
+        if (nsteps_b[b] == 0) real = real && real_ft(m->gd_ft.data() + (size_t)12 * b, 12);
+    if (real == m->gd_real) return GADE_OK;
+    set_form(m, real);
+    return nsteps_b ? dia_gsums(m, m->gd_ft) : GADE_OK;
 }
 
 }  // namespace
@@ -2371,6 +2390,7 @@ int gade_model_create_batch(const gade_inputs_t *in, int B, double h, double dt,
         return fail(GADE_ENOMEM);
     }
     m->ft.assign((size_t)12 * B, 0.0);
+    m->gd_ft = m->ft;
     *out = m;
     return GADE_OK;
 }
@@ -3224,11 +3244,11 @@ int run_steps(gade_model *m, double2 *psi, const double *times, int nsteps, cons
         const bool table = m->radial_kind == 2;
         if (table) {
             GADE_TRY(ensure_cfwin(m, W));
-            set_form(m, real_form(m, ft));
+            GADE_TRY(window_form(m, ft, nsteps_b));
             Coef6 *tab = (Coef6 *)m->h_cfwin;
             for (int w = 0; w < W; w++) {
                 std::copy(ft.data() + (size_t)12 * B * w, ft.data() + (size_t)12 * B * (w + 1), m->ft.begin());
-                for (int b = 0; b < B; b++) tab[(size_t)w * B + b] = coef_of(m, b);
+                for (int b = 0; b < B; b++) tab[(size_t)w * B + b] = coef_of(m, m->ft.data() + (size_t)12 * b);
             }
             GADE_HIP(hipMemcpyAsync(m->d_cfwin, m->h_cfwin, sizeof(Coef6) * (size_t)W * B, hipMemcpyHostToDevice,
                                     m->stream));
@@ -3263,6 +3283,13 @@ int run_steps(gade_model *m, double2 *psi, const double *times, int nsteps, cons
                 gade::set_error("device-driven stepping: inconsistent stall record");
                 return GADE_EHIP;
             }
+        }
+        for (int b = 0; table && b < B; b++) {  // the last step whose G-sums each instance has formed
+            const int last = std::min(stalled ? done : s + W - 1, (nsteps_b ? nsteps_b[b] : nsteps) - 1);
+            if (last >= s)
+                std::copy_n(ft.data() + (size_t)12 * ((size_t)B * (last - s) + b), 12, m->gd_ft.data() + (size_t)12 * b);
+        }
+        if (stalled) {
             GADE_TRY(finish_stalled_step(m, psi, done, K));
             GADE_HIP(hipStreamSynchronize(m->stream));
             done += 1;
@@ -3950,7 +3977,11 @@ int gade_set_param(gade_model_t *m, const char *name, int value) {
         if (m->ang_list != value) {
             drop_step_graph(m);
             m->ang_list = value;
-            if (m->radial_kind == 2) GADE_TRY(launch_gsums(m, false));  // the current f(t) in that form's layout
+            const bool real = real_form(m, m->gd_ft);
+            if (m->radial_kind == 2 && real != m->gd_real) {  // the sums that every instance has, in that form's layout
+                set_form(m, real);
+                GADE_TRY(dia_gsums(m, m->gd_ft));
+            }
         }
         return GADE_OK;
     }

@@ -92,6 +92,7 @@ struct gade_model {
     std::vector<int> rad_Ap, rad_Ai, hall_Ap, hall_Ai, kap_blk, kap_q;  // kap_q: kappa of each distinct index
     std::vector<int> blk_q;   // distinct-kappa index of each block
     std::vector<double> ft;   // last f(t) of every instance, [B][12] doubles
+    std::vector<double> gd_ft;  // the f(t) that each instance's banded G-sums hold (a batch's instances stop on their own)
 
     // radial pattern (ELL, transposed: [slot][row])
     int *d_ell_col = nullptr, *d_ell_src = nullptr, *d_tmap = nullptr, *d_ell_pos = nullptr;
