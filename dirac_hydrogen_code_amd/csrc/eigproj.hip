@@ -220,7 +220,9 @@ int gade_populations(gade_model_t *m, const double *x, double *norm, double *bou
     if (!m || !x) return GADE_EINVAL;
     GADE_TRY(gade_eig_setup(m));
     const double csq = gade::kSoL * gade::kSoL;
-    // the sums go straight to pinned host memory: four numbers per workgroup, read once the stream is done
+    // the sums go straight to pinned host memory: four numbers per workgroup, read once the stream is done; calls of
+    // several threads take turns, as they did on the stream
+    std::lock_guard<std::mutex> one(m->eig_mutex);
     const int ny = eig_split(m->nblk, m->n);
     hipLaunchKernelGGL(k_eigproj<false>, dim3(m->nblk, ny), dim3(kEigThreads), sizeof(double2) * m->n, m->stream,
                        (const double2 *)x, m->d_D, m->d_ell_col, m->d_blk_q, m->d_evec, m->d_eval, m->n, m->ellw,

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -189,6 +190,7 @@ struct gade_model {
     double *d_evec = nullptr;
     double *d_eval = nullptr;
     double *h_eig = nullptr;       // pinned: the populations of every block, per workgroup
+    std::mutex eig_mutex;          // h_eig serves one gade_populations call at a time
     // device-driven CN stepping: control words, per-step outputs, launch gate
     int *d_ctl = nullptr;          // [B][CT_STRIDE] per-instance words
     int *h_ctl = nullptr;          // pinned mirror
