@@ -2311,6 +2311,7 @@ int gade_model_create_batch(const gade_inputs_t *in, int B, double h, double dt,
         (rc = upload(&m->d_nloc, nloc.data(), nloc.size())) ||
         (rc = upload(&m->d_ell_src, ell_src.data(), ell_src.size())) ||
         (rc = upload(&m->d_ell_pos, ell_pos.data(), ell_pos.size())) ||
+        (rc = upload(&m->d_subAp, m->rad_Ap.data(), m->rad_Ap.size())) ||
         (rc = upload(&m->d_tmap, tmap.data(), tmap.size())) ||
         (rc = upload(&m->d_g, (const double2 *)gbuf.data(), gbuf.size() / 2)) ||
         (rc = upload(&m->d_s, (const double2 *)sbuf.data(), sbuf.size() / 2)) ||
@@ -3857,7 +3858,6 @@ int gade_assembled_setup(gade_model_t *m) {
 int gade_assembled_timedep_into(gade_model_t *m, const int *Ap_dev, double *Ax_dev) {
     if (!m || !Ap_dev || !Ax_dev) return GADE_EINVAL;
     if (m->radial_kind == 2) GADE_TRY(launch_gsums(m, true));  // the fused path keeps only the DIA layout
-    if (!m->d_subAp) GADE_TRY(upload(&m->d_subAp, m->rad_Ap.data(), m->rad_Ap.size()));
     // several workgroups per compute unit, each staging its radial rows' G-sums for many block rows
     const int na = (m->n + 1) / 2;
     const dim3 grid((unsigned)na, (unsigned)std::max(1, std::min(m->nblk, (4096 + na - 1) / na)));
