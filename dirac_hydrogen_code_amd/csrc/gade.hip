@@ -3121,15 +3121,15 @@ int ensure_cfwin(gade_model *m, int slots) {
     return GADE_OK;
 }
 
-// The run stalled at 'step': finish it for every instance from the device state.
-int finish_stalled_step(gade_model *m, double2 *psi, int step, int K) {
+// The run stalled at 'step': finish it for every instance that takes it (nsteps_b) from the device state.
+int finish_stalled_step(gade_model *m, double2 *psi, int step, int K, const int *nsteps_b) {
     const int B = m->B;
     for (int round = 0;; round++) {
         GADE_HIP(hipMemcpyAsync(m->h_ctl, m->d_ctl, sizeof(int) * B * CT_STRIDE, hipMemcpyDeviceToHost, m->stream));
         GADE_HIP(hipMemcpyAsync(m->h_sc, m->d_sc, sizeof(double) * B * SC_STRIDE, hipMemcpyDeviceToHost, m->stream));
         GADE_HIP(hipStreamSynchronize(m->stream));
-        // instances idle at this step (pulse over) keep PSKIP set by k_step_begin; k_stall_spread set it for
-        // the others, so activity is read from the step's status instead
+        // k_stall_spread has set PSKIP for every instance, so activity is read from the step's status, which an
+        // instance that is idle at this step (pulse over, or no step in the run) does not have: it stays skipped
         bool more = false, restart = false;
         for (int b = 0; b < B; b++) {
             int *c = m->h_ctl + (size_t)b * CT_STRIDE;
@@ -3137,6 +3137,8 @@ int finish_stalled_step(gade_model *m, double2 *psi, int step, int K) {
             const int st = c[CT_STATUS];
             c[CT_HSEL] = 1;
             c[CT_PSKIP] = 1;
+            c[CT_SKIP] = 1;
+            if (nsteps_b && step >= nsteps_b[b]) continue;
             if (st == 2) {
                 if (sc[SC_RHSSQ] == 0) {
                     // zero rhs: x = 0 (tools/gpu_bicgstab.c:183-189)
@@ -3291,7 +3293,7 @@ int run_steps(gade_model *m, double2 *psi, const double *times, int nsteps, cons
                 std::copy_n(ft.data() + (size_t)12 * ((size_t)B * (last - s) + b), 12, m->gd_ft.data() + (size_t)12 * b);
         }
         if (stalled) {
-            GADE_TRY(finish_stalled_step(m, psi, done, K));
+            GADE_TRY(finish_stalled_step(m, psi, done, K, nsteps_b));
             GADE_HIP(hipStreamSynchronize(m->stream));
             done += 1;
         }
