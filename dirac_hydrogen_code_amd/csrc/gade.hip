@@ -2601,6 +2601,7 @@ int applyA(gade_model *m, const double2 *x, double2 *out, int *napply) {
 
 // Host-driven BiCGSTAB iterations from iteration i, with r, r0, p, v, x and the
 // scalars as they stand on the device (tools/gpu_bicgstab.c:133-307).
+// One kernel per operation: what the device-driven body (bicg_body) merges is checked against it, bit for bit.
 int bicg_host_loop(gade_model *m, const double2 *rhs, double2 *x, int i, double tol, int maxit, int *iters,
                    double *tol_error, int *napply) {
     GADE_TRY(read_scalars(m));
@@ -2621,20 +2622,15 @@ int bicg_host_loop(gade_model *m, const double2 *rhs, double2 *x, int i, double 
             GADE_TRY(read_scalars(m));
             r0_sq = m->h_sc[SC_R0SQ];
         }
-        if (fused_sums(m)) {
-            GADE_TRY(bicg_body(m, x));
-            if (napply) *napply += 2;
-        } else {
-            GADE_TRY(bicg_op<OP_P>(m, rhs));              // p = r + beta (p - w v)
-            GADE_TRY(psolve_async(m, m->p, m->y));        // y = M^-1 p
-            GADE_TRY(applyA(m, m->y, m->v, napply));      // v = A y
-            GADE_TRY(bicg_op<OP_ALPHA>(m, rhs));          // alpha = rho / (r0 . v)
-            GADE_TRY(bicg_op<OP_S>(m, rhs));              // s = r - alpha v
-            GADE_TRY(psolve_async(m, m->s, m->z));        // z = M^-1 s
-            GADE_TRY(applyA(m, m->z, m->t, napply));      // t = A z
-            GADE_TRY(bicg_op<OP_W>(m, rhs));              // w = (t . s) / |t|^2
-            GADE_TRY(bicg_op<OP_XR>(m, rhs, x));          // x += alpha y + w z ; r = s - w t
-        }
+        GADE_TRY(bicg_op<OP_P>(m, rhs));                 // p = r + beta (p - w v)
+        GADE_TRY(psolve_async(m, m->p, m->y));           // y = M^-1 p
+        GADE_TRY(applyA(m, m->y, m->v, napply));         // v = A y
+        GADE_TRY(bicg_op<OP_ALPHA>(m, rhs));             // alpha = rho / (r0 . v)
+        GADE_TRY(bicg_op<OP_S>(m, rhs));                 // s = r - alpha v
+        GADE_TRY(psolve_async(m, m->s, m->z));           // z = M^-1 s
+        GADE_TRY(applyA(m, m->z, m->t, napply));         // t = A z
+        GADE_TRY(bicg_op<OP_W>(m, rhs));                 // w = (t . s) / |t|^2
+        GADE_TRY(bicg_op<OP_XR>(m, rhs, x));             // x += alpha y + w z ; r = s - w t
         GADE_TRY(read_scalars(m));
         rnorm2 = m->h_sc[SC_RNORM2];
         rho_next_abs = std::hypot(m->h_sc[SC_RHONEXT], m->h_sc[SC_RHONEXT + 1]);

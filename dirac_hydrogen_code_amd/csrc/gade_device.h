@@ -1081,7 +1081,7 @@ __global__ __launch_bounds__(128) void k_psolve_tw(const T *__restrict__ b, T *_
         if (u < nf) ld4(fwd_level(u), 0, ff[u]);
     double2 alpha[NR];  // PRE_S
     if constexpr (PRE == PRE_S) {
-        __shared__ double red[2][2];
+        __shared__ double red[kRedThreads / 64][2];
 #pragma unroll
         for (int j = 0; j < NR; j++) {
             alpha[j] = make_double2(0, 0);
@@ -1091,23 +1091,39 @@ __global__ __launch_bounds__(128) void k_psolve_tw(const T *__restrict__ b, T *_
                 alpha[j] = alpha[j - 1];
                 continue;
             }
+            // summed in k_bicg_fin's order, each wave in the place of two of its kRedThreads / 64: alpha is the same
+            // number bit for bit (a wave without partials has the sum 0)
             const double *fp = kv.fold + (size_t)inst * kv.nparts * 4;
-            double t0 = 0, t1 = 0;
-            for (int u = threadIdx.x; u < kv.nparts; u += 128) {
-                t0 += fp[(size_t)u * 4];
-                t1 += fp[(size_t)u * 4 + 1];
+            constexpr int H = kRedThreads / 128;
+            double t0[H], t1[H];
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                t0[h] = t1[h] = 0;
+                for (int u = threadIdx.x + 128 * h; u < kv.nparts; u += kRedThreads) {
+                    t0[h] += fp[(size_t)u * 4];
+                    t1[h] += fp[(size_t)u * 4 + 1];
+                }
             }
-            t0 = wave_sum(t0);
-            t1 = wave_sum(t1);
+#pragma unroll
+            for (int h = 0; h < H; h++)
+                if (128 * h + 64 * wave < kv.nparts) {
+                    t0[h] = wave_sum(t0[h]);
+                    t1[h] = wave_sum(t1[h]);
+                }
             __syncthreads();
             if (lane == 0) {
-                red[wave][0] = t0;
-                red[wave][1] = t1;
+#pragma unroll
+                for (int h = 0; h < H; h++) {
+                    red[wave + 2 * h][0] = t0[h];
+                    red[wave + 2 * h][1] = t1[h];
+                }
             }
             __syncthreads();
+            double2 dot = make_double2(0, 0);
+#pragma unroll
+            for (int u = 0; u < kRedThreads / 64; u++) dot = cadd(dot, make_double2(red[u][0], red[u][1]));
             const double *sc = kv.sc + (size_t)inst * SC_STRIDE;
-            alpha[j] = cdiv(make_double2(sc[SC_RHONEXT], sc[SC_RHONEXT + 1]),
-                            make_double2(red[0][0] + red[1][0], red[0][1] + red[1][1]));
+            alpha[j] = cdiv(make_double2(sc[SC_RHONEXT], sc[SC_RHONEXT + 1]), dot);
         }
 #pragma unroll
         for (int j = 0; j < NR; j++)
