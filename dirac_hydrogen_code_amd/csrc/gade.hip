@@ -748,12 +748,15 @@ __global__ void k_build_DD(const double2 *__restrict__ D, const int *__restrict_
 // four and half the coefficient bytes; the factor i (rot 2) or i*i (rot 1) is applied to the finished sum G.  The
 // terms left out are products with zero, so the results equal the complex form's bit for bit.  At 400 x 510 and 4 rows
 // the complex form takes 93 us where the real one takes 58 (both without FUSED), 16 and 11 us at 40 x 110.
+// Complex form, a product call at 400 x 510 with 4 rows and both halves: 147 us with the angular kernel before it, 115
+// FUSED; at 104 x 210 42 and 28, at 40 x 110 27 and 24.  Left alone the compiler takes more registers than half the file at 8 rows, and no
+// second workgroup fits a compute unit; with the budget of 16 / R waves per SIMD 204 -> 146 us, FUSED 251 -> 151.
 // KB (with RC): the zero pattern of kb_unit.  Waves 1 and 3 have one source half, the windows of the vanishing products
 // are neither formed nor staged, and the half without a kappa part takes single coefficients; the terms left out are
 // products with zero.  4 rows, both halves, FUSED: 400 x 510 67 us without and 60 with it, eight such instances 470 and
 // 388, 64 of 40 x 110 20 and 18; one of 40 x 110 is a chain of latencies, 11.7 and 11.5.
 template <int BW, bool DUAL, class T, int R, int P, int HV, bool FUSED, bool RC, bool KB>
-__global__ __launch_bounds__(256) void k_radial_dia(
+__global__ __launch_bounds__(256, !RC && P == 1 && R < 16 ? 16 / R : 1) void k_radial_dia(
     const T *__restrict__ x, const T *__restrict__ V, const T *__restrict__ GD, const T *__restrict__ DD,
     const int *__restrict__ tiles, const int *__restrict__ tile_q, const double *__restrict__ tile_k, int nblk, int n,
     int nh, int nhp, int nseg, int lgrid, int nq, int sel, double cH, double beta, T *__restrict__ y,
@@ -1648,11 +1651,11 @@ bool dia_shape_ok(int r, int p) {
     return (r == 4 && (p == 1 || p == 2 || p == 4)) || (r == 8 && (p == 1 || p == 2)) || (r == 16 && p == 1);
 }
 
-// phase A inside the banded radial kernel (its windows formed from x and the coupling lists, no V): built for the
-// real form of the couplings; otherwise the two kernels run, with the same results
+// phase A inside the banded radial kernel (its windows formed from x and the coupling lists, no V), whichever angular
+// kernel ang_list names for the two-kernel form.  The matrix-core kernel reads V; the FP32 products never run on it.
 template <class T>
 bool ang_in_radial(const gade_model *m) {
-    return m->ang_fused && m->radial_kind == 2 && m->gd_real;
+    return m->ang_fused && m->radial_kind == 2 && (sizeof(T) == sizeof(float2) || !m->radial_mfma);
 }
 
 // tile shapes with a fused form: one row's window sums per lane fit the registers for up to 2 outputs per lane
@@ -1666,9 +1669,10 @@ int launch_dia(gade_model *m, int lgrid, const T *x, const T *V, const T *GD, co
     const int P = m->dia_p;
     const int nseg = (m->nh + 64 * P - 1) / (64 * P);
     const bool fused = ang_in_radial<T>(m);
-    const int hv = m->gd_real ? m->dia_hw : 2;  // the complex form is built for both halves per workgroup
+    const int hv = m->dia_hw;
     const dim3 grid((unsigned)m->ndtiles * (2 / hv) * nseg * lgrid);
     const T *acr = sizeof(T) == sizeof(float2) ? (const T *)m->d_acr32 : (const T *)m->d_acr;
+    const T *acf = sizeof(T) == sizeof(float2) ? (const T *)m->d_acf32 : (const T *)m->d_acf;
     if (fused && !fused_shape_ok(m->dia_r, P)) {
         gade::set_error("the fused angular + radial form needs at most 2 outputs per lane");
         return GADE_EINVAL;
@@ -1680,7 +1684,10 @@ int launch_dia(gade_model *m, int lgrid, const T *x, const T *V, const T *GD, co
                        m->d_aoff, (const int2 *)m->d_ack, CF_, m->lmax, m->nblk1, m->h_rot)
 #define GADE_DIA(R_, P_, F_)                         \
     if (!m->gd_real) {                               \
-        GADE_DIA1(R_, P_, 2, false, false, false, nullptr); \
+        if (hv == 2)                                 \
+            GADE_DIA1(R_, P_, 2, F_, false, false, acf); \
+        else                                         \
+            GADE_DIA1(R_, P_, 1, F_, false, false, acf); \
     } else if (m->g_kb) {                            \
         if (hv == 2)                                 \
             GADE_DIA1(R_, P_, 2, F_, true, true, acr);  \
