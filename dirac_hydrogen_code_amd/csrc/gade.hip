@@ -749,8 +749,9 @@ __global__ void k_build_DD(const double2 *__restrict__ D, const int *__restrict_
 // terms left out are products with zero, so the results equal the complex form's bit for bit.  At 400 x 510 and 4 rows
 // the complex form takes 93 us where the real one takes 58 (both without FUSED), 16 and 11 us at 40 x 110.
 // Complex form, a product call at 400 x 510 with 4 rows and both halves: 147 us with the angular kernel before it, 115
-// FUSED; at 104 x 210 42 and 28, at 40 x 110 27 and 24.  Left alone the compiler takes more registers than half the file at 8 rows, and no
-// second workgroup fits a compute unit; with the budget of 16 / R waves per SIMD 204 -> 146 us, FUSED 251 -> 151.
+// FUSED; at 104 x 210 42 and 28, at 40 x 110 27 and 24.  Left alone the compiler takes more registers than half the
+// file at 8 rows, and no second workgroup fits a compute unit; with the budget of 16 / R waves per SIMD 204 -> 146 us,
+// FUSED 251 -> 151.
 // KB (with RC): the zero pattern of kb_unit.  Waves 1 and 3 have one source half, the windows of the vanishing products
 // are neither formed nor staged, and the half without a kappa part takes single coefficients; the terms left out are
 // products with zero.  4 rows, both halves, FUSED: 400 x 510 67 us without and 60 with it, eight such instances 470 and
@@ -1645,8 +1646,8 @@ int angular_phase(gade_model *m, const double2 *x) {
     return launch_angular(m, x);
 }
 
-// tile shapes (rows per tile, outputs per lane) with an instantiated banded kernel: rows x outputs <= 16
-// complex accumulators per lane
+// tile shapes (rows per tile, outputs per lane) with an instantiated banded kernel: rows x outputs <= 16 complex
+// accumulators per lane and output half
 bool dia_shape_ok(int r, int p) {
     return (r == 4 && (p == 1 || p == 2 || p == 4)) || (r == 8 && (p == 1 || p == 2)) || (r == 16 && p == 1);
 }
@@ -1905,16 +1906,6 @@ int set_shape(gade_model *m, int r, int p, int hw, int fused) {
     m->dia_p = p;
     m->dia_hw = hw;
     m->ang_fused = fused;
-    return GADE_OK;
-}
-
-// the same as a caller's choice
-int use_shape(gade_model *m, int r, int p, int hw, int fused) {
-    GADE_TRY(set_shape(m, r, p, hw, fused));
-    m->par_r = r;
-    m->par_p = p;
-    m->par_hw = hw;
-    m->par_fused = fused;
     return GADE_OK;
 }
 
@@ -3602,7 +3593,8 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
                 if (one_tile && hw != m->dia_hw) continue;
                 for (int lb : {4, 2, 8})
                     if (ang_lds_ok(m, lb))
-                        cands.push_back({m->window, m->iter_batch, g0, rp.first, rp.second, lb, hw, 0, 0.0});
+                        cands.push_back({m->window, m->iter_batch, g0, rp.first, rp.second, lb, hw,
+                                         one_tile ? m->ang_fused : 0, 0.0});
                 if (!one_tile && fused_shape_ok(rp.first, rp.second))
                     cands.push_back({m->window, m->iter_batch, g0, rp.first, rp.second, m->ang_lb, hw, 1, 0.0});
             }
@@ -3758,8 +3750,7 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
     m->iter_batch = cands[pick].iter_batch;
     m->use_graph = cands[pick].graph != 0;
     GADE_TRY(shape(cands[pick].dia_r, cands[pick].dia_p, cands[pick].ang_lb, cands[pick].dia_hw, cands[pick].fused));
-    if (m->radial_kind == 2)
-        GADE_TRY(use_shape(m, cands[pick].dia_r, cands[pick].dia_p, cands[pick].dia_hw, cands[pick].fused));
+    m->fused_set = m->fused_set || (m->radial_kind == 2 && !one_tile);
     if (report)
         for (size_t c = 0; c < cands.size() && c < GADE_TUNE_MAX; c++) {
             double *r = report + (size_t)GADE_TUNE_COLS * c;
@@ -4002,29 +3993,30 @@ int gade_set_param(gade_model_t *m, const char *name, int value) {
     if (!strcmp(name, "ang_fused")) {
         // 1: the banded radial kernel forms each V window from x and the coupling lists (no angular kernel, no
         // V in HBM; bit-identical results), 0: the angular kernel writes V and the radial kernel reads it
-        if ((value != 0 && value != 1) || (value == 1 && !fused_shape_ok(m->par_r, m->par_p))) {
+        if ((value != 0 && value != 1) || (value == 1 && !fused_shape_ok(m->dia_r, m->dia_p))) {
             gade::set_error("ang_fused must be 0 or 1 (1 needs a tile shape with at most 2 outputs per lane)");
             return GADE_EINVAL;
         }
-        return use_shape(m, m->par_r, m->par_p, m->par_hw, value);
+        m->fused_set = true;
+        return set_shape(m, m->dia_r, m->dia_p, m->dia_hw, value);
     }
     if (!strcmp(name, "dia_halves")) {
-        // output halves per banded workgroup: 1 (one wave per half) or 2 (two waves share each window)
+        // output halves per banded workgroup: 1, or 2 (both share each window)
         if (value != 1 && value != 2) {
             gade::set_error("dia_halves must be 1 or 2");
             return GADE_EINVAL;
         }
-        return use_shape(m, m->par_r, m->par_p, value, m->par_fused);
+        return set_shape(m, m->dia_r, m->dia_p, value, m->ang_fused);
     }
     if (!strcmp(name, "dia_rows") || !strcmp(name, "dia_outputs")) {
         const bool rows = name[4] == 'r';
-        const int r = rows ? value : m->par_r, pp = rows ? m->par_p : value;
+        const int r = rows ? value : m->dia_r, pp = rows ? m->dia_p : value;
         if (!dia_shape_ok(r, pp)) {
             gade::set_error("banded tile shape (dia_rows, dia_outputs) must be (4,1), (4,2), (4,4), (8,1), (8,2) "
                             "or (16,1)");
             return GADE_EINVAL;
         }
-        if (m->par_fused && !fused_shape_ok(r, pp)) {
+        if (m->fused_set && m->ang_fused && !fused_shape_ok(r, pp)) {
             gade::set_error("the fused angular + radial form (ang_fused 1) has no (4,4) tile shape");
             return GADE_EINVAL;
         }
@@ -4032,7 +4024,7 @@ int gade_set_param(gade_model_t *m, const char *name, int value) {
             gade::set_error("the radial pattern is not banded");
             return GADE_EINVAL;
         }
-        return use_shape(m, r, pp, m->par_hw, m->par_fused);
+        return set_shape(m, r, pp, m->dia_hw, m->fused_set ? m->ang_fused : (int)fused_shape_ok(r, pp));
     }
     if (!strcmp(name, "precision")) {
         if (value != 0 && value != 1) {
@@ -4168,7 +4160,7 @@ int gade_get_param(const gade_model_t *m, const char *name, int *value) {
         return GADE_OK;
     }
     if (!strcmp(name, "dia_rows")) {
-        *value = m->par_r;
+        *value = m->dia_r;
         return GADE_OK;
     }
     if (!strcmp(name, "ang_list")) {
@@ -4184,15 +4176,15 @@ int gade_get_param(const gade_model_t *m, const char *name, int *value) {
         return GADE_OK;
     }
     if (!strcmp(name, "dia_halves")) {
-        *value = m->par_hw;
+        *value = m->dia_hw;
         return GADE_OK;
     }
     if (!strcmp(name, "ang_fused")) {
-        *value = m->par_fused;
+        *value = m->ang_fused;
         return GADE_OK;
     }
     if (!strcmp(name, "dia_outputs")) {
-        *value = m->par_p;
+        *value = m->dia_p;
         return GADE_OK;
     }
     if (!strcmp(name, "lg_features")) {

@@ -143,13 +143,11 @@ struct gade_model {
     int *d_dtiles = nullptr, *d_dtile_q = nullptr;
     double *d_dtile_k = nullptr;
     int *d_dtile_b = nullptr;      // instance of each tile (tiles never mix instances)
-    // banded tile shape in use: rows per tile, outputs per lane, output halves per workgroup (2: both halves share
-    // each window).  par_*: what a caller has set or tuned; until then the shape in use is the model's own choice:
-    // 4 rows, 1 output, both halves, fused, the fastest of the shapes at every size measured (apply, us, against the
+    // banded tile shape: rows per tile, outputs per lane, output halves per workgroup (2: both halves share each
+    // window).  4 rows, 1 output, both halves, fused is the fastest shape at every size measured (apply, us, against the
     // next shapes fused and the best unfused one: 40 x 110: 20, 22.5, 22; 5 x 60 x 76: 26, 27, 29.5; 400 x 510: 85,
     // 117, 111)
     int dia_r = 4, dia_p = 1, dia_hw = 2;
-    int par_r = 8, par_p = 1, par_hw = 1, par_fused = 0;
     // FP64 banded radial phase on the matrix cores: waves of two 8-row halves of one kappa each
     bool mfma_ok = false;          // the banded pattern fits the MFMA kernel (set up)
     int radial_mfma = 0;           // 1: FP64 radial products on MFMA (k_radial_mfma), 0: k_radial_dia (default)
@@ -161,6 +159,7 @@ struct gade_model {
     double *d_mg_k = nullptr;      // [nmg][2] kappa of each half
     int ang_lb = 2;                // multipoles per angular block
     int ang_fused = 1;             // 1: the banded radial kernel forms its V windows from x (no V in HBM)
+    bool fused_set = false;        // ang_fused was set or tuned (else it follows the tile shape: 1 where there is such a form)
     int psolve_ch = 16;            // preconditioner level height (16 or 32 rows)
     size_t gd_stride = 0;          // GD entries per instance
     double2 *d_V = nullptr;        // [lmax][4][nblk][n]

@@ -141,7 +141,7 @@ int gade_cn_run_batch(gade_model_t *m, double *psi_dev, const double *params, co
  * dia_outputs) in {(8,2), (4,2), (4,4), (8,1), (16,1), (4,1)} x output halves per workgroup dia_halves in
  * {1, 2} x the angular multipole group ang_lb in {4, 2, 8}, and the fused angular + radial form
  * (ang_fused 1) for the shapes with up to 2 outputs per lane, with the model's stepping (with the FP64 MFMA
- * radial kernel in FP64 only ang_lb varies); stage 2, with the fastest shapes:
+ * radial kernel in FP64 only ang_lb varies, and the shape stays as it was); stage 2, with the fastest shapes:
  * window in {2,4,8,16,32}, iter_batch in {0,1,2,4}, graph in {0,1} (the graph only with the banded
  * kernel and when the model's "graph" parameter is 1).  The fastest stage-2 candidate is kept.  Every candidate
  * must give the same trajectory, iterations and tolerances bit for bit, else GADE_EINVAL with the
@@ -300,22 +300,22 @@ int gade_assembled_get(gade_model_t *m, int *Ap, int *Ai, int *Ai_sub_map, doubl
  *             reference), 1..3 polynomial extrapolation (gade_extrapolate),
  *             GADE_GUESS_LEARNED the learned guess;
  *   "dia_rows", "dia_outputs"  banded tile shape: rows per tile and outputs per
- *             lane, (8,1) by default; (4,1), (4,2), (4,4), (8,2), (16,1) also;
- *   "dia_halves"  1 (default): one output half of a tile per workgroup; 2: both halves
- *             in one workgroup sharing each staged window;
- *             (until one of these or "ang_fused" is set or tuned, the model runs the
- *             shape it finds fastest, (4,1) with both halves and the angular phase inside);
+ *             lane, (4,1) by default; (4,2), (4,4), (8,1), (8,2), (16,1) also;
+ *   "dia_halves"  2 (default): both output halves of a tile in one workgroup, sharing
+ *             each staged window; 1: one half per workgroup;
  *   "ang_lb"  multipoles per angular block (2 by default; 4, 8);
- *   "ang_list"  1 (default): angular phase over the coupling lists; 0: Hall rows;
+ *   "ang_list"  angular kernel of the two-kernel form (ang_fused 0): 1 (default) over
+ *             the coupling lists, 0 over the Hall rows;
  *   "radial_mfma"  1: FP64 banded products on the matrix cores (0 by default);
  *   "psolve_chunk"  preconditioner level height, 16 (default) or 32 rows;
  *   "precision"  0 (default): FP64 solve; 1: FP32 inner solves with FP64 defect
  *             correction (gade_cn_run / gade_cn_run_batch);
  *   "graph"  1 (default): device-driven windows replay a captured step graph;
- *   "ang_fused"  1: the banded radial kernel forms its windows of the angular
- *             phase from x and the coupling lists itself (no angular kernel, no V in
- *             HBM; tile shapes with up to 2 outputs per lane); 0 (default): the
- *             angular kernel writes V, the radial kernel reads it;
+ *   "ang_fused"  1 (default where the tile shape has the form: up to 2 outputs per
+ *             lane): the banded radial kernel forms its windows of the angular phase
+ *             from x and the coupling lists itself (no angular kernel, no V in HBM);
+ *             0: the angular kernel writes V, the radial kernel reads it.  Set to 1 it
+ *             refuses the shape (4,4), and (4,4) refuses it;
  *   "lg_zmax"  range gate of the learned guess's inputs (gade_lg_uses).
  * Results do not depend on the choice. */
 int gade_set_param(gade_model_t *m, const char *name, int value);
