@@ -3645,7 +3645,8 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
         }
         return GADE_OK;
     };
-    const int sv_window = m->window, sv_batch = m->iter_batch, sv_profile = m->profile, sv_k = m->last_k;
+    const int sv_window = m->window, sv_batch = m->iter_batch, sv_profile = m->profile, sv_k = m->last_k,
+              sv_slack = m->slack_windows;
     const int sv_r = m->dia_r, sv_p = m->dia_p, sv_lb = m->ang_lb, sv_hw = m->dia_hw, sv_fused = m->ang_fused;
     const bool sv_graph = m->use_graph;
     auto shape = [&](int r, int pp, int lb, int hw, int fused) -> int {
@@ -3661,6 +3662,7 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
         m->use_graph = sv_graph;
         m->profile = sv_profile;
         m->last_k = sv_k;
+        m->slack_windows = sv_slack;
         (void)shape(sv_r, sv_p, sv_lb, sv_hw, sv_fused);
         const int rc = copy_state(false);
         (void)hipStreamSynchronize(m->stream);
@@ -3708,6 +3710,7 @@ int gade_autotune(gade_model_t *m, const double *psi, const double *params, doub
                 rc = GADE_EHIP;
             if (rc == GADE_OK) rc = copy_state(false);
             m->last_k = sv_k;
+            m->slack_windows = sv_slack;
             const auto t_a = std::chrono::steady_clock::now();
             if (rc == GADE_OK)
                 rc = cn_run_device(m, work, times.data(), nsteps, params, nullptr, tol, maxit, it.data(), tl.data(),
