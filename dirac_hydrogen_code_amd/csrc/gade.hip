@@ -4538,7 +4538,7 @@ int launch_tw(const gade_blocklu *lu, const T *F, const T *b, T *x, hipStream_t 
 #define TWI(T_, P_)                                                                                              \
     template int launch_tw<T_, P_>(const gade_blocklu *, const T_ *, const T_ *, T_ *, hipStream_t, const int *, \
                                    int, int, const PsolveVecs<T_> &);
-TWI(double2, PRE_P) TWI(double2, PRE_S) TWI(float2, PRE_NONE) TWI(float2, PRE_P) TWI(float2, PRE_S)
+TWI(double2, PRE_P) TWI(double2, PRE_S) TWI(float2, PRE_P) TWI(float2, PRE_S)
 #undef TWI
 
 int blocklu_solve_async(const gade_blocklu *lu, const double2 *b, double2 *x, hipStream_t stream, const int *gate,

@@ -646,17 +646,18 @@ __global__ void k_lg_gather_rows(const float *__restrict__ x, const float *mean,
 // The weights in the order in which the training kernel's lanes read them, next to the row-major copy: a 16-wide
 // step of a 16-wide tile is 64 lanes times four bf16, 512 contiguous bytes.
 //   fw[l]: the forward operand, tile n/16, step k/16, lane ((k/4)%4)*16 + n%16, element k%4
-//   bw[l]: the operand of dA = dZ W, tile k/16, step n/16, lane ((n/4)%4)*16 + k%16, element n%4
-template <int K, int N>
+//   bw[l]: the operand of dA = dZ W, tile k/16, step n/16, lane ((n/4)%4)*16 + k%16, element n%4 (the first layer's
+//          inputs have no gradient: not W1)
+template <int K, int N, bool BW = true>
 __device__ __forceinline__ void lg_put_w(int j, uint16_t v, uint16_t *__restrict__ fw, uint16_t *__restrict__ bw) {
     const int n = j / K, k = j % K;
     fw[(((n >> 4) * (K / 16) + (k >> 4)) * 64 + ((k >> 2) & 3) * 16 + (n & 15)) * 4 + (k & 3)] = v;
-    bw[(((k >> 4) * (N / 16) + (n >> 4)) * 64 + ((n >> 2) & 3) * 16 + (k & 15)) * 4 + (n & 3)] = v;
+    if (BW) bw[(((k >> 4) * (N / 16) + (n >> 4)) * 64 + ((n >> 2) & 3) * 16 + (k & 15)) * 4 + (n & 3)] = v;
 }
 __device__ __forceinline__ void lg_put(int i, uint16_t v, uint16_t *__restrict__ pbf, uint16_t *__restrict__ pfw,
                                        uint16_t *__restrict__ pbw) {
     pbf[i] = v;
-    if (i < (int)P_B1) lg_put_w<kIn, kHid>(i, v, pfw, pbw);
+    if (i < (int)P_B1) lg_put_w<kIn, kHid, false>(i, v, pfw, pbw);
     else if (i >= (int)P_W2 && i < (int)P_B2) lg_put_w<kHid, kHid>(i - P_W2, v, pfw + P_W2, pbw + P_W2);
     else if (i >= (int)P_W3 && i < (int)P_B3) lg_put_w<kHid, kHid>(i - P_W3, v, pfw + P_W3, pbw + P_W3);
     else if (i >= (int)P_W4 && i < (int)P_B4) lg_put_w<kHid, kOut>(i - P_W4, v, pfw + P_W4, pbw + P_W4);
@@ -1034,8 +1035,8 @@ struct gade_lg {
     uint16_t *pfw = nullptr, *pbw = nullptr;  // the weights again, in the training kernel's operand orders
     float *h_loss = nullptr;      // pinned: the mean loss of gade_lg_grad
     long adam_t = 0;
-    // training buffers (batch Mt)
-    int Mt = 0;
+    // training buffers (batch Mt; zt and yt: forward passes of Mf rows)
+    int Mt = 0, Mf = 0;
     uint16_t *xt = nullptr, *at[3] = {}, *gt[4] = {};
     float *zt[3] = {}, *yt = nullptr, *db = nullptr, *loss = nullptr;
 };
@@ -1128,26 +1129,35 @@ int lg_net_alloc(gade_lg *lg) {
     return GADE_OK;
 }
 
+// n elements in place of what *p held
+template <class T>
+int lg_realloc(T *&p, size_t n) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    return hip_alloc((void **)&p, sizeof(T) * n);
+}
+
+// buffers of a batch of Mt training samples
 int lg_train_alloc(gade_lg *lg, int Mt) {
     if (lg->Mt >= Mt) return GADE_OK;
-    for (void *q : {(void *)lg->xt, (void *)lg->yt, (void *)lg->db, (void *)lg->loss})
-        if (q) (void)hipFree(q);
-    for (int k = 0; k < 3; k++) {
-        if (lg->at[k]) (void)hipFree(lg->at[k]);
-        if (lg->zt[k]) (void)hipFree(lg->zt[k]);
-    }
-    for (int k = 0; k < 4; k++)
-        if (lg->gt[k]) (void)hipFree(lg->gt[k]);
+    lg->Mt = 0;  // until all are there
+    const size_t n = Mt;
+    GADE_TRY(lg_realloc(lg->xt, n * kIn));
+    GADE_TRY(lg_realloc(lg->db, n / 4 * kDb));
+    GADE_TRY(lg_realloc(lg->loss, n));
+    for (int k = 0; k < 3; k++) GADE_TRY(lg_realloc(lg->at[k], n * kHid));
+    for (int k = 0; k < 4; k++) GADE_TRY(lg_realloc(lg->gt[k], n * kHid));
     lg->Mt = Mt;
-    GADE_TRY(hip_alloc((void **)&lg->xt, sizeof(uint16_t) * Mt * kIn));
-    GADE_TRY(hip_alloc((void **)&lg->yt, sizeof(float) * Mt * kOut));
-    GADE_TRY(hip_alloc((void **)&lg->db, sizeof(float) * (Mt / 4) * kDb));
-    GADE_TRY(hip_alloc((void **)&lg->loss, sizeof(float) * Mt));
-    for (int k = 0; k < 3; k++) {
-        GADE_TRY(hip_alloc((void **)&lg->at[k], sizeof(uint16_t) * Mt * kHid));
-        GADE_TRY(hip_alloc((void **)&lg->zt[k], sizeof(float) * Mt * kHid));
-    }
-    for (int k = 0; k < 4; k++) GADE_TRY(hip_alloc((void **)&lg->gt[k], sizeof(uint16_t) * Mt * kHid));
+    return GADE_OK;
+}
+
+// what a forward pass of M rows needs besides a batch's inputs and activations
+int lg_rows_alloc(gade_lg *lg, int M) {
+    if (lg->Mf >= M) return GADE_OK;
+    lg->Mf = 0;
+    GADE_TRY(lg_realloc(lg->yt, (size_t)M * kOut));
+    for (int k = 0; k < 3; k++) GADE_TRY(lg_realloc(lg->zt[k], (size_t)M * kHid));
+    lg->Mf = M;
     return GADE_OK;
 }
 
@@ -1526,6 +1536,7 @@ int gade_lg_forward(gade_model_t *m, const float *x, int M, float *y) {
     if (!m->lg || !m->lg->net) return GADE_EINVAL;
     gade_lg *lg = m->lg;
     GADE_TRY(lg_train_alloc(lg, M));
+    GADE_TRY(lg_rows_alloc(lg, M));
     hipLaunchKernelGGL(k_lg_gather_rows, dim3(M), dim3(64), 0, m->stream, x, (const float *)lg->mean,
                        (const float *)lg->stdv, lg->xt);
     mlp_forward(lg, m->stream, M, lg->xt, lg->zt, lg->at, lg->yt);
