@@ -87,13 +87,13 @@ __device__ __forceinline__ float gelu_d(float z) {
 // tile of C (v_mfma_f32_16x16x16_bf16: lane l holds A[l%16][4(l/16)..+3], B[4(l/16)..+3][l%16] and
 // C[4(l/16)+i][l%16]).  The block's KS waves take the 16-wide k steps in turn (wave w: steps w, w + KS, ...) and
 // their accumulators are added in wave order; KS = 4 for the few rows of inference (short per-wave chains), 1 for
-// more rows.  M, N, K multiples of 16.
+// more rows.  A wave has the loads of U steps in flight.  M, N, K multiples of 16.
 // ---------------------------------------------------------------------------
 typedef short bf4 __attribute__((ext_vector_type(4)));
 typedef float fl4 __attribute__((ext_vector_type(4)));
 enum { EPI_BIAS = 1, EPI_BIAS_GELU = 2 };
 
-template <int EPI, int KS = 1>
+template <int EPI, int KS, int U>
 __global__ __launch_bounds__(64 * KS) void k_gemm_bf16(int M, int N, int K, const uint16_t *__restrict__ a,
                                                        const uint16_t *__restrict__ b, float *__restrict__ c, int ldc, const float *__restrict__ bias,
                                                        uint16_t *__restrict__ act, int ldact) {
@@ -104,17 +104,16 @@ __global__ __launch_bounds__(64 * KS) void k_gemm_bf16(int M, int N, int K, cons
     const uint16_t *ap = a + (long)(tm * 16 + r) * K;
     const uint16_t *bp = b + (long)(tn * 16 + r) * K;
     fl4 acc = {0.f, 0.f, 0.f, 0.f};
-    // loads of six steps in flight (the whole chain of a wave at KS = 4)
-    for (int k0 = 16 * w; k0 < K; k0 += 6 * 16 * KS) {
-        uint2 au[6], bu[6];
+    for (int k0 = 16 * w; k0 < K; k0 += U * 16 * KS) {
+        uint2 au[U], bu[U];
 #pragma unroll
-        for (int u = 0; u < 6; u++) {
+        for (int u = 0; u < U; u++) {
             const int k = min(k0 + 16 * KS * u, K - 16) + 4 * g;
             au[u] = *reinterpret_cast<const uint2 *>(ap + k);
             bu[u] = *reinterpret_cast<const uint2 *>(bp + k);
         }
 #pragma unroll
-        for (int u = 0; u < 6; u++)
+        for (int u = 0; u < U; u++)
             if (k0 + 16 * KS * u < K) {
                 bf4 av, bv;
                 __builtin_memcpy(&av, &au[u], sizeof av);
@@ -1177,33 +1176,35 @@ void lg_project(gade_model *m, int v0, int nv, const int *gate, int gstride) {
                        (const double2 *)lg->ppart, lg->proj, gate, gstride);
 }
 
-// forward of M rows: X (bf16 [M][kIn]) -> Z_l, A_l, Y; up to kSplitKRows rows (inference) each tile's k steps are
-// split over four waves
-constexpr int kSplitKRows = 64;
-void mlp_forward(const gade_lg *lg, hipStream_t st, int M, const uint16_t *X, float *const Z[3], uint16_t *const A[3],
-                 float *Y) {
+// Rows of a forward pass, X (bf16 [M][kIn]) -> Z_l, A_l, Y: up to kSplitKRows (inference) each tile's k steps are split
+// over four waves, the whole chain of a wave in flight.  With a wave per tile six steps' loads hide the latency of the
+// chain while the chip has few waves, but do not divide a layer's 16 or 18 steps; from kManyRows on, where it has
+// waves enough, two do: us with 6 / 2: 128 rows 34.0 / 37.9, 512 37.1 / 38.7, 1024 43.6 / 43.4, 8192 132 / 126.
+constexpr int kSplitKRows = 64, kManyRows = 1024;
+template <int KS, int U>
+void mlp_layers(const gade_lg *lg, hipStream_t st, int M, const uint16_t *X, float *const Z[3], uint16_t *const A[3],
+                float *Y) {
     const uint16_t *in = X;
     for (int l = 0; l < kLayers; l++) {
         const int K = kLin[l], N = kLout[l];
         const dim3 grid((M / 16) * (N / 16));
         const uint16_t *W = lg->pbf + kWoff[l];
         const float *bias = lg->p + kBoff[l];
-        if (M <= kSplitKRows) {
-            if (l < 3)
-                hipLaunchKernelGGL((k_gemm_bf16<EPI_BIAS_GELU, 4>), grid, dim3(256), 0, st, M, N, K, in, W, Z[l], N,
-                                   bias, A[l], N);
-            else
-                hipLaunchKernelGGL((k_gemm_bf16<EPI_BIAS, 4>), grid, dim3(256), 0, st, M, N, K, in, W, Y, N, bias,
-                                   (uint16_t *)nullptr, 0);
-        } else if (l < 3) {
-            hipLaunchKernelGGL(k_gemm_bf16<EPI_BIAS_GELU>, grid, dim3(64), 0, st, M, N, K, in, W, Z[l], N, bias, A[l],
-                               N);
+        if (l < 3) {
+            hipLaunchKernelGGL((k_gemm_bf16<EPI_BIAS_GELU, KS, U>), grid, dim3(64 * KS), 0, st, M, N, K, in, W, Z[l], N,
+                               bias, A[l], N);
+            in = A[l];
         } else {
-            hipLaunchKernelGGL(k_gemm_bf16<EPI_BIAS>, grid, dim3(64), 0, st, M, N, K, in, W, Y, N, bias,
+            hipLaunchKernelGGL((k_gemm_bf16<EPI_BIAS, KS, U>), grid, dim3(64 * KS), 0, st, M, N, K, in, W, Y, N, bias,
                                (uint16_t *)nullptr, 0);
         }
-        if (l < 3) in = A[l];
     }
+}
+void mlp_forward(const gade_lg *lg, hipStream_t st, int M, const uint16_t *X, float *const Z[3], uint16_t *const A[3],
+                 float *Y) {
+    if (M <= kSplitKRows) mlp_layers<4, 6>(lg, st, M, X, Z, A, Y);
+    else if (M < kManyRows) mlp_layers<1, 6>(lg, st, M, X, Z, A, Y);
+    else mlp_layers<1, 2>(lg, st, M, X, Z, A, Y);
 }
 
 // Four samples a workgroup while every workgroup finds a CU of its own (256), sixteen beyond: a call takes 36 and
