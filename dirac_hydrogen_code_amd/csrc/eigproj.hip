@@ -47,6 +47,13 @@ constexpr int kItems = kEigThreads / kLanes;
 inline int eig_split(int nblk, int n) {
     return std::max(1, std::min((n + kItems - 1) / kItems, 512 / std::max(1, nblk)));
 }
+// threads of a workgroup: no more than the eigenpairs need, and 256 when there are more blocks than the chip holds
+// workgroups of kEigThreads (two per CU): their phases then overlap instead of following each other.  Populations,
+// us with kEigThreads throughout / now (one thread per eigenpair, the form before): 364 x 30: 26 / 19 (31); 1300 x 30:
+// 49 / 25 (37-50); 1300 x 130: 77 / 64 (64); 544 x 130: 47 / 40 (52); 544 x 270: 83 / 80 (113).
+inline int eig_threads(int nblk, int n) {
+    return (std::min(n, nblk > 512 ? 32 : kItems) + 7) / 8 * 64;
+}
 template <bool COEF>
 __global__ __launch_bounds__(kEigThreads) void k_eigproj(const double2 *__restrict__ x, const double2 *__restrict__ D,
                                                          const int *__restrict__ ell_col,
@@ -60,7 +67,8 @@ __global__ __launch_bounds__(kEigThreads) void k_eigproj(const double2 *__restri
     const int lane = threadIdx.x & 63, part = lane >> 3;
     const int item = (threadIdx.x >> 6) * 8 + (lane & 7);  // eigenpair (or row of S) of this lane's group
     const double *V = VT + (size_t)q * n * n;
-    const int jf = blockIdx.y * kItems;  // first pass of this workgroup
+    const int items = blockDim.x / kLanes;
+    const int jf = blockIdx.y * items;  // first pass of this workgroup
     double v0[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; u++) {
@@ -70,7 +78,7 @@ __global__ __launch_bounds__(kEigThreads) void k_eigproj(const double2 *__restri
     const double2 *Sq = D + ((size_t)2 * nq + q) * ellw * n;  // S(k) in ELL layout
     const double2 *xr = x + (size_t)r * n;
     double acc[4] = {0, 0, 0, 0};
-    for (int a0 = 0; a0 < n; a0 += kItems) {
+    for (int a0 = 0; a0 < n; a0 += items) {
         const int a = a0 + item;
         double sx = 0, sy = 0;
         if (a < n) {
@@ -94,7 +102,7 @@ __global__ __launch_bounds__(kEigThreads) void k_eigproj(const double2 *__restri
         }
     }
     __syncthreads();
-    for (int j0 = jf; j0 < n; j0 += gridDim.y * kItems) {
+    for (int j0 = jf; j0 < n; j0 += gridDim.y * items) {
         const int j = j0 + item;
         double cx = 0, cy = 0;
         if (j < n) {
@@ -224,7 +232,7 @@ int gade_populations(gade_model_t *m, const double *x, double *norm, double *bou
     // several threads take turns, as they did on the stream
     std::lock_guard<std::mutex> one(m->eig_mutex);
     const int ny = eig_split(m->nblk, m->n);
-    hipLaunchKernelGGL(k_eigproj<false>, dim3(m->nblk, ny), dim3(kEigThreads), sizeof(double2) * m->n, m->stream,
+    hipLaunchKernelGGL(k_eigproj<false>, dim3(m->nblk, ny), dim3(eig_threads(m->nblk, m->n)), sizeof(double2) * m->n, m->stream,
                        (const double2 *)x, m->d_D, m->d_ell_col, m->d_blk_q, m->d_evec, m->d_eval, m->n, m->ellw,
                        m->nq, csq, m->h_eig);
     hipError_t e = hipGetLastError();
@@ -255,8 +263,8 @@ int gade_psiev(gade_model_t *m, const double *x, double *psiev) {
     const size_t cnt = (size_t)m->nblk * m->n;
     double2 *d_out = nullptr;
     GADE_TRY(gade::hip_alloc((void **)&d_out, sizeof(double2) * cnt));
-    hipLaunchKernelGGL(k_eigproj<true>, dim3(m->nblk, eig_split(m->nblk, m->n)), dim3(kEigThreads), sizeof(double2) * m->n, m->stream,
-                       (const double2 *)x, m->d_D, m->d_ell_col, m->d_blk_q, m->d_evec, m->d_eval, m->n, m->ellw,
+    hipLaunchKernelGGL(k_eigproj<true>, dim3(m->nblk, eig_split(m->nblk, m->n)), dim3(eig_threads(m->nblk, m->n)),
+                       sizeof(double2) * m->n, m->stream, (const double2 *)x, m->d_D, m->d_ell_col, m->d_blk_q, m->d_evec, m->d_eval, m->n, m->ellw,
                        m->nq, 0.0, (double *)d_out);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(psiev, d_out, sizeof(double2) * cnt, hipMemcpyDeviceToHost, m->stream);
