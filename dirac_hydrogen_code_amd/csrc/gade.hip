@@ -1448,8 +1448,12 @@ __global__ void k_full_submap(const int *hAp, const int *subAp, const int *fAp, 
 // the couplings come by scalar loads and a multipole with a zero coupling is skipped by the whole wave.  It was one
 // workgroup per (R, a), whose G loads (up to 8 LM of 16 bytes per entry, a radial row apart) came from L2 each time:
 // 388 us for the 13.4 M entries of 104 x 210 with 4 multipoles, now 90 (the stores alone, 215 MB, take about 45).
-template <int LM>
-__global__ __launch_bounds__(256) void k_assemble(const int *__restrict__ hAp, const int *__restrict__ hAi,
+// A workgroup has four waves, and sixteen from 11 multipoles on, where its G-sums take more than half a CU's LDS and the
+// CU holds one: us at 24 x 50, 60 x 110 with 12 multipoles 34, 140 (50, 293 with four waves), with 16 40, 176 (66, 376;
+// one workgroup per row: 52, 340).
+constexpr int asm_waves(int lmax) { return lmax > 10 ? 16 : 4; }
+template <int LM, int NW = asm_waves(LM)>
+__global__ __launch_bounds__(64 * NW) void k_assemble(const int *__restrict__ hAp, const int *__restrict__ hAi,
                                                   const int *__restrict__ kap, const double2 *__restrict__ coef,
                                                   const int *__restrict__ diag, const int *__restrict__ subAp,
                                                   const double2 *__restrict__ GE, const double2 *__restrict__ D,
@@ -1462,13 +1466,13 @@ __global__ __launch_bounds__(256) void k_assemble(const int *__restrict__ hAp, c
     const bool on = t < len && 2 * (int)blockIdx.x + (lane >> 5) < n;
     const size_t slab = (size_t)ellw * n;
     const size_t ep = (size_t)(on ? t : 0) * n + a;
-    for (int lm = wave; lm < 8 * LM; lm += 4) sg[lm][lane] = GE[(size_t)lm * slab + ep];
+    for (int lm = wave; lm < 8 * LM; lm += NW) sg[lm][lane] = GE[(size_t)lm * slab + ep];
     __syncthreads();
     for (int R = blockIdx.y; R < nblk; R += gridDim.y) {
         const int p0 = hAp[R], nb = hAp[R + 1] - p0;
         const double ki = kap[R];
         double2 *out = fAx + fAp[(size_t)R * n + a] + t;
-        for (int pos = wave; pos < nb; pos += 4) {
+        for (int pos = wave; pos < nb; pos += NW) {
             const int p = p0 + pos;
             const double kj = kap[hAi[p]];
             double2 val = make_double2(0, 0);
@@ -3863,7 +3867,7 @@ int gade_assembled_timedep_into(gade_model_t *m, const int *Ap_dev, double *Ax_d
     {
         Prof pr(m, "assemble", GADE_PROF_ASSEMBLE);
 #define ASM(LM) \
-    case LM: hipLaunchKernelGGL(k_assemble<LM>, grid, dim3(256), 0, m->stream, m->d_hAp, m->d_hAi, m->d_kap, m->d_coef, m->d_diag, m->d_subAp, m->d_GE, m->d_D, m->d_blk_q, Ap_dev, m->nblk, m->n, m->ellw, m->nq, (double2 *)Ax_dev); break;
+    case LM: hipLaunchKernelGGL(k_assemble<LM>, grid, dim3(64 * asm_waves(LM)), 0, m->stream, m->d_hAp, m->d_hAi, m->d_kap, m->d_coef, m->d_diag, m->d_subAp, m->d_GE, m->d_D, m->d_blk_q, Ap_dev, m->nblk, m->n, m->ellw, m->nq, (double2 *)Ax_dev); break;
         switch (m->lmax) {
             ASM(1) ASM(2) ASM(3) ASM(4) ASM(5) ASM(6) ASM(7) ASM(8) ASM(9) ASM(10) ASM(11) ASM(12) ASM(13) ASM(14) ASM(15) ASM(16)
             default: return GADE_EINVAL;
