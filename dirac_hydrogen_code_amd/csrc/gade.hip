@@ -757,7 +757,7 @@ __global__ void k_build_DD(const double2 *__restrict__ D, const int *__restrict_
 // products with zero.  4 rows, both halves, FUSED: 400 x 510 67 us without and 60 with it, eight such instances 470 and
 // 388, 64 of 40 x 110 20 and 18; one of 40 x 110 is a chain of latencies, 11.7 and 11.5.
 template <int BW, bool DUAL, class T, int R, int P, int HV, bool FUSED, bool RC, bool KB>
-__global__ __launch_bounds__(256, !RC && P == 1 && R < 16 ? 16 / R : 1) void k_radial_dia(
+__global__ __launch_bounds__(256, !RC && P == 1 && R < 16 ? 16 / R : 0) void k_radial_dia(
     const T *__restrict__ x, const T *__restrict__ V, const T *__restrict__ GD, const T *__restrict__ DD,
     const int *__restrict__ tiles, const int *__restrict__ tile_q, const double *__restrict__ tile_k, int nblk, int n,
     int nh, int nhp, int nseg, int lgrid, int nq, int sel, double cH, double beta, T *__restrict__ y,
