@@ -75,6 +75,11 @@ def ensure_inputs(config, datadir):
     return datadir
 
 
+def real_form(gp):
+    """Whether the generated couplings and a real f(t) run the banded kernels' real form (zero quadrants left out)."""
+    return gp.get_param("radial") == 2 and not gp.get_param("radial_mfma") and bool(gp.get_param("ang_list"))
+
+
 def kernel_models(gp):
     """Algorithmic work per launch of each kernel family (flops or HBM bytes)."""
     from dirac_hydrogen_code_amd.couplings import csr_read
@@ -95,11 +100,11 @@ def kernel_models(gp):
     nnz_full = gp.hall_nnz * nnzb
     # the banded kernel runs the generated couplings on real coefficients (4 flops a product instead of 8) and leaves
     # out a quarter of the G products, zero in their basis; the stationary operator is complex
-    real = gp.get_param("radial") == 2 and not gp.get_param("radial_mfma")
+    real = real_form(gp)
     radial = nb * nnzb * ((12.0 if real else 32.0) * L + 8.0)
     # the fused form does the angular contraction inside the radial kernel, without the vanishing products' windows
-    fused = gp.get_param("ang_fused") and real
-    angular = (6.0 if fused else 8.0 if real else 16.0) * ang_nnz * n
+    fused = gp.get_param("ang_fused") and gp.get_param("radial") == 2 and not gp.get_param("radial_mfma")
+    angular = (16.0 if not real else 6.0 if fused else 8.0) * ang_nnz * n
     return {
         # fused radial SpMM: per block, 4 kappa-folded radial products per l + the diagonal operator (and the
         # angular contraction with ang_fused)
@@ -566,12 +571,13 @@ def main():
     else:
         fused = gp.get_param("ang_fused")
         rp = f"{gp.get_param('dia_rows')}, {gp.get_param('dia_outputs')}"
-        # the generated couplings run the real form with the zero quadrants left out (the last two flags)
-        form = f"{rp}, {gp.get_param('dia_halves')}, {'true' if fused else 'false'}, true, true>"
+        real = "true" if real_form(gp) else "false"
+        form = f"{rp}, {gp.get_param('dia_halves')}, {'true' if fused else 'false'}, {real}, {real}>"
         KERNEL_NAMES["radial"] = f"k_radial_dia<7, false, double2, {form}"
         KERNEL_NAMES["radial_pair"] = f"k_radial_dia<7, true, double2, {form}"
-    ang = "k_angular_list" if gp.get_param("ang_list") else "k_angular"
-    KERNEL_NAMES["angular"] = f"{ang}<{gp.get_param('ang_lb')}, double2>"
+    lb = f"{gp.get_param('ang_lb')}, double2"
+    KERNEL_NAMES["angular"] = (f"k_angular_list<{lb}, {'true' if real_form(gp) else 'false'}>"
+                               if gp.get_param("ang_list") else f"k_angular<{lb}>")
 
     # timed region: K steps continuing the trajectory; every profile_period-th launch of the dominant
     # family carries a HIP event pair (each pair costs a few microseconds of idle time on the stream);
