@@ -4051,7 +4051,10 @@ int gade_set_param(gade_model_t *m, const char *name, int value) {
         if (value != m->radial_mfma) {
             drop_step_graph(m);
             m->radial_mfma = value;
-            if (m->radial_kind == 2) GADE_TRY(launch_gsums(m, false));  // the current f(t) in the kernel's layout
+            if (m->radial_kind == 2) {  // the sums that every instance has, in the kernel's layout
+                set_form(m, real_form(m, m->gd_ft));
+                GADE_TRY(dia_gsums(m, m->gd_ft));
+            }
         }
         return GADE_OK;
     }

@@ -63,13 +63,14 @@ def test_instances_without_a_step_keep_their_sums(datadir, cfg, cplx, nsteps_b, 
     assert np.array_equal(psi.view(np.float64), want.view(np.float64))
 
 
+@pytest.mark.parametrize("name,values", [("ang_list", (0, 1)), ("radial_mfma", (1, 0))])
 @pytest.mark.parametrize("cfg", ["dipole", "nondipole_small"])
-def test_angular_kernel_switch_keeps_every_instance(datadir, cfg):
-    """ang_list changes the layout of the G-sums, not the f(t) that each instance stopped at."""
-    print(f"[gpu] ang_list after a batch of unequal lengths {cfg}", flush=True)
+def test_kernel_switch_keeps_every_instance(datadir, cfg, name, values):
+    """ang_list and radial_mfma change the layout of the G-sums, not the f(t) that each instance stopped at."""
+    print(f"[gpu] {name} after a batch of unequal lengths {cfg}", flush=True)
     held = [gade.pulse(10, 50, 2, 0.01)] * len(PARAMS)
     om = O.Model(datadir(cfg), LMAX[cfg], dt_of(cfg), nthreads=4)
     gp, _, f = batch_of(datadir, cfg, held, [9, 0, 4])
-    for value in (0, 1):
-        gp.set_param("ang_list", value)
-        check(gp, om, f, f"ang_list {value}")
+    for value in values:
+        gp.set_param(name, value)
+        check(gp, om, f, f"{name} {value}")
